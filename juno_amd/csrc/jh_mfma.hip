@@ -9,17 +9,23 @@
 // accumulator of a lane holds one weight row (its own) for 16 batch columns:
 //
 //  * Weights: each format turns its packed integers into exact fp16 integers
-//    (Q4_K: ls*q <= 945 from 1024 + ls*q by one 24-bit multiply-add and one
-//    fp16 subtraction per pair; Q6_K:
-//    u - 32; Q8_0: q) and applies its fp32 scales per row in registers -- Q4_K
-//    once per 256 columns with d and dmin (the min term is one extra MFMA
-//    against per-sub-block sums of x), Q6_K per 16-column sub-block with the
-//    reference's d*sc, Q8_0 per 32-column block with d.
+//    (or half-integers) and applies its fp32 scales per row in registers: Q4_K,
+//    Q5_K and Q2_K fold their small integer scales into the operand (ls * (q - C),
+//    one packed FMA per pair, centred where the sub-block has a min) and apply d
+//    and dmin per 256 or 128 columns, the min term and the centre as extra MFMAs
+//    against sums of x; Q6_K and Q3_K fold per 16-column sub-block with d * sc,
+//    Q8_0 per 32-column block with d.
 //  * Activations: x is split into fp16 hi + lo limbs (x = hi + lo to ~2^-22,
 //    so only the order of summation differs from fp32) after a power-of-two
 //    scale per (column, 256-column super-block) that keeps fp16 in range.
 //    Each workgroup converts the fp32 x slice of a super-block straight into
 //    its LDS image while it stages the weights (no separate prep launch).
+//    Up to 16 columns (HL) the two limbs share one MFMA, rows 0..15 and 16..31
+//    of its A operand.  What bounds the walk is the reading of x from LDS: every
+//    wave needs all of it for its own 32 rows, 33 KB per super-block and wave at
+//    143 B/ns per CU (1.85 us for 8 waves, against 1.2 us of MFMA); HL halves that
+//    and the MFMAs (us, 16 columns, before -> after: 2 x 14336 x 4096 Q4_K 36 -> 29,
+//    4096 x 14336 Q6_K 30 -> 27, 4096^2 Q4_K 13.5 -> 11.6, 9216 x 3072 Q8_0 18.1 -> 16.0).
 //  * Work split: a workgroup is kWaves waves x 32 rows, all B columns, and a
 //    range of super-blocks.  Per super-block it stages the x slice in LDS
 //    (shared by all its rows) and each wave stages its rows' packed blocks in
@@ -35,6 +41,7 @@
 
 #include <mutex>
 #include <stdlib.h>
+#include <utility>
 
 namespace jh {
 namespace {
@@ -42,12 +49,6 @@ namespace {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-// 2-byte-aligned views for Q6_K / Q8_0 fields (gfx950 global loads take any
-// byte address; the compiler still emits single dwordx2 / dwordx4 loads)
-typedef uint32_t u32x2a2 __attribute__((ext_vector_type(2), aligned(2)));
-typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32a2 __attribute__((aligned(2)));
-constexpr int kPrefetch = 1;  // super-blocks of weight chunks in flight per wave (B <= 32)
 constexpr int kMinWorkgroups = 256;  // split K until the grid has this many
 
 // Timeline builds (-DJH_TIMELINE, juno_amd/timeline.py; never the shipped
@@ -75,195 +76,239 @@ constexpr int kThreads = 64 * kWaves;
 constexpr int kRowsPerWG = kWaves * kRowsPerWave;
 constexpr int kXPad = 8;  // halves of padding per LDS column (spreads banks)
 
-// Reductions over the 16 lanes of one DPP row (lanes 16 r .. 16 r + 15): xor-1
-// and xor-2 butterflies, then the half-row and row mirrors.  Each step adds two
-// values that are equal across the lanes being paired, so every lane ends with
-// the bit-identical result.
+// f(integral_constant i) for i = 0 .. N - 1
+template <class F, int... I>
+__device__ __forceinline__ void for_seq(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_c(F f) {
+    for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// Maximum over the 16 lanes of one DPP row (lanes 16 r .. 16 r + 15): xor-1 and
+// xor-2 butterflies, then the half-row and row mirrors.
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float row16_sum(float v) {
-    v += dpp_f<0xB1>(v);   // quad_perm 1,0,3,2
-    v += dpp_f<0x4E>(v);   // quad_perm 2,3,0,1
-    v += dpp_f<0x141>(v);  // row_half_mirror
-    return v + dpp_f<0x140>(v);  // row_mirror
-}
 __device__ __forceinline__ float row16_max(float v) {
-    v = fmaxf(v, dpp_f<0xB1>(v));
-    v = fmaxf(v, dpp_f<0x4E>(v));
-    v = fmaxf(v, dpp_f<0x141>(v));
-    return fmaxf(v, dpp_f<0x140>(v));
+    v = fmaxf(v, dpp_f<0xB1>(v));   // quad_perm 1,0,3,2
+    v = fmaxf(v, dpp_f<0x4E>(v));   // quad_perm 2,3,0,1
+    v = fmaxf(v, dpp_f<0x141>(v));  // row_half_mirror
+    return fmaxf(v, dpp_f<0x140>(v));  // row_mirror
 }
 
-// x into the LDS image of one column and super-block, inside the GEMM: 16
-// consecutive lanes hold its 256 values, 16 each (xv).  A power-of-two scale
-// puts max |x s| in [2^12, 2^13) (exact, undone on the partial sums), then x s
-// is split into fp16 hi + lo limbs, and the 32-column sub-block sums (as hi and
-// lo halves) and the super-block sum S are formed over 4-value groups with
-// fixed butterflies (deterministic).
-__device__ __forceinline__ void stage_x_column(const float (&xv)[16], int q, _Float16 *sh_hi, _Float16 *sh_lo,
-                                               _Float16 *sh_xs, _Float16 *sh_x16, float2 *sh_S, int col, int colh) {
+// One column and super-block of x as MFMA operands: 16 consecutive lanes hold
+// its 256 values, lane q the values 16 q .. +16 (xv).  A power-of-two scale puts
+// max |x s| in [2^12, 2^13) (exact, undone on the partial sums by cs = 1 / s),
+// then x s is split into fp16 hi + lo limbs by mixed-precision FMAs (x s is
+// exact, so hi is x s rounded and lo the rounded rest): two units of 8 values per
+// lane and limb, in the order 0 2 1 3 4 6 5 7, in which packed weight bytes
+// become fp16 pairs (b0, b2), (b1, b3) by a mask alone.  The 16-value sums times
+// 2^-4 and (even q) the 32-value sums times 2^-5 stay in fp16's range for any x.
+// All sums run in fixed orders.
+constexpr int kXsShift = 5, kX16Shift = 4;
+struct XColumn {
+    half8 h[2], l[2];
+    float s16, s32, cs;
+};
+__device__ __forceinline__ XColumn split_x(const float (&xv)[16]) {
+    XColumn r;
     float m = 0.f;
 #pragma unroll
     for (int j = 0; j < 16; j++) m = fmaxf(m, fabsf(xv[j]));
     m = row16_max(m);  // the 16 lanes of the column
-    int e = 0;
-    if (m > 0.f) (void)frexpf(m, &e);
-    const float s = m > 0.f ? ldexpf(1.f, 13 - e) : 1.f;
-    float g[4];  // sums of the 4-value groups
+    int k = 0;
+    if (m > 0.f) {
+        int e;
+        (void)frexpf(m, &e);
+        k = min(13 - e, 126);  // both 2^k and 2^-k are normal
+    }
+    const float s = ldexpf(1.f, k);
+    r.cs = ldexpf(1.f, -k);
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        _Float16 h4[4], l4[4];
-        float sum = 0.f;
+    for (int u = 0; u < 2; u++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float v = xv[4 * k + j] * s;
-            const _Float16 h = (_Float16)v;
-            const _Float16 l = (_Float16)(v - (float)h);
-            h4[j] = h;
-            l4[j] = l;
-            sum += (float)h + (float)l;
+        for (int i = 0; i < 8; i++) {
+            constexpr int ord[8] = {0, 2, 1, 3, 4, 6, 5, 7};
+            const float x = xv[8 * u + ord[i]];
+            const _Float16 h = (_Float16)(x * s);
+            r.h[u][i] = h;
+            r.l[u][i] = (_Float16)fmaf(x, s, -(float)h);
         }
-        _Float16 *ph = sh_hi + col * colh + 16 * q + 4 * k, *pl = sh_lo + col * colh + 16 * q + 4 * k;
+    float g[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            ph[j] = h4[j];
-            pl[j] = l4[j];
-        }
-        g[k] = sum;
-    }
-    // 16-value group q (this lane's values): hi + lo in sh_x16 (the Q2_K min term)
-    float sub = (g[0] + g[1]) + (g[2] + g[3]);
-    {
-        const _Float16 h = (_Float16)sub;
-        sh_x16[col * 32 + q] = h;
-        sh_x16[col * 32 + 16 + q] = (_Float16)(sub - (float)h);
-    }
-    // sub-block (32 values = groups 8i .. 8i+7 = this lane and its neighbour)
-    sub += dpp_f<0xB1>(sub);
-    if ((q & 1) == 0) {
-        const _Float16 h = (_Float16)sub;
-        sh_xs[col * 16 + (q >> 1)] = h;
-        sh_xs[col * 16 + 8 + (q >> 1)] = (_Float16)(sub - (float)h);
-    }
-    // super-block total: the lane's 4 groups, then across the column's 16 lanes
-    const float tot = row16_sum((g[0] + g[2]) + (g[1] + g[3]));
-    if (q == 0) sh_S[col] = make_float2(tot, 1.f / s);
+    for (int i = 0; i < 4; i++) g[i] = (xv[4 * i] + xv[4 * i + 1]) + (xv[4 * i + 2] + xv[4 * i + 3]);
+    const float sub = ((g[0] + g[1]) + (g[2] + g[3])) * s;
+    r.s16 = ldexpf(sub, -kX16Shift);
+    r.s32 = ldexpf(sub + dpp_f<0xB1>(sub), -kXsShift);  // this lane's and its neighbour's
+    return r;
 }
 
-// ------------------------------------------------------------------ format policies
-// Each format supplies, for one 256-column stretch ("super-block") of a row:
-//   Regs              the lane's weight bytes (row lr, K half kh), in VGPRs
-//   load(r, p, kh)    p = first byte of the row's stretch
-//   Smem / publish    per-row fp32 scales, shared through LDS
-//   compute<NT>(...)  the MFMAs and the fold into the fp32 totals
-// K-step t covers 16 columns; lane half kh supplies 8 of them.  Every weight
-// enters the MFMA as an exact fp16 integer; scales are applied in fp32.
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
+// ------------------------------------------------------------------ the x operand
+// Virtual columns are the 32 rows of the MFMA's A operand for one column group:
+//   !HL  32 batch columns, their hi limbs and their lo limbs in two planes (two
+//        MFMAs per K-step)
+//   HL   16 batch columns, rows 0..15 their hi limbs and rows 16..31 their lo
+//        limbs: one MFMA per K-step does both, and half the operand is read from
+//        LDS.  (The rows past a batch of 3..16 would be padding otherwise.)
+// Contexts give a lane (row lr of A, K half kh) its operands of a super-block:
+//   x(n, off) / xlo(n, off)  unit at column offset off, column group n
+//   xs(n)                    the 8 32-value sums, limb kh (hi, lo)
+//   x16(n, limb)             the 16-value sums 8 kh .. +8
+//   cs()                     1 / scale per batch column
+// The sums' rows 16..31 are zero with HL.
 constexpr int COLH = 256 + kXPad;  // halves per LDS column of the staged x slice
 
-// x fragments of the padded image the fused kernel converts into LDS: column
-// col at col * COLH halves (hi and lo), its sub-block sums at col * 16.
+// The padded image the fused kernel converts into LDS: column col at col * COLH
+// halves, its sums at col * 16 and col * 32.
+template <bool HL, int NT>
+struct XImage {
+    static constexpr int kCols = (HL ? 16 : 32) * NT;
+    static constexpr int kLo = (HL ? 16 : 32 * NT) * COLH;     // halves from a column's hi limbs to its lo limbs
+    static constexpr int kXs = (HL ? 1 : 2) * 32 * NT * COLH;  // halves: 32 NT x [8 hi, 8 lo]
+    static constexpr int kX16 = kXs + 32 * NT * 16;            // halves: 32 NT x [16 hi, 16 lo]
+    static constexpr int kCs = 2 * (kX16 + 32 * NT * 32);      // bytes: 32 NT floats
+    static constexpr int kBytes = kCs + 32 * NT * 4;
+    // one lane's share of column col (lane q of its 16), with the sums that the format reads
+    template <int SUMS>
+    static __device__ __forceinline__ void store(uint8_t *buf, const float (&xv)[16], int q, int col) {
+        const XColumn x = split_x(xv);
+        _Float16 *base = reinterpret_cast<_Float16 *>(buf), *hi = base + col * COLH + 16 * q;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            *reinterpret_cast<half8 *>(hi + 8 * u) = x.h[u];
+            *reinterpret_cast<half8 *>(hi + kLo + 8 * u) = x.l[u];
+        }
+        if (SUMS == 16) {
+            const _Float16 h = (_Float16)x.s16;
+            base[kX16 + col * 32 + q] = h;
+            base[kX16 + col * 32 + 16 + q] = (_Float16)(x.s16 - (float)h);
+        }
+        if (SUMS == 32 && (q & 1) == 0) {
+            const _Float16 h = (_Float16)x.s32;
+            base[kXs + col * 16 + (q >> 1)] = h;
+            base[kXs + col * 16 + 8 + (q >> 1)] = (_Float16)(x.s32 - (float)h);
+        }
+        if (q == 0) reinterpret_cast<float *>(buf + kCs)[col] = x.cs;
+    }
+    // the sums' row of a virtual column that holds lo limbs (HL)
+    static __device__ __forceinline__ void zero_sums(uint8_t *buf, int q, int row) {
+        _Float16 *base = reinterpret_cast<_Float16 *>(buf);
+        base[kXs + row * 16 + q] = (_Float16)0.f;
+        base[kX16 + row * 32 + q] = (_Float16)0.f;
+        base[kX16 + row * 32 + 16 + q] = (_Float16)0.f;
+    }
+};
+template <bool HL, int NT>
 struct Ctx {
-    int wave, lr, kh;
-    const _Float16 *sh_hi, *sh_lo, *sh_xs, *sh_x16;
-    const float2 *sh_S;
-    // 16-column group sums of x, K-half kh: hi limbs, then lo limbs
-    __device__ __forceinline__ half8 x16h(int col) const { return *reinterpret_cast<const half8 *>(sh_x16 + col * 32 + 8 * kh); }
-    __device__ __forceinline__ half8 x16l(int col) const {
-        return *reinterpret_cast<const half8 *>(sh_x16 + col * 32 + 16 + 8 * kh);
-    }
-    __device__ __forceinline__ half8 xh(int col, int xoff) const {
-        return *reinterpret_cast<const half8 *>(sh_hi + col * COLH + xoff);
-    }
-    __device__ __forceinline__ half8 xl(int col, int xoff) const {
-        return *reinterpret_cast<const half8 *>(sh_lo + col * COLH + xoff);
-    }
-    __device__ __forceinline__ half8 xm(int col) const { return *reinterpret_cast<const half8 *>(sh_xs + col * 16 + 8 * kh); }
-    __device__ __forceinline__ const float2 *S() const { return sh_S; }
-};
-
-// ------------------------------------------------------------------ prepared x (B <= 32)
-// One super-block of x for 32 batch columns, laid out exactly as the GEMM's
-// LDS image so that it moves in as a contiguous DMA copy:
-//   [hi: 32 columns x 32 units][lo: the same][sub-block sums: 32 x 16 halves]
-//   [(S, 1 / scale): 32 x float2][pad to 34 x 1 KB]
-// A unit is 16 bytes (8 consecutive values of one column).  Unit u of column
-// col sits at slot col * 32 + (u ^ (col & 31)): the XOR swizzle lets the 32
-// lanes that read unit u of 32 columns hit distinct LDS banks without padding.
-constexpr int kSlabHi = 0, kSlabLo = 16384, kSlabXs = 32768, kSlabS = 33792;
-constexpr int kSlabRows = 34;  // 1 KB DMA rows
-constexpr int kSlabBytes = kSlabRows * 1024;
-
-struct CtxP {
+    using I = XImage<HL, NT>;
     int lr, kh;
-    const uint8_t *x;  // the slab in LDS
-    __device__ __forceinline__ static int slot(int col, int xoff) { return (col << 5) | ((xoff >> 3) ^ (col & 31)); }
-    __device__ __forceinline__ half8 xh(int col, int xoff) const {
-        return *reinterpret_cast<const half8 *>(x + kSlabHi + 16 * slot(col, xoff));
+    const uint8_t *buf;
+    __device__ __forceinline__ half8 at(int half) const {
+        return *reinterpret_cast<const half8 *>(reinterpret_cast<const _Float16 *>(buf) + half);
     }
-    __device__ __forceinline__ half8 xl(int col, int xoff) const {
-        return *reinterpret_cast<const half8 *>(x + kSlabLo + 16 * slot(col, xoff));
-    }
-    __device__ __forceinline__ half8 xm(int col) const {
-        return *reinterpret_cast<const half8 *>(x + kSlabXs + 32 * col + 16 * kh);
-    }
-    __device__ __forceinline__ const float2 *S() const { return reinterpret_cast<const float2 *>(x + kSlabS); }
+    __device__ __forceinline__ half8 x(int n, int off) const { return at((32 * n + lr) * COLH + off); }
+    __device__ __forceinline__ half8 xlo(int n, int off) const { return at((32 * n + lr) * COLH + off + I::kLo); }
+    __device__ __forceinline__ half8 xs(int n) const { return at(I::kXs + (32 * n + lr) * 16 + 8 * kh); }
+    __device__ __forceinline__ half8 x16(int n, int limb) const { return at(I::kX16 + (32 * n + lr) * 32 + 16 * limb + 8 * kh); }
+    __device__ __forceinline__ const float *cs() const { return reinterpret_cast<const float *>(buf + I::kCs); }
 };
 
-// Operand roles: x is the A operand (its 32 rows are batch columns) and the
-// weights are B, so D[b][r] = sum_k x[b][k] w[r][k].  In the 32x32x16 layout
-// lane (lr, kh) supplies weight row lr (K elements 8kh .. 8kh+7) and holds
-// D for row lr and batch columns 8(i/4) + 4kh + (i%4), i < 16: every per-row
-// scale (d, dmin, d*sc) lives in the lane's own registers, and consecutive
-// lanes store consecutive rows.
-__device__ __forceinline__ int batch_of(int n, int i, int kh) { return n * 32 + 8 * (i >> 2) + 4 * kh + (i & 3); }
+// Prepared x (B <= 32): one super-block of the column group, laid out exactly as
+// the GEMM's LDS image so that it moves in as a contiguous DMA copy: the plane(s)
+// of 32 virtual columns x 32 units, the 32-value sums (32 x 16 halves), cs (32
+// floats), padding to whole KB.  Unit u of virtual column v sits at slot v * 32 +
+// (u ^ v): the XOR swizzle lets the 32 lanes that read unit u of 32 columns hit
+// distinct LDS banks without padding.
+template <bool HL>
+struct Slab {
+    static constexpr int kLo = 16384;  // !HL: the lo limbs' plane
+    static constexpr int kXs = HL ? 16384 : 32768, kCs = kXs + 1024;
+    static constexpr int kRows = kXs / 1024 + 2;  // 1 KB DMA rows
+    static constexpr int kBytes = kRows * 1024;
+    static __device__ __forceinline__ int slot(int v, int off) { return 16 * ((v << 5) | ((off >> 3) ^ v)); }
+    static __device__ __forceinline__ void store(uint8_t *slab, const float (&xv)[16], int q, int col) {
+        const XColumn x = split_x(xv);
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            *reinterpret_cast<half8 *>(slab + slot(col, 8 * (2 * q + u))) = x.h[u];
+            *reinterpret_cast<half8 *>(HL ? slab + slot(16 + col, 8 * (2 * q + u)) : slab + kLo + slot(col, 8 * (2 * q + u))) = x.l[u];
+        }
+        _Float16 *xs = reinterpret_cast<_Float16 *>(slab + kXs);
+        if ((q & 1) == 0) {
+            const _Float16 h = (_Float16)x.s32;
+            xs[col * 16 + (q >> 1)] = h;
+            xs[col * 16 + 8 + (q >> 1)] = (_Float16)(x.s32 - (float)h);
+        }
+        if (HL) xs[(16 + col) * 16 + q] = (_Float16)0.f;
+        if (q == 0) reinterpret_cast<float *>(slab + kCs)[col] = x.cs;
+    }
+};
+template <bool HL>
+struct CtxP {
+    using I = Slab<HL>;
+    int lr, kh;
+    const uint8_t *buf;  // the slab in LDS
+    __device__ __forceinline__ half8 x(int, int off) const { return *reinterpret_cast<const half8 *>(buf + I::slot(lr, off)); }
+    __device__ __forceinline__ half8 xlo(int, int off) const {
+        return *reinterpret_cast<const half8 *>(buf + I::kLo + I::slot(lr, off));
+    }
+    __device__ __forceinline__ half8 xs(int) const { return *reinterpret_cast<const half8 *>(buf + I::kXs + 32 * lr + 16 * kh); }
+    __device__ __forceinline__ half8 x16(int, int) const { return half8{}; }  // no format of this path reads them
+    __device__ __forceinline__ const float *cs() const { return reinterpret_cast<const float *>(buf + I::kCs); }
+};
 
-// four byte pairs of two words -> fp16 1024 + u in 16-bit lanes: one byte
-// permute per pair takes u from the word and the exponent byte 0x64 from a
-// constant second source
+// Operand roles: x is the A operand and the weights are B, so D[b][r] = sum_k
+// x[b][k] w[r][k].  In the 32x32x16 layout lane (lr, kh) supplies weight row lr (K
+// elements 8kh .. 8kh+7) and holds D for row lr and A rows 8(i/4) + 4kh + (i%4), i <
+// 16: every per-row scale (d, dmin, d*sc) lives in the lane's own registers, and
+// consecutive lanes store consecutive rows.  With HL, registers i >= 8 are the lo
+// limbs' sums of the columns of registers i - 8.
+__device__ __forceinline__ int batch_of(int n, int i, int kh) { return n * 32 + 8 * (i >> 2) + 4 * kh + (i & 3); }
+template <bool HL>
+constexpr int kOut = HL ? 8 : 16;  // outputs per lane and column group
+__device__ __forceinline__ f32x16 mfma(const half8 &x, const half8 &w, const f32x16 &c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w, c, 0, 0, 0);
+}
+// 1 / scale of the batch columns a lane holds for group n
+template <int NI, class C>
+__device__ __forceinline__ void col_scales(const C &c, int n, float (&cs)[NI]) {
+#pragma unroll
+    for (int i = 0; i < NI / 4; i++) {
+        const float4 v = *reinterpret_cast<const float4 *>(c.cs() + n * 32 + 8 * i + 4 * c.kh);
+        cs[4 * i] = v.x;
+        cs[4 * i + 1] = v.y;
+        cs[4 * i + 2] = v.z;
+        cs[4 * i + 3] = v.w;
+    }
+}
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ half2v dup(float v) { return half2v{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ half8 join(half2v a, half2v b, half2v c, half2v d) {
+    return half8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+// a constant held in a register: v_and_or_b32 takes one literal, not two
+__device__ __forceinline__ uint32_t in_vgpr(uint32_t v) {
+    asm("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+
+// the bytes of two words -> fp16 1024 + u - off in unit order: one byte permute
+// per pair takes two bytes and the exponent byte 0x64 from a constant
 __device__ __forceinline__ half8 bytes_to_h8(uint32_t w0, uint32_t w1, half2v off) {
     const uint32_t e = 0x64646464u;
-    const uint32_t p[4] = {__builtin_amdgcn_perm(e, w0, 0x04010400u), __builtin_amdgcn_perm(e, w0, 0x04030402u),
-                           __builtin_amdgcn_perm(e, w1, 0x04010400u), __builtin_amdgcn_perm(e, w1, 0x04030402u)};
-    half8 a;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const half2v h = __builtin_bit_cast(half2v, p[j]) - off;  // exact: small integers
-        a[2 * j] = h[0];
-        a[2 * j + 1] = h[1];
-    }
-    return a;
+    return join(as_h2(__builtin_amdgcn_perm(e, w0, 0x04020400u)) - off, as_h2(__builtin_amdgcn_perm(e, w0, 0x04030401u)) - off,
+                as_h2(__builtin_amdgcn_perm(e, w1, 0x04020400u)) - off, as_h2(__builtin_amdgcn_perm(e, w1, 0x04030401u)) - off);
 }
-
-// acc[n] += x_hi . w + x_lo . w over one K-step (x columns at xoff)
-template <int NT, class C>
-__device__ __forceinline__ void mfma_xw(const C &c, const half8 &w, int xoff, f32x16 *acc) {
-#pragma unroll
-    for (int n = 0; n < NT; n++) {
-        const int col = n * 32 + c.lr;
-        const half8 xh = c.xh(col, xoff);
-        const half8 xl = c.xl(col, xoff);
-        acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, w, acc[n], 0, 0, 0);
-        acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, w, acc[n], 0, 0, 0);
-    }
-}
-
-// (S, 1/scale) of the 16 batch columns a lane holds for tile n
-template <int NT, class C>
-__device__ __forceinline__ void col_terms(const C &c, int n, float (&S)[16], float (&cs)[16]) {
-#pragma unroll
-    for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const float4 v = *reinterpret_cast<const float4 *>(c.S() + n * 32 + 8 * q + 4 * c.kh + 2 * h);
-            S[4 * q + 2 * h] = v.x;
-            cs[4 * q + 2 * h] = v.y;
-            S[4 * q + 2 * h + 1] = v.z;
-            cs[4 * q + 2 * h + 1] = v.w;
-        }
+// the same in natural order (the operands that meet the sums of x)
+__device__ __forceinline__ half8 bytes_to_h8_plain(uint32_t w0, uint32_t w1, half2v off) {
+    const uint32_t e = 0x64646464u;
+    return join(as_h2(__builtin_amdgcn_perm(e, w0, 0x04010400u)) - off, as_h2(__builtin_amdgcn_perm(e, w0, 0x04030402u)) - off,
+                as_h2(__builtin_amdgcn_perm(e, w1, 0x04010400u)) - off, as_h2(__builtin_amdgcn_perm(e, w1, 0x04030402u)) - off);
 }
 
 // N dwords at a 2-byte-aligned LDS address, read as aligned dwords and
@@ -298,29 +343,82 @@ __device__ __forceinline__ u32x4 lds_u32x4(const uint8_t *p) {
 template <int CH, int RC>
 __device__ __forceinline__ int win_chunk(int j) { return RC == CH ? j : j + (RC - CH) * (j / CH); }
 
+// ------------------------------------------------------------------ format policies
+// Each format supplies, for one 256-column stretch ("super-block") of a row:
+//   Regs                  the lane's weight bytes (row lr, K half kh), in VGPRs
+//   load(r, p, kh)        p = first byte of the row's stretch, in LDS
+//   compute<HL, NT>(...)  the MFMAs and the fold into the fp32 totals
+// K-step t covers 16 columns; lane half kh supplies 8 of them.  Every weight
+// enters the MFMA as an exact fp16 integer (or half-integer); scales are applied
+// in fp32.  Quants of a sub-block with a nonzero min are centred (Q4_K q - 8, Q5_K
+// q - 16, Q2_K q - 1.5): the products then have the size of the weights
+// themselves, and what the centre took out comes back with the min term from the
+// sums of x.  Uncentred, the accumulators carry that offset through every
+// rounding (N(0, 0.02) weights, K = 4096: error against 64 bits 3.95e-7 for Q4_K).
+// A sub-block whose min is 0 is not centred: its weights with q = 0 are exactly
+// zero, and must stay so under an x of any size.
+
+// acc (+)= x . w over one K-step at column offset off: the hi limbs' MFMA, then the
+// lo limbs' into the same sum (HL: one MFMA, the two sums in different registers).
+// The hi limbs come first: with the lo limbs' sum as the accumulator input, the
+// MFMA drops its low bits always in one direction, a bias that adds up over K
+// (Q8_0, K = 14336: 1.73e-7 against 1.24e-7).
+template <bool HL, int NT, class C>
+__device__ __forceinline__ void mfma_xw(const C &c, const half8 &w, int off, f32x16 (&acc)[NT]) {
+#pragma unroll
+    for (int n = 0; n < NT; n++) acc[n] = mfma(c.x(n, off), w, acc[n]);
+    if constexpr (!HL) {
+#pragma unroll
+        for (int n = 0; n < NT; n++) acc[n] = mfma(c.xlo(n, off), w, acc[n]);
+    }
+}
+// part += ds * acc
+template <int NT>
+__device__ __forceinline__ void fold(f32x16 (&part)[NT], float ds, const f32x16 (&acc)[NT]) {
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) part[n][i] = fmaf(ds, acc[n][i], part[n][i]);
+}
+// Ends a run of K-steps: the folds are done here, and no operand read of the next
+// run has started.  Without it the compiler issues the reads of all K-steps first
+// and keeps their sums to the end, which spills.
+template <int NT>
+__device__ __forceinline__ void step_fence(f32x16 (&part)[NT]) {
+#pragma unroll
+    for (int n = 0; n < NT; n++) asm volatile("" : "+v"(part[n]));
+    __builtin_amdgcn_sched_barrier(0);
+}
+// tot += cs * (the super-block's folded sums)
+template <bool HL, int NT, class C>
+__device__ __forceinline__ void fold_columns(const C &c, const f32x16 (&part)[NT], float (&tot)[NT][kOut<HL>]) {
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        float cs[kOut<HL>];
+        col_scales(c, n, cs);
+#pragma unroll
+        for (int i = 0; i < kOut<HL>; i++)
+            tot[n][i] = fmaf(cs[i], HL ? part[n][i] + part[n][(i + 8) & 15] : part[n][i], tot[n][i]);
+    }
+}
+
 // Q4_K (matVecQ4Kraw, LlamaTransformerHandler.java:1428-1468): w = d*ls*q - dmin*lm.
-// B = ls*q (<= 945, exact), built as fp16 1024 + ls*q by one 24-bit multiply-
-// add per pair into the exponent byte and one packed fp16 subtraction of 1024
-// (exact); the min term (one more MFMA: A = [sub-block sums hi | lo], B =
-// [lm | lm]) is removed per super-block with d and dmin.  Keeping the 1024 in
-// B and subtracting 1024 * sum(x) afterwards would cost fp32 cancellation
-// wherever |x| is large and the row's weights there are small.
-// Q5_K (Q5 = true, matVecQ5Kraw :1525-1576): q has a 5th bit from qh, so
-// ls*q reaches 1953 and 1024 + ls*q would pass fp16's exact integers; B =
-// ls*q is converted instead (v_cvt_f16_u16, exact below 2048).
+// B = ls*(q - C), C = 8 where lm is not 0, |.| <= 945: a nibble moved to bits 4..7
+// under fp16 64's exponent is 64 + q (one shift, one and-or per pair), and one
+// packed FMA gives (64 + q) ls - (64 + C) ls, exact.  Q5_K (Q5 = true,
+// matVecQ5Kraw :1525-1576): q has a 5th bit from qh, bits 4..8, C = 16, |.| <= 1953.
 template <bool Q5>
 struct FmtKQ {
     static constexpr int kBytes = Q5 ? 176 : 144;
+    static constexpr int kSums = 32;  // sums of x it reads (0, 16 or 32 values each)
     static constexpr int kChunks = kBytes / 16;  // rows are 16-byte aligned (pitch kBytes * n, aligned base)
     static constexpr int kRowChunks = kChunks;   // LDS window row stride (16-byte chunks)
     static constexpr int kQs = Q5 ? 48 : 16;
-    static constexpr bool kSums = true;
     struct Regs {
         u32x4 hd;
         u32x2 qp[4][2];
         u32x2 qh[2];  // Q5_K: qh bytes 16 j + 8 kh .. +8 (bit s for sub-block s)
     };
-    template <bool RA>  // rows are 16-byte aligned: the reads are aligned either way
     static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int kh) {
         r.hd = *reinterpret_cast<const u32x4 *>(p);
 #pragma unroll
@@ -333,68 +431,63 @@ struct FmtKQ {
             r.qh[1] = *reinterpret_cast<const u32x2 *>(p + 32 + 8 * kh);
         }
     }
-    template <int NT, class C>
-    static __device__ __forceinline__ void compute(const Regs &r, const C &c, f32x16 *tot) {
-        // 6-bit scales and mins of the 8 sub-blocks (q4kScaleRaw / q4kMinRaw, :1471-1482)
-        int ls[8], lm[8];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            ls[j] = (int)byte_of(r.hd.y, j) & 63;
-            lm[j] = (int)byte_of(r.hd.z, j) & 63;
-            ls[j + 4] = (int)((byte_of(r.hd.w, j) & 0x0F) | ((byte_of(r.hd.y, j) & 0xC0) >> 2));
-            lm[j + 4] = (int)((byte_of(r.hd.w, j) >> 4) | ((byte_of(r.hd.z, j) & 0xC0) >> 2));
+    // the pair of one dword's bytes (odd ? (b1, b3) : (b0, b2)) of sub-block s
+    template <int S, int ODD>
+    static __device__ __forceinline__ half2v pair(uint32_t w, uint32_t hb, half2v ls, half2v off, uint32_t top) {
+        constexpr int sh = (S & 1 ? 4 : 0) + 8 * ODD - 4;  // the nibble's bit within the half word, to bit 4
+        if (Q5) {
+            constexpr int hs = S + 8 * ODD - 8;  // the 5th bit, to bit 8
+            const uint32_t v = hs > 0 ? hb >> (hs > 0 ? hs : 0) : hb << (hs < 0 ? -hs : 0);
+            top |= v & 0x01000100u;
         }
-        const half2v k1024 = {(_Float16)1024.f, (_Float16)1024.f};
+        const uint32_t v = sh > 0 ? w >> (sh > 0 ? sh : 0) : w << (sh < 0 ? -sh : 0);
+        return __builtin_elementwise_fma(as_h2((v & 0x00F000F0u) | top), ls, off);
+    }
+    template <bool HL, int NT, class C>
+    static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
+        // 6-bit scales and mins of the 8 sub-blocks, one per byte (q4kScaleRaw / q4kMinRaw, :1471-1482),
+        // and their centres: 8 (Q5_K 16) where the min is not zero
+        uint32_t ls4[2], lm4[2], c4[2];
+        ls4[0] = r.hd.y & 0x3F3F3F3Fu;
+        lm4[0] = r.hd.z & 0x3F3F3F3Fu;
+        ls4[1] = (r.hd.w & 0x0F0F0F0Fu) | ((r.hd.y >> 2) & 0x30303030u);
+        lm4[1] = ((r.hd.w >> 4) & 0x0F0F0F0Fu) | ((r.hd.z >> 2) & 0x30303030u);
+#pragma unroll
+        for (int h = 0; h < 2; h++) c4[h] = ((lm4[h] + 0x3F3F3F3Fu) & 0x40404040u) >> (Q5 ? 2 : 3);
+        const half2v k1024 = dup(1024.f);
+        const uint32_t top = in_vgpr(0x54005400u);
         f32x16 acc[NT];
 #pragma unroll
         for (int n = 0; n < NT; n++) acc[n] = (f32x16){};
-#pragma unroll
-        for (int t = 0; t < 16; t++) {
-            // sub-block s = t/2: low nibbles of qs group s/2 for even s, high for odd
-            const int s = t >> 1, g = s >> 1, hiN = s & 1;
-            const u32x2 q = r.qp[g][t & 1];
-            uint32_t nib0 = hiN ? (q.x >> 4) & 0x0F0F0F0Fu : q.x & 0x0F0F0F0Fu;
-            uint32_t nib1 = hiN ? (q.y >> 4) & 0x0F0F0F0Fu : q.y & 0x0F0F0F0Fu;
-            if (Q5) {
-                const u32x2 h = r.qh[t & 1];
-                nib0 |= ((h.x >> s) & 0x01010101u) << 4;
-                nib1 |= ((h.y >> s) & 0x01010101u) << 4;
-            }
-            const uint32_t pr[4] = {__builtin_amdgcn_perm(0u, nib0, 0x0C010C00u),
-                                    __builtin_amdgcn_perm(0u, nib0, 0x0C030C02u),
-                                    __builtin_amdgcn_perm(0u, nib1, 0x0C010C00u),
-                                    __builtin_amdgcn_perm(0u, nib1, 0x0C030C02u)};
-            half8 w;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (Q5) {
-                    const uint32_t v = __umul24(pr[j], (uint32_t)ls[s]);  // two 16-bit products <= 1953
-                    w[2 * j] = (_Float16)(uint16_t)(v & 0xFFFF);
-                    w[2 * j + 1] = (_Float16)(uint16_t)(v >> 16);
-                } else {
-                    // 1024 + ls*q by the exponent byte, then 1024 off in fp16: exact, and
-                    // the MFMA sums stay the size of the weights' own products
-                    const uint32_t v = __umul24(pr[j], (uint32_t)ls[s]) + 0x64006400u;
-                    const half2v h = __builtin_bit_cast(half2v, v) - k1024;
-                    w[2 * j] = h[0];
-                    w[2 * j + 1] = h[1];
-                }
-            }
-            mfma_xw<NT>(c, w, 16 * t + 8 * c.kh, acc);
-        }
-        half8 wm;
-#pragma unroll
-        for (int j = 0; j < 8; j++) wm[j] = (_Float16)lm[j];
+        for_c<8>([&](auto si) {
+            constexpr int S = decltype(si)::value, g = S / 2;
+            constexpr uint32_t sel = 0x04000400u + 0x00010001u * (S % 4);  // byte S % 4 under the exponent byte, twice
+            const half2v ls = as_h2(__builtin_amdgcn_perm(0x64646464u, ls4[S / 4], sel)) - k1024;
+            const half2v off = ls * (dup(960.f) - as_h2(__builtin_amdgcn_perm(0x64646464u, c4[S / 4], sel)));  // -(64 + C) ls
+            for_c<2>([&](auto oi) {
+                constexpr int o = decltype(oi)::value;
+                const u32x2 q = r.qp[g][o], h = Q5 ? r.qh[o] : u32x2{0u, 0u};
+                mfma_xw<HL, NT>(c, join(pair<S, 0>(q.x, h.x, ls, off, top), pair<S, 1>(q.x, h.x, ls, off, top),
+                                        pair<S, 0>(q.y, h.y, ls, off, top), pair<S, 1>(q.y, h.y, ls, off, top)),
+                                16 * (2 * S + o) + 8 * c.kh, acc);
+            });
+        });
+        // the centre's share and the min term, from the sums of x: C ls X and lm X with X = 2^-5 sum(x)
+        const half2v mm = dup((float)(1 << kXsShift));
+        const half8 wm = bytes_to_h8_plain(lm4[0], lm4[1], k1024) * join(mm, mm, mm, mm);
+        const half8 wl = bytes_to_h8_plain(ls4[0], ls4[1], k1024) *
+                         (bytes_to_h8_plain(c4[0], c4[1], k1024) * join(mm, mm, mm, mm));
         const float d = half_bits_to_float(r.hd.x), dmin = half_bits_to_float(r.hd.x >> 16);
 #pragma unroll
         for (int n = 0; n < NT; n++) {
-            const int col = n * 32 + c.lr;
-            const half8 xm = c.xm(col);
-            const f32x16 mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(xm, wm, (f32x16){}, 0, 0, 0);
-            float S[16], cs[16];
-            col_terms<NT>(c, n, S, cs);
+            if (NT > 1) __builtin_amdgcn_sched_barrier(0);  // one column group's sums at a time
+            const half8 xs = c.xs(n);
+            const f32x16 a = mfma(xs, wl, acc[n]), mn = mfma(xs, wm, (f32x16){});
+            float cs[kOut<HL>];
+            col_scales(c, n, cs);
 #pragma unroll
-            for (int i = 0; i < 16; i++) tot[n][i] = fmaf(cs[i], fmaf(d, acc[n][i], -dmin * mn[i]), tot[n][i]);
+            for (int i = 0; i < kOut<HL>; i++)
+                tot[n][i] = fmaf(cs[i], fmaf(d, HL ? a[i] + a[(i + 8) & 15] : a[i], -dmin * mn[i]), tot[n][i]);
         }
     }
 };
@@ -408,43 +501,40 @@ using FmtQ5K = FmtKQ<true>;
 // d*sc_j of the lane's row (the reference's dN).  Step t = 8n + 2qd + j
 // covers columns 128n + 32qd + 16j .. +16 and uses scale t.
 struct FmtQ6K {
+    static constexpr int kSums = 0;
     static constexpr int kBytes = 210;
     static constexpr int kChunks = (kBytes + 14 + 15) / 16;  // a 2-byte-aligned block spans <= 14 chunks
     // window rows 15 chunks (60 dwords) apart: the dword reads of 32 rows hit 16
     // banks (2-way) instead of the 8 of a 56-dword stride
     static constexpr int kRowChunks = kChunks + 1;
-    static constexpr bool kSums = false;
     struct Regs {
         u32x2 ql[2][2][2];  // [half n][ql +32 p][j]: bytes 64n + 32p + 16j + 8kh
         u32x2 qh[2][2];     // [n][j]: bytes 128 + 32n + 16j + 8kh
         u32x4 sc;           // bytes 192..207
         uint32_t dw;        // bytes 206..209: d in the high half
     };
-    template <bool RA>  // realign in registers (aligned LDS reads) or read the 2-byte-aligned fields directly
     static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int kh) {
 #pragma unroll
         for (int n = 0; n < 2; n++)
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const uint8_t *a = p + 64 * n + 16 * j + 8 * kh, *h = p + 128 + 32 * n + 16 * j + 8 * kh;
-                r.ql[n][0][j] = RA ? lds_u32x2(a) : *reinterpret_cast<const u32x2a2 *>(a);
-                r.ql[n][1][j] = RA ? lds_u32x2(a + 32) : *reinterpret_cast<const u32x2a2 *>(a + 32);
-                r.qh[n][j] = RA ? lds_u32x2(h) : *reinterpret_cast<const u32x2a2 *>(h);
+                const uint8_t *a = p + 64 * n + 16 * j + 8 * kh;
+                r.ql[n][0][j] = lds_u32x2(a);
+                r.ql[n][1][j] = lds_u32x2(a + 32);
+                r.qh[n][j] = lds_u32x2(p + 128 + 32 * n + 16 * j + 8 * kh);
             }
-        if (RA) {
-            r.sc = lds_u32x4(p + 192);
-            uint32_t dw[1];
-            lds_read_u<1>(p + 206, dw);
-            r.dw = dw[0];
-        } else {
-            r.sc = *reinterpret_cast<const u32x4a2 *>(p + 192);
-            r.dw = *reinterpret_cast<const u32a2 *>(p + 206);
-        }
+        r.sc = lds_u32x4(p + 192);
+        uint32_t dw[1];
+        lds_read_u<1>(p + 206, dw);
+        r.dw = dw[0];
     }
-    template <int NT, class C>
-    static __device__ __forceinline__ void compute(const Regs &r, const C &c, f32x16 *tot) {
-        const half2v off = {(_Float16)1056.f, (_Float16)1056.f};  // 1024 + 32
+    template <bool HL, int NT, class C>
+    static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
+        const half2v off = dup(1056.f);  // 1024 + 32
         const float d = half_bits_to_float(r.dw >> 16);
+        f32x16 part[NT];
+#pragma unroll
+        for (int n = 0; n < NT; n++) part[n] = (f32x16){};
 #pragma unroll
         for (int t = 0; t < 16; t++) {
             const int n = t >> 3, qd = (t >> 1) & 3, j = t & 1;
@@ -454,13 +544,11 @@ struct FmtQ6K {
             f32x16 acc[NT];
 #pragma unroll
             for (int m = 0; m < NT; m++) acc[m] = (f32x16){};
-            mfma_xw<NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
-            const float ds = d * (float)(int8_t)byte_of(t < 4 ? r.sc.x : t < 8 ? r.sc.y : t < 12 ? r.sc.z : r.sc.w, t & 3);
-#pragma unroll
-            for (int m = 0; m < NT; m++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) tot[m][i] = fmaf(ds, acc[m][i], tot[m][i]);
+            mfma_xw<HL, NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
+            fold<NT>(part, d * (float)(int8_t)byte_of(t < 4 ? r.sc.x : t < 8 ? r.sc.y : t < 12 ? r.sc.z : r.sc.w, t & 3), acc);
+            if (t % (NT > 1 ? 2 : 4) == (NT > 1 ? 1 : 3)) step_fence(part);
         }
+        fold_columns<HL, NT>(c, part, tot);
     }
 };
 
@@ -468,43 +556,41 @@ struct FmtQ6K {
 // of 34 B per 256 columns.  Lane half kh holds columns 16kh .. 16kh+15 of
 // block b (one 16-byte load), split over the block's two K-steps; B = q exact.
 struct FmtQ8_0 {
+    static constexpr int kSums = 0;
     static constexpr int kBytes = 8 * 34;
     static constexpr int kChunks = (kBytes + 14 + 15) / 16;
     static constexpr int kRowChunks = kChunks + 1;  // 76-dword window rows (see FmtQ6K)
-    static constexpr bool kSums = false;
     struct Regs {
-        u32x4 q[8];     // block b: bytes 34b + 2 + 16kh .. +16
-        uint32_t d[8];  // d of block b (low half)
+        const uint8_t *p;  // 40 registers of quants and scales would spill: each block is read ahead of its MFMAs
     };
-    template <bool RA>
-    static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int kh) {
+    static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int) { r.p = p; }
+    template <bool HL, int NT, class C>
+    static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
+        const half2v off = dup(1152.f);  // 1024 + 128
+        f32x16 part[NT];
+#pragma unroll
+        for (int n = 0; n < NT; n++) part[n] = (f32x16){};
+        u32x4 q = lds_u32x4(r.p + 2 + 16 * c.kh);  // block b: bytes 34b + 2 + 16kh .. +16
+        uint32_t d = *reinterpret_cast<const uint16_t *>(r.p);
 #pragma unroll
         for (int b = 0; b < 8; b++) {
-            const uint8_t *a = p + 34 * b + 2 + 16 * kh;
-            r.q[b] = RA ? lds_u32x4(a) : *reinterpret_cast<const u32x4a2 *>(a);
-            r.d[b] = *reinterpret_cast<const uint16_t *>(p + 34 * b);
-        }
-    }
-    template <int NT, class C>
-    static __device__ __forceinline__ void compute(const Regs &r, const C &c, f32x16 *tot) {
-        const half2v off = {(_Float16)1152.f, (_Float16)1152.f};  // 1024 + 128
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
+            const u32x4 qb = q;
+            const uint32_t db = d;
+            if (b < 7) {
+                q = lds_u32x4(r.p + 34 * (b + 1) + 2 + 16 * c.kh);
+                d = *reinterpret_cast<const uint16_t *>(r.p + 34 * (b + 1));
+            }
             f32x16 acc[NT];
 #pragma unroll
             for (int m = 0; m < NT; m++) acc[m] = (f32x16){};
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const uint32_t w0 = (j ? r.q[b].z : r.q[b].x) ^ 0x80808080u;  // q + 128
-                const uint32_t w1 = (j ? r.q[b].w : r.q[b].y) ^ 0x80808080u;
-                mfma_xw<NT>(c, bytes_to_h8(w0, w1, off), 32 * b + 16 * c.kh + 8 * j, acc);
-            }
-            const float d = half_bits_to_float(r.d[b]);
-#pragma unroll
-            for (int m = 0; m < NT; m++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) tot[m][i] = fmaf(d, acc[m][i], tot[m][i]);
+            for (int j = 0; j < 2; j++)
+                mfma_xw<HL, NT>(c, bytes_to_h8((j ? qb.z : qb.x) ^ 0x80808080u, (j ? qb.w : qb.y) ^ 0x80808080u, off),
+                                32 * b + 16 * c.kh + 8 * j, acc);
+            fold<NT>(part, half_bits_to_float(db), acc);
+            if (HL || NT > 1) step_fence(part);
         }
+        fold_columns<HL, NT>(c, part, tot);
     }
 };
 
@@ -512,20 +598,25 @@ struct FmtQ8_0 {
 // [qs 64][d][dmin]; element 128h + 16k + l takes 2 bits at shift 2(k/2) of
 // qs[32h + 16(k&1) + l] and sub-block scale byte sc[8h + k] (low nibble scale,
 // high nibble min): w = d*(sc&15)*q - dmin*(sc>>4).  A 16-column sub-block is one
-// K-step t = 8h + k: B = q (exact), folded per K-step with d*(sc&15); the min
-// term is one MFMA pair per super-block against the 16-column sums of x.
+// K-step t = 8h + k: B = (sc&15)*(q - C), C = 1.5 where the min is not 0 (|.| <= 45,
+// exact: the 2 bits at bits 4..5 under fp16 64's exponent, then one packed FMA);
+// the centre's share and the min term are MFMAs per super-block against the
+// 16-column sums of x.  The sums are folded with d every 8 K-steps: every 16 is
+// 6 % faster at B = 48 but its error against 64 bits (K = 1024: 1.77e-7) is larger
+// than the VALU kernel's 1.61e-7; every 8 gives 1.52e-7, every 4 1.40e-7 (and
+// folding each K-step with d*(sc&15) is 7 % slower).
 // Blocks are 4-byte aligned (84 = 4 * 21).
 struct FmtQ2K {
+    static constexpr int kSums = 16;
     static constexpr int kBytes = 84;
     static constexpr int kChunks = (kBytes + 12 + 15) / 16;  // a 4-byte-aligned block spans <= 6 chunks
     static constexpr int kRowChunks = kChunks + 1;           // 28-dword window rows (2-way bank conflicts)
-    static constexpr bool kSums = false;
+    static constexpr int kFold = 8;  // K-steps per fold: see above
     struct Regs {
         u32x2 q[2][2];  // [h][k&1]: qs bytes 32h + 16(k&1) + 8kh .. +8
         u32x4 sc;       // the 16 scale bytes
         uint32_t dm;    // d (low half), dmin (high half)
     };
-    template <bool RA>
     static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int kh) {
 #pragma unroll
         for (int h = 0; h < 2; h++)
@@ -536,38 +627,59 @@ struct FmtQ2K {
         lds_read_u<1>(p + 80, dm);
         r.dm = dm[0];
     }
-    template <int NT, class C>
-    static __device__ __forceinline__ void compute(const Regs &r, const C &c, f32x16 *tot) {
-        const half2v off = {(_Float16)1024.f, (_Float16)1024.f};
+    template <int J, int ODD>
+    static __device__ __forceinline__ half2v pair(uint32_t w, half2v sc, half2v off, uint32_t top) {
+        constexpr int sh = 2 * J + 8 * ODD - 4;  // the 2 bits' place within the half word, to bit 4
+        const uint32_t v = sh > 0 ? w >> (sh > 0 ? sh : 0) : w << (sh < 0 ? -sh : 0);
+        return __builtin_elementwise_fma(as_h2((v & 0x00300030u) | top), sc, off);
+    }
+    template <bool HL, int NT, class C>
+    static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const float d = half_bits_to_float(r.dm), dmin = half_bits_to_float(r.dm >> 16);
-        auto scb = [&](int t) { return byte_of(t < 4 ? r.sc.x : t < 8 ? r.sc.y : t < 12 ? r.sc.z : r.sc.w, t & 3); };
+        const uint32_t top = in_vgpr(0x54005400u);
+        const half2v k = dup(1024.f);
+        // the low byte of each sub-block's fp16 64 + C: 0x18 where the min is not 0
+        uint32_t c4[4], m4[4], s4[4];
 #pragma unroll
-        for (int t = 0; t < 16; t++) {
-            const int h = t >> 3, k = t & 7;
-            const u32x2 q = r.q[h][k & 1];
-            const uint32_t u0 = (q.x >> (2 * (k >> 1))) & 0x03030303u, u1 = (q.y >> (2 * (k >> 1))) & 0x03030303u;
-            f32x16 acc[NT];
-#pragma unroll
-            for (int m = 0; m < NT; m++) acc[m] = (f32x16){};
-            mfma_xw<NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
-            const float ds = d * (float)(scb(t) & 15u);
-#pragma unroll
-            for (int m = 0; m < NT; m++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) tot[m][i] = fmaf(ds, acc[m][i], tot[m][i]);
+        for (int i = 0; i < 4; i++) {
+            m4[i] = (r.sc[i] >> 4) & 0x0F0F0F0Fu;
+            s4[i] = r.sc[i] & 0x0F0F0F0Fu;
+            c4[i] = ((m4[i] + 0x0F0F0F0Fu) & 0x10101010u) * 3u >> 1;
         }
-        // min term: sum_t (sc_t >> 4) * X16_t, K-half kh holding t = 8kh .. 8kh+7
-        half8 wm;
+        f32x16 part[NT], acc[NT];
 #pragma unroll
-        for (int j = 0; j < 8; j++) wm[j] = (_Float16)(float)(scb(8 * c.kh + j) >> 4);
+        for (int n = 0; n < NT; n++) part[n] = (f32x16){};
+        for_c<16>([&](auto ti) {
+            constexpr int t = decltype(ti)::value, J = (t & 7) >> 1;
+            constexpr uint32_t sel = 0x04000400u + 0x00010001u * (t & 3);
+            const u32x2 q = r.q[t >> 3][t & 1];
+            const half2v sc = as_h2(__builtin_amdgcn_perm(0x64646464u, s4[t >> 2], sel)) - k;
+            const half2v off = -sc * as_h2(__builtin_amdgcn_perm(0x54545454u, c4[t >> 2], sel));  // -(64 + C) sc
+            if constexpr (t % kFold == 0) {
+#pragma unroll
+                for (int m = 0; m < NT; m++) acc[m] = (f32x16){};
+            }
+            mfma_xw<HL, NT>(c, join(pair<J, 0>(q.x, sc, off, top), pair<J, 1>(q.x, sc, off, top), pair<J, 0>(q.y, sc, off, top),
+                                    pair<J, 1>(q.y, sc, off, top)),
+                            16 * t + 8 * c.kh, acc);
+            if constexpr (t % kFold == kFold - 1) fold<NT>(part, d, acc);
+        });
+        // centre and min term: sum_t C (sc_t & 15) X16_t and (sc_t >> 4) X16_t with X16 = 2^-4 sum(x), K half kh
+        // holding t = 8kh .. 8kh+7
+        const half2v mm = dup((float)(1 << kX16Shift)), centre = dup(1.5f);
+        // the scales of the centred sub-blocks: bytes with a nonzero min keep theirs
+        const uint32_t k0 = (((c.kh ? c4[2] : c4[0]) >> 4) & 0x01010101u) * 15u, k1 = (((c.kh ? c4[3] : c4[1]) >> 4) & 0x01010101u) * 15u;
+        const half2v cm = mm * centre;
+        const half8 wl = bytes_to_h8_plain((c.kh ? s4[2] : s4[0]) & k0, (c.kh ? s4[3] : s4[1]) & k1, k) * join(cm, cm, cm, cm);
+        const half8 wm = bytes_to_h8_plain(c.kh ? m4[2] : m4[0], c.kh ? m4[3] : m4[1], k) * join(mm, mm, mm, mm);
 #pragma unroll
         for (int n = 0; n < NT; n++) {
-            const int col = n * 32 + c.lr;
-            f32x16 mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(c.x16h(col), wm, (f32x16){}, 0, 0, 0);
-            mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(c.x16l(col), wm, mn, 0, 0, 0);
+            const half8 xh = c.x16(n, 0), xl = c.x16(n, 1);
+            const f32x16 ct = mfma(xl, wl, mfma(xh, wl, (f32x16){})), mn = mfma(xl, wm, mfma(xh, wm, (f32x16){}));
 #pragma unroll
-            for (int i = 0; i < 16; i++) tot[n][i] = fmaf(-dmin, mn[i], tot[n][i]);
+            for (int i = 0; i < 16; i++) part[n][i] += fmaf(d, ct[i], -dmin * mn[i]);
         }
+        fold_columns<HL, NT>(c, part, tot);
     }
 };
 
@@ -578,16 +690,15 @@ struct FmtQ2K {
 // w = d*(sc - 32)*(q - 4).  B = q - 4 (exact), folded per K-step.  Blocks are
 // 2-byte aligned: fields are read as aligned dwords and realigned.
 struct FmtQ3K {
+    static constexpr int kSums = 0;
     static constexpr int kBytes = 110;
     static constexpr int kChunks = (kBytes + 14 + 15) / 16;  // a 2-byte-aligned block spans <= 8 chunks
     static constexpr int kRowChunks = kChunks + 1;           // 36-dword window rows (2-way bank conflicts)
-    static constexpr bool kSums = false;
     struct Regs {
         u32x2 q[2][2];  // [h][r]: qs bytes 32 + 32h + 16r + 8kh .. +8
         u32x2 hm[2];    // [r]: hmask bytes 16r + 8kh .. +8
         u32x4 sd;       // scale bytes 96..107 (aux0, aux1, aux2), then d in the low half of .w
     };
-    template <bool RA>
     static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int kh) {
 #pragma unroll
         for (int h = 0; h < 2; h++)
@@ -597,9 +708,12 @@ struct FmtQ3K {
         for (int o = 0; o < 2; o++) r.hm[o] = lds_u32x2(p + 16 * o + 8 * kh);
         r.sd = lds_u32x4(p + 96);
     }
-    template <int NT, class C>
-    static __device__ __forceinline__ void compute(const Regs &r, const C &c, f32x16 *tot) {
-        const half2v off = {(_Float16)1028.f, (_Float16)1028.f};  // 1024 + 4
+    template <bool HL, int NT, class C>
+    static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
+        const half2v off = dup(1028.f);  // 1024 + 4
+        f32x16 part[NT];
+#pragma unroll
+        for (int n = 0; n < NT; n++) part[n] = (f32x16){};
         const float d = half_bits_to_float(r.sd.w);
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -619,15 +733,26 @@ struct FmtQ3K {
                     f32x16 acc[NT];
 #pragma unroll
                     for (int m = 0; m < NT; m++) acc[m] = (f32x16){};
-                    mfma_xw<NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
+                    mfma_xw<HL, NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
                     const int s6 = (int)byte_of(j < 2 ? ua : ub, 2 * (j & 1) + rr) - 32;
-                    const float ds = d * (float)s6;
-#pragma unroll
-                    for (int m = 0; m < NT; m++)
-#pragma unroll
-                        for (int i = 0; i < 16; i++) tot[m][i] = fmaf(ds, acc[m][i], tot[m][i]);
+                    fold<NT>(part, d * (float)s6, acc);
                 }
         }
+        fold_columns<HL, NT>(c, part, tot);
+    }
+};
+
+// A wave's 32 weight rows (past the end: the last row again): a wave-uniform
+// 16-byte-aligned base and 32-bit offsets from it, which cost a lane half the
+// registers of addresses.  mfma_applies bounds the pitch so that they hold.
+struct RowSpan {
+    size_t pitch;
+    int row0, rbase, nrows;
+    __device__ __forceinline__ int row(int rho) const { return min(rbase + rho, nrows - 1); }
+    __device__ __forceinline__ size_t first() const { return (size_t)(row0 + row(0)) * pitch; }
+    __device__ __forceinline__ size_t base() const { return first() & ~size_t(15); }
+    __device__ __forceinline__ uint32_t offset(int rho) const {
+        return (uint32_t)(first() & 15) + (uint32_t)(row(rho) - row(0)) * (uint32_t)pitch;
     }
 };
 
@@ -643,8 +768,8 @@ struct FmtQ3K {
 // launch costs ~5 us.
 constexpr int kMaxTileCounters = kCounterSlots;
 
-template <int NT>
-__device__ __forceinline__ void store_tile(const f32x16 (&tot)[NT], int r, int nrows, int kh, int B, float *__restrict__ Y,
+template <int NT, int NI>
+__device__ __forceinline__ void store_tile(const float (&tot)[NT][NI], int r, int nrows, int kh, int B, float *__restrict__ Y,
                                            float *part, int *counters, int tile, int split, int ksplit) {
     const bool live = r < nrows;
     if (ksplit == 1) {
@@ -652,7 +777,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&tot)[NT], int r, int n
 #pragma unroll
         for (int n = 0; n < NT; n++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
+            for (int i = 0; i < NI; i++) {
                 const int b = batch_of(n, i, kh);
                 if (b < B) Y[(size_t)b * nrows + r] = tot[n][i];
             }
@@ -664,7 +789,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&tot)[NT], int r, int n
 #pragma unroll
         for (int n = 0; n < NT; n++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
+            for (int i = 0; i < NI; i++) {
                 const int b = batch_of(n, i, kh);
                 if (b < B) __hip_atomic_store(mine + (size_t)b * nrows + r, tot[n][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -695,20 +820,20 @@ __device__ __forceinline__ void store_tile(const f32x16 (&tot)[NT], int r, int n
     // KB splits' partials in flight at a time, added in split order
     constexpr int KB = 4 / NT;
     const int ks = ksplit;
-    float acc[NT][16];
+    float acc[NT][NI];
 #pragma unroll
     for (int n = 0; n < NT; n++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[n][i] = 0.f;
+        for (int i = 0; i < NI; i++) acc[n][i] = 0.f;
     for (int k0 = 0; k0 < ks; k0 += KB) {
-        float v[KB][NT][16];
+        float v[KB][NT][NI];
 #pragma unroll
         for (int kk = 0; kk < KB; kk++) {
             const int k = k0 + kk;
 #pragma unroll
             for (int n = 0; n < NT; n++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
+                for (int i = 0; i < NI; i++) {
                     // unconditional (clamped) loads, so that they issue back to back;
                     // this split's own partial comes back from memory unchanged
                     const int b = min(batch_of(n, i, kh), B - 1);
@@ -722,12 +847,12 @@ __device__ __forceinline__ void store_tile(const f32x16 (&tot)[NT], int r, int n
 #pragma unroll
                 for (int n = 0; n < NT; n++)
 #pragma unroll
-                    for (int i = 0; i < 16; i++) acc[n][i] += v[kk][n][i];
+                    for (int i = 0; i < NI; i++) acc[n][i] += v[kk][n][i];
     }
 #pragma unroll
     for (int n = 0; n < NT; n++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < NI; i++) {
             const int b = batch_of(n, i, kh);
             if (b < B) Y[(size_t)b * nrows + r] = acc[n][i];
         }
@@ -769,13 +894,10 @@ __host__ __device__ constexpr int max_chunks() {
     if (MASK & 32) c = c > FmtQ3K::kRowChunks ? c : FmtQ3K::kRowChunks;
     return c;
 }
-// LDS image: [x hi: BP x COLH][x lo: BP x COLH][32-column sums: BP x 16 halves][16-column sums: BP x 32 halves]
-// [(S, 1/s): BP][weight windows]
-template <int NT>
-__host__ __device__ constexpr int lds_w_offset() { return (2 * 32 * NT * COLH + 32 * NT * 16 + 32 * NT * 32) * 2 + 32 * NT * 8; }
-template <int NT, int MASK>
+// LDS: the x image (two of them for NT = 1), then the weight windows
+template <bool HL, int NT, int MASK>
 __host__ __device__ constexpr int lds_bytes() {
-    return (NT == 1 ? 2 : 1) * lds_w_offset<NT>() + kWaves * kRowsPerWave * max_chunks<MASK>() * 16 + kWinPad;
+    return (NT == 1 ? 2 : 1) * XImage<HL, NT>::kBytes + kWaves * kRowsPerWave * max_chunks<MASK>() * 16 + kWinPad;
 }
 
 // store_tile for a SwiGLU pair workgroup (B <= 32): split partials over virtual
@@ -783,20 +905,21 @@ __host__ __device__ constexpr int lds_bytes() {
 // the up waves pass their totals to the gate waves through LDS and those store
 // silu(gate) * up.  r is the lane's row within its matrix, lw its row within
 // the workgroup's 128.
-__device__ __forceinline__ void store_pair(const f32x16 (&tot)[1], int r, int lw, bool up, int nrows, int kh, int B,
+template <int NI>
+__device__ __forceinline__ void store_pair(const float (&tot)[1][NI], int r, int lw, bool up, int nrows, int kh, int B,
                                            float *__restrict__ out, float *part, int *counters, int tile, int split,
                                            int ksplit, uint8_t *lds) {
     const bool live = r < nrows;
     const int vr = r + (up ? nrows : 0);
-    float fin[16];
+    float fin[NI];
 #pragma unroll
-    for (int i = 0; i < 16; i++) fin[i] = tot[0][i];
+    for (int i = 0; i < NI; i++) fin[i] = tot[0][i];
     if (ksplit > 1) {
         const size_t plane = (size_t)B * 2 * nrows;
         if (live) {
             float *mine = part + split * plane;
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
+            for (int i = 0; i < NI; i++) {
                 const int b = batch_of(0, i, kh);
                 if (b < B) __hip_atomic_store(mine + (size_t)b * 2 * nrows + vr, tot[0][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -813,16 +936,16 @@ __device__ __forceinline__ void store_pair(const f32x16 (&tot)[1], int r, int lw
         __syncthreads();
         if (!s_last) return;  // uniform across the workgroup
         constexpr int KB = 4;
-        float acc[16];
+        float acc[NI];
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[i] = 0.f;
+        for (int i = 0; i < NI; i++) acc[i] = 0.f;
         const int rr = min(vr, 2 * nrows - 1);
         for (int k0 = 0; k0 < ksplit; k0 += KB) {
-            float v[KB][16];
+            float v[KB][NI];
 #pragma unroll
             for (int kk = 0; kk < KB; kk++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
+                for (int i = 0; i < NI; i++) {
                     const int b = min(batch_of(0, i, kh), B - 1);
                     v[kk][i] = __hip_atomic_load(part + min(k0 + kk, ksplit - 1) * plane + (size_t)b * 2 * nrows + rr,
                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -831,20 +954,20 @@ __device__ __forceinline__ void store_pair(const f32x16 (&tot)[1], int r, int lw
             for (int kk = 0; kk < KB; kk++)
                 if (k0 + kk < ksplit)
 #pragma unroll
-                    for (int i = 0; i < 16; i++) acc[i] += v[kk][i];
+                    for (int i = 0; i < NI; i++) acc[i] += v[kk][i];
         }
 #pragma unroll
-        for (int i = 0; i < 16; i++) fin[i] = acc[i];
+        for (int i = 0; i < NI; i++) fin[i] = acc[i];
     }
     float *xl = reinterpret_cast<float *>(lds);  // [128 rows][33]: the up totals
     __syncthreads();  // every wave is done with the x buffers
     if (up)
 #pragma unroll
-        for (int i = 0; i < 16; i++) xl[lw * 33 + batch_of(0, i, kh)] = fin[i];
+        for (int i = 0; i < NI; i++) xl[lw * 33 + batch_of(0, i, kh)] = fin[i];
     __syncthreads();
     if (!up && live)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < NI; i++) {
             const int b = batch_of(0, i, kh);
             if (b < B) out[(size_t)b * nrows + r] = silu_times(fin[i], xl[lw * 33 + b]);
         }
@@ -852,57 +975,53 @@ __device__ __forceinline__ void store_pair(const f32x16 (&tot)[1], int r, int lw
 
 // One workgroup's tile (32 rows per wave x all batch columns) over the K
 // range of its split, x converted into LDS super-block by super-block.
-template <class F, int NT, int PD, bool PAIR>  // NT = padded batch / 32, PD = weight prefetch depth (super-blocks)
+template <class F, bool HL, int NT, bool PAIR>  // NT: column groups of 32 (HL: one of 16)
 __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int split, const MfmaGroup &g, uint8_t *lds) {
-    constexpr int BP = 32 * NT;
-    constexpr int CPT = BP / 32;  // x columns converted per thread (16 lanes per column and super-block)
+    using I = XImage<HL, NT>;
+    constexpr int NI = kOut<HL>;
     constexpr int CH = F::kChunks;          // 16-byte chunks staged per row and super-block
     constexpr int CL = (kRowsPerWave * CH + 63) / 64;  // chunks per lane
-    _Float16 *sh_hi = reinterpret_cast<_Float16 *>(lds);
-    _Float16 *sh_lo = sh_hi + BP * COLH;
-    _Float16 *sh_xs = sh_lo + BP * COLH;
-    _Float16 *sh_x16 = sh_xs + BP * 16;
-    float2 *sh_S = reinterpret_cast<float2 *>(sh_x16 + BP * 32);  // (sum of x, 1 / column scale) per column
     const bool up_half = PAIR && (threadIdx.x >> 6) >= kWaves / 2;  // SwiGLU pairs: waves 4-7 take the up rows
-    const uint8_t *__restrict__ W = up_half ? g.w2 : P.w;
+    const uint8_t *W = up_half ? g.w2 : P.w;
     const float *__restrict__ X = P.x;
     const size_t pitch = P.pitch;
     const int nrows = P.rows, row0 = P.row0, B = g.B, cols = 256 * g.nsb;
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    const Ctx c{wave, lane & 31, lane >> 5, sh_hi, sh_lo, sh_xs, sh_x16, sh_S};
+    const int lane = threadIdx.x & 63, lr = lane & 31, kh = lane >> 5;
     const int rbase = PAIR ? tile * (kRowsPerWG / 2) + (wave & (kWaves / 2 - 1)) * kRowsPerWave
                            : tile * kRowsPerWG + wave * kRowsPerWave;
     const int sb0 = split * g.ksb, sb1 = min(g.nsb, sb0 + g.ksb);
-    auto row_off = [&](int rho) { return (size_t)(row0 + min(rbase + rho, nrows - 1)) * pitch; };
     // Weight staging: chunk j = lane + 64 k of the wave's 32 x CH chunk grid is
     // row j / CH, 16-byte piece j % CH of that row's aligned window.  Whole
     // aligned 16-byte lanes, consecutive within a row: few cache accesses per
     // load, instead of 8-byte gathers from 32 rows at 2-byte alignment.
-    size_t coff[CL];
+    const RowSpan rows{pitch, row0, rbase, nrows};
+    uint32_t coff[CL];
 #pragma unroll
     for (int k = 0; k < CL; k++) {
         const int j = min(lane + 64 * k, kRowsPerWave * CH - 1);
-        coff[k] = row_off(j / CH) + 16 * (j % CH);
+        coff[k] = rows.offset(j / CH) + 16 * (j % CH);
     }
-    const size_t myoff = row_off(c.lr);
+    const uint32_t myoff = rows.offset(lr);
+    W += rows.base();
     constexpr int RC = NT == 1 ? F::kRowChunks : CH;  // window row stride (chunks): padded for the realigned reads
-    uint8_t *wslot = lds + lds_w_offset<NT>() + wave * (kRowsPerWave * RC * 16);
+    uint8_t *wslot = lds + (NT == 1 ? 2 : 1) * I::kBytes + wave * (kRowsPerWave * RC * 16);
 
-    u32x4 ch_n[PD][CL];
-    float xv_n[CPT][16];  // the next super-block's raw x: column (threadIdx.x >> 4) + 32 i, values 16 q .. +16
+    u32x4 ch_n[CL];
+    float xv_n[NT][16];  // the next super-block's raw x: column (threadIdx.x >> 4) + 32 i, values 16 q .. +16
     const int xq = threadIdx.x & 15, xcol = threadIdx.x >> 4;
+    const bool stager = xcol < I::kCols;  // HL: half of the threads hold the 16 columns
     // (a macro rather than a lambda: the register arrays must stay in VGPRs)
-#define JH_LOAD_W(ST, SB)                                                                                  \
+#define JH_LOAD_W(SB)                                                                                      \
     do {                                                                                                   \
-        const size_t sbo = (size_t)(SB) * F::kBytes;                                                       \
+        const uint32_t sbo = (uint32_t)(SB) * F::kBytes;                                                       \
         _Pragma("unroll") for (int k = 0; k < CL; k++)                                                     \
-            ch_n[ST][k] = *reinterpret_cast<const u32x4 *>(W + ((coff[k] + sbo) & ~size_t(15)));           \
+            ch_n[k] = *reinterpret_cast<const u32x4 *>(W + ((coff[k] + sbo) & ~15u));               \
     } while (0)
 #define JH_LOAD_X(SB)                                                                                      \
     do {                                                                                                   \
-        _Pragma("unroll") for (int i = 0; i < CPT; i++) {                                                  \
+        _Pragma("unroll") for (int i = 0; i < NT; i++) {                                                   \
             const int b = xcol + 32 * i;                                                                   \
             const float4 *xp = reinterpret_cast<const float4 *>(X + (size_t)min(b, B - 1) * cols +        \
                                                                 (SB) * 256 + 16 * xq);                     \
@@ -912,182 +1031,113 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int sp
             }                                                                                              \
         }                                                                                                  \
     } while (0)
+#define JH_PARK()                                                                                          \
+    do {                                                                                                   \
+        _Pragma("unroll") for (int k = 0; k < CL; k++)                                                     \
+            if (lane + 64 * k < kRowsPerWave * CH)                                                         \
+                *reinterpret_cast<u32x4 *>(wslot + 16 * win_chunk<CH, RC>(lane + 64 * k)) = ch_n[k];       \
+    } while (0)
 
-    f32x16 tot[NT];
+    float tot[NT][NI];
 #pragma unroll
-    for (int n = 0; n < NT; n++) tot[n] = (f32x16){};
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int i = 0; i < NI; i++) tot[n][i] = 0.f;
 
-    auto fold = [&](const typename F::Regs &w, const Ctx &cx) {
-        if constexpr (F::kSums) {
-            F::template compute<NT>(w, cx, tot);
-        } else {
-            f32x16 part[NT];
-#pragma unroll
-            for (int n = 0; n < NT; n++) part[n] = (f32x16){};
-            F::template compute<NT>(w, cx, part);
-#pragma unroll
-            for (int n = 0; n < NT; n++) {
-                float S[16], cs[16];
-                col_terms<NT>(cx, n, S, cs);
-#pragma unroll
-                for (int i = 0; i < 16; i++) tot[n][i] = fmaf(cs[i], part[n][i], tot[n][i]);
-            }
-        }
-    };
-
-    if constexpr (NT == 1 && PD == 1) {
+    if constexpr (NT == 1) {
         // Two x buffers: super-block sb + 1's x is converted into the free
         // buffer while sb's MFMAs run, with one barrier per super-block.  The
         // buffer a step writes was last read by the previous step's MFMAs,
         // which every wave finished before this step's barrier.
-        constexpr int XS = lds_w_offset<1>();  // bytes of one x buffer
-        auto ctx_at = [&](int buf) {
-            _Float16 *hi = reinterpret_cast<_Float16 *>(lds + buf * XS);
-            _Float16 *lo = hi + BP * COLH, *xs = lo + BP * COLH, *x16 = xs + BP * 16;
-            return Ctx{wave, lane & 31, lane >> 5, hi, lo, xs, x16, reinterpret_cast<float2 *>(x16 + BP * 32)};
-        };
-        auto stage_into = [&](int buf) {
-            const Ctx cx = ctx_at(buf);
-            stage_x_column(xv_n[0], xq, const_cast<_Float16 *>(cx.sh_hi), const_cast<_Float16 *>(cx.sh_lo),
-                           const_cast<_Float16 *>(cx.sh_xs), const_cast<_Float16 *>(cx.sh_x16),
-                           const_cast<float2 *>(cx.sh_S), xcol, COLH);
-        };
-        uint8_t *wslot2 = lds + 2 * XS + wave * (kRowsPerWave * RC * 16);
         JH_MT(0);
+        if (HL && !stager) {  // the lo limbs' rows carry no sums
+            I::zero_sums(lds, xq, xcol);
+            I::zero_sums(lds + I::kBytes, xq, xcol);
+        }
         if (sb0 < sb1) {
-            JH_LOAD_X(sb0);
-            JH_LOAD_W(0, sb0);
-            stage_into(0);
-            if (sb0 + 1 < sb1) JH_LOAD_X(sb0 + 1);
+            if (stager) JH_LOAD_X(sb0);
+            JH_LOAD_W(sb0);
+            if (stager) I::template store<F::kSums>(lds, xv_n[0], xq, xcol);
+            if (stager && sb0 + 1 < sb1) JH_LOAD_X(sb0 + 1);
         }
         for (int sb = sb0; sb < sb1; sb++) {
             const int buf = (sb - sb0) & 1;
             __syncthreads();  // x of sb is staged; the other buffer is free
             JH_MT(1 + 4 * (sb - sb0));
-#pragma unroll
-            for (int k = 0; k < CL; k++)
-                if (lane + 64 * k < kRowsPerWave * CH) *reinterpret_cast<u32x4 *>(wslot2 + 16 * win_chunk<CH, RC>(lane + 64 * k)) = ch_n[0][k];
+            JH_PARK();
             JH_MT(2 + 4 * (sb - sb0));
             typename F::Regs w;
-            F::template load<true>(w, wslot2 + c.lr * RC * 16 + ((myoff + (size_t)sb * F::kBytes) & 15), c.kh);
+            F::load(w, wslot + lr * RC * 16 + ((myoff + (uint32_t)sb * F::kBytes) & 15), kh);
             if (sb + 1 < sb1) {
-                stage_into(buf ^ 1);
-                if (sb + 2 < sb1) JH_LOAD_X(sb + 2);
-                JH_LOAD_W(0, sb + 1);
+                if (stager) {
+                    I::template store<F::kSums>(lds + (buf ^ 1) * I::kBytes, xv_n[0], xq, xcol);
+                    if (sb + 2 < sb1) JH_LOAD_X(sb + 2);
+                }
+                JH_LOAD_W(sb + 1);
             }
             JH_MT(3 + 4 * (sb - sb0));
-            fold(w, ctx_at(buf));
+            F::template compute<HL, NT>(w, Ctx<HL, NT>{lr, kh, lds + buf * I::kBytes}, tot);
             JH_MT(4 + 4 * (sb - sb0));
         }
     } else {
-    if (sb0 < sb1) JH_LOAD_X(sb0);
+        if (sb0 < sb1) {
+            JH_LOAD_X(sb0);
+            JH_LOAD_W(sb0);
+        }
+        for (int sb = sb0; sb < sb1; sb++) {
+            __syncthreads();  // the previous super-block's LDS contents are consumed
 #pragma unroll
-    for (int st = 0; st < PD; st++)
-        if (sb0 + st < sb1) JH_LOAD_W(st, sb0 + st);
-    for (int sb = sb0; sb < sb1; sb++) {
-        __syncthreads();  // the previous super-block's LDS contents are consumed
-#pragma unroll
-        for (int i = 0; i < CPT; i++)
-            stage_x_column(xv_n[i], xq, sh_hi, sh_lo, sh_xs, sh_x16, sh_S, xcol + 32 * i, COLH);
-#pragma unroll
-        for (int k = 0; k < CL; k++)
-            if (lane + 64 * k < kRowsPerWave * CH) *reinterpret_cast<u32x4 *>(wslot + 16 * win_chunk<CH, RC>(lane + 64 * k)) = ch_n[0][k];
-        // this lane's row block inside its staged window (same wave: no barrier)
-        typename F::Regs w;
-        F::template load<NT == 1>(w, wslot + c.lr * RC * 16 + ((myoff + (size_t)sb * F::kBytes) & 15), c.kh);
-        // the loads below overlap this super-block's math
-        if (sb + 1 < sb1) JH_LOAD_X(sb + 1);
-#pragma unroll
-        for (int st = 0; st + 1 < PD; st++)
-#pragma unroll
-            for (int k = 0; k < CL; k++) ch_n[st][k] = ch_n[st + 1][k];
-        if (sb + PD < sb1) JH_LOAD_W(PD - 1, sb + PD);
-        __syncthreads();
-        fold(w, c);
-    }
+            for (int i = 0; i < NT; i++) I::template store<F::kSums>(lds, xv_n[i], xq, xcol + 32 * i);
+            JH_PARK();
+            // this lane's row block inside its staged window (same wave: no barrier)
+            typename F::Regs w;
+            F::load(w, wslot + lr * RC * 16 + ((myoff + (uint32_t)sb * F::kBytes) & 15), kh);
+            // The loads below overlap this super-block's math.  They are unconditional (after the last
+            // super-block, that one again): a load inside a branch is waited for at the branch's end
+            // (2 x 14336 x 4096 Q4_K, B = 64: 65 -> 59 us).
+            JH_LOAD_X(min(sb + 1, sb1 - 1));
+            JH_LOAD_W(min(sb + 1, sb1 - 1));
+            __syncthreads();
+            F::template compute<HL, NT>(w, Ctx<HL, NT>{lr, kh, lds}, tot);
+        }
     }
 #undef JH_LOAD_X
 #undef JH_LOAD_W
+#undef JH_PARK
 
     if constexpr (PAIR) {
-        store_pair(tot, rbase + c.lr, (wave & (kWaves / 2 - 1)) * kRowsPerWave + c.lr, up_half, nrows, c.kh, B,
+        store_pair(tot, rbase + lr, (wave & (kWaves / 2 - 1)) * kRowsPerWave + lr, up_half, nrows, kh, B,
                    g.swiglu, g.part, g.counters, tile, split, g.ksplit, lds);
         return;
     }
-    store_tile<NT>(tot, rbase + c.lr, nrows, c.kh, B, P.y, g.part + P.part0, g.counters + (size_t)P.cnt0 * kCounterStride, tile, split,
-                   g.ksplit);
+    store_tile(tot, rbase + lr, nrows, kh, B, P.y, g.part + P.part0, g.counters + (size_t)P.cnt0 * kCounterStride, tile, split,
+               g.ksplit);
 }
 
 // A group of matrices with the same K in one launch (1-D grid): each
 // workgroup finds its matrix and runs that matrix's format.
-template <int NT, int MASK, bool PAIR = false>
+template <bool HL, int NT, int MASK, bool PAIR = false>
 __global__ __launch_bounds__(kThreads) void mfma_group(MfmaGroup g) {
-    __shared__ __align__(16) uint8_t lds[lds_bytes<NT, MASK>()];
+    __shared__ __align__(16) uint8_t lds[lds_bytes<HL, NT, MASK>()];
     const int id = blockIdx.x;
     int m = 0;
     for (int i = 1; i < g.n; i++)
         if (id >= g.p[i].wg0) m = i;
     const MfmaProblem &P = g.p[m];
     const int local = id - P.wg0, tile = local / g.ksplit, split = local - tile * g.ksplit;
-    constexpr int PD = NT == 1 ? kPrefetch : 1;
     switch (P.type) {
-        case 12: if constexpr ((MASK & 1) != 0) gemm_body<FmtQ4K, NT, PD, PAIR>(P, tile, split, g, lds); break;
-        case 13: if constexpr ((MASK & 2) != 0) gemm_body<FmtQ5K, NT, PD, PAIR>(P, tile, split, g, lds); break;
-        case 14: if constexpr ((MASK & 4) != 0) gemm_body<FmtQ6K, NT, PD, PAIR>(P, tile, split, g, lds); break;
-        case 10: if constexpr ((MASK & 16) != 0) gemm_body<FmtQ2K, NT, PD, PAIR>(P, tile, split, g, lds); break;
-        case 11: if constexpr ((MASK & 32) != 0) gemm_body<FmtQ3K, NT, PD, PAIR>(P, tile, split, g, lds); break;
-        default: if constexpr ((MASK & 8) != 0) gemm_body<FmtQ8_0, NT, PD, PAIR>(P, tile, split, g, lds); break;
+        case 12: if constexpr ((MASK & 1) != 0) gemm_body<FmtQ4K, HL, NT, PAIR>(P, tile, split, g, lds); break;
+        case 13: if constexpr ((MASK & 2) != 0) gemm_body<FmtQ5K, HL, NT, PAIR>(P, tile, split, g, lds); break;
+        case 14: if constexpr ((MASK & 4) != 0) gemm_body<FmtQ6K, HL, NT, PAIR>(P, tile, split, g, lds); break;
+        case 10: if constexpr ((MASK & 16) != 0) gemm_body<FmtQ2K, HL, NT, PAIR>(P, tile, split, g, lds); break;
+        case 11: if constexpr ((MASK & 32) != 0) gemm_body<FmtQ3K, HL, NT, PAIR>(P, tile, split, g, lds); break;
+        default: if constexpr ((MASK & 8) != 0) gemm_body<FmtQ8_0, HL, NT, PAIR>(P, tile, split, g, lds); break;
     }
 }
 
-// x of one column and super-block into its prepared slab: 16 consecutive
-// lanes hold the column's 256 values, 16 each (xv).  The same arithmetic as
-// stage_x_column (scale, limbs, sums, butterflies), so both layouts carry
-// identical values.
-__device__ __forceinline__ void prep_x_column(const float (&xv)[16], int q, uint8_t *slab, int col) {
-    float m = 0.f;
-#pragma unroll
-    for (int j = 0; j < 16; j++) m = fmaxf(m, fabsf(xv[j]));
-    m = row16_max(m);
-    int e = 0;
-    if (m > 0.f) (void)frexpf(m, &e);
-    const float s = m > 0.f ? ldexpf(1.f, 13 - e) : 1.f;
-    half8 h[2], l[2];
-    float g[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        float sum = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float v = xv[4 * k + j] * s;
-            const _Float16 hh = (_Float16)v;
-            const _Float16 ll = (_Float16)(v - (float)hh);
-            h[k >> 1][4 * (k & 1) + j] = hh;
-            l[k >> 1][4 * (k & 1) + j] = ll;
-            sum += (float)hh + (float)ll;
-        }
-        g[k] = sum;
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int slot = CtxP::slot(col, 8 * (2 * q + i));
-        *reinterpret_cast<half8 *>(slab + kSlabHi + 16 * slot) = h[i];
-        *reinterpret_cast<half8 *>(slab + kSlabLo + 16 * slot) = l[i];
-    }
-    float sub = (g[0] + g[1]) + (g[2] + g[3]);
-    sub += dpp_f<0xB1>(sub);
-    if ((q & 1) == 0) {
-        _Float16 *xs = reinterpret_cast<_Float16 *>(slab + kSlabXs) + col * 16;
-        const _Float16 hs = (_Float16)sub;
-        xs[q >> 1] = hs;
-        xs[8 + (q >> 1)] = (_Float16)(sub - (float)hs);
-    }
-    const float tot = row16_sum((g[0] + g[2]) + (g[1] + g[3]));
-    if (q == 0) reinterpret_cast<float2 *>(slab + kSlabS)[col] = make_float2(tot, 1.f / s);
-}
-
-// one workgroup per super-block: 32 columns x 16 lanes (columns >= B are zero)
-__global__ __launch_bounds__(512) void x_prep(const float *__restrict__ X, int B, int cols, uint8_t *__restrict__ slabs) {
+// one workgroup per super-block: 32 (HL: 16) columns x 16 lanes (columns >= B are zero)
+template <bool HL>
+__global__ __launch_bounds__(HL ? 256 : 512) void x_prep(const float *__restrict__ X, int B, int cols, uint8_t *__restrict__ slabs) {
     const int sb = blockIdx.x, q = threadIdx.x & 15, col = threadIdx.x >> 4;
     float xv[16];
     const float4 *xp = reinterpret_cast<const float4 *>(X + (size_t)min(col, B - 1) * cols + sb * 256 + 16 * q);
@@ -1099,7 +1149,7 @@ __global__ __launch_bounds__(512) void x_prep(const float *__restrict__ X, int B
         xv[4 * k + 2] = v.z;
         xv[4 * k + 3] = v.w;
     }
-    prep_x_column(xv, q, slabs + (size_t)sb * kSlabBytes, col);
+    Slab<HL>::store(slabs + (size_t)sb * Slab<HL>::kBytes, xv, q, col);
 }
 
 // The B <= 32 kernel on prepared x, for matrices with enough row tiles to
@@ -1118,14 +1168,15 @@ __global__ __launch_bounds__(512) void x_prep(const float *__restrict__ X, int B
 // Loads are issued unconditionally (addresses clamped to the last super-block
 // of the range) so that every wave's count of memory operations in flight is
 // the same static number at each wait.
-template <class F>
-__global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *__restrict__ W, size_t pitch, int row0, int nrows,
+template <class F, bool HL>
+__global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pitch, int row0, int nrows,
                                                     int nsb, const uint8_t *__restrict__ slabs,
                                                     float *__restrict__ Y, int B) {
     constexpr int CH = F::kChunks;
     constexpr int CL = (kRowsPerWave * CH + 63) / 64;
-    constexpr int XI = (kSlabRows + kWaves - 1) / kWaves;  // slab rows per wave
-    __shared__ __align__(16) uint8_t sh_x[2][kSlabBytes];
+    using I = Slab<HL>;
+    constexpr int XI = (I::kRows + kWaves - 1) / kWaves;  // slab rows per wave
+    __shared__ __align__(16) uint8_t sh_x[2][I::kBytes];
     constexpr int RC = F::kRowChunks;  // window row stride (chunks)
     __shared__ __align__(16) uint8_t sh_w[kWaves * kRowsPerWave * RC * 16 + kWinPad];
 
@@ -1133,14 +1184,15 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *__restrict__ 
     const int lane = threadIdx.x & 63, lr = lane & 31, kh = lane >> 5;
     const int rbase = blockIdx.x * kRowsPerWG + wave * kRowsPerWave;
     const int sb0 = 0, last = nsb - 1;
-    auto row_off = [&](int rho) { return (size_t)(row0 + min(rbase + rho, nrows - 1)) * pitch; };
-    size_t coff[CL];
+    const RowSpan rows{pitch, row0, rbase, nrows};
+    uint32_t coff[CL];
 #pragma unroll
     for (int k = 0; k < CL; k++) {
         const int j = min(lane + 64 * k, kRowsPerWave * CH - 1);
-        coff[k] = row_off(j / CH) + 16 * (j % CH);
+        coff[k] = rows.offset(j / CH) + 16 * (j % CH);
     }
-    const size_t myoff = row_off(lr);
+    const uint32_t myoff = rows.offset(lr);
+    W += rows.base();
     uint8_t *wslot = sh_w + wave * (kRowsPerWave * RC * 16);
 
     // The slab DMA is issued from inline asm, outside the compiler's
@@ -1150,11 +1202,11 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *__restrict__ 
     // keeps them exact (each step's weight chunks are waited for before the
     // step issues its DMA).
     auto dma_x = [&](int sb, int buf) {
-        const uint8_t *src = slabs + (size_t)min(sb, last) * kSlabBytes + 16 * lane;
+        const uint8_t *src = slabs + (size_t)min(sb, last) * I::kBytes + 16 * lane;
         const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)sh_x[buf];
 #pragma unroll
         for (int k = 0; k < XI; k++) {
-            const int r = min(wave + kWaves * k, kSlabRows - 1);  // surplus waves repeat the last row (same bytes)
+            const int r = min(wave + kWaves * k, I::kRows - 1);  // surplus waves repeat the last row (same bytes)
             asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src + 1024 * r),
                          "s"(dst + 1024 * r)
                          : "memory", "m0");
@@ -1163,12 +1215,12 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *__restrict__ 
     u32x4 wa[CL], wb[CL];
 #define JH_LOAD_W(SET, SB)                                                                                 \
     do {                                                                                                   \
-        const size_t sbo = (size_t)min((SB), last) * F::kBytes;                                            \
+        const uint32_t sbo = (uint32_t)min((SB), last) * F::kBytes;                                        \
         _Pragma("unroll") for (int k = 0; k < CL; k++)                                                     \
-            SET[k] = *reinterpret_cast<const u32x4 *>(W + ((coff[k] + sbo) & ~size_t(15)));                \
+            SET[k] = *reinterpret_cast<const u32x4 *>(W + ((coff[k] + sbo) & ~15u));                \
     } while (0)
 
-    f32x16 tot[1] = {(f32x16){}};
+    float tot[1][kOut<HL>] = {};
 #define JH_STEP(SET, SB, BUF)                                                                              \
     do {                                                                                                   \
         /* this wave's part of slab SB and its chunks of SB have landed (only SB + 1's are in flight) */   \
@@ -1179,18 +1231,9 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *__restrict__ 
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");                                   \
         dma_x((SB) + 1, (BUF) ^ 1);                                                                        \
         typename F::Regs w;                                                                                \
-        F::template load<true>(w, wslot + lr * RC * 16 + ((myoff + (size_t)(SB) * F::kBytes) & 15), kh);  \
+        F::load(w, wslot + lr * RC * 16 + ((myoff + (uint32_t)(SB) * F::kBytes) & 15), kh);  \
         JH_LOAD_W(SET, (SB) + 2);                                                                          \
-        const CtxP c{lr, kh, sh_x[BUF]};                                                                   \
-        if constexpr (F::kSums) {                                                                          \
-            F::template compute<1>(w, c, tot);                                                             \
-        } else {                                                                                           \
-            f32x16 pt[1] = {(f32x16){}};                                                                   \
-            F::template compute<1>(w, c, pt);                                                              \
-            float S[16], cs[16];                                                                           \
-            col_terms<1>(c, 0, S, cs);                                                                     \
-            _Pragma("unroll") for (int i = 0; i < 16; i++) tot[0][i] = fmaf(cs[i], pt[0][i], tot[0][i]);   \
-        }                                                                                                  \
+        F::template compute<HL, 1>(w, CtxP<HL>{lr, kh, sh_x[BUF]}, tot);                                   \
     } while (0)
 
     dma_x(sb0, 0);
@@ -1206,17 +1249,21 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *__restrict__ 
 #undef JH_STEP
 #undef JH_LOAD_W
 
-    store_tile<1>(tot, rbase + lr, nrows, kh, B, Y, nullptr, nullptr, blockIdx.x, 0, 1);
+    store_tile(tot, rbase + lr, nrows, kh, B, Y, nullptr, nullptr, blockIdx.x, 0, 1);
 }
 
 }  // namespace
 
 // ------------------------------------------------------------------ host side
+// Up to 16 batch columns take the kernels whose MFMAs hold both limbs (HL).
+constexpr int kHlMaxBatch = 16;
+
 static bool mfma_applies(const MfmaDesc &d, int B) {
     if ((d.type != 12 && d.type != 13 && d.type != 14 && d.type != 8 && d.type != 10 && d.type != 11) ||
         B < kMfmaMinBatch || B > 64 || d.cols % 256 ||
         d.cols <= 0 || d.row_end <= d.row_start)
         return false;
+    if (d.pitch > (size_t(1) << 26)) return false;  // 32 rows' offsets in 32 bits
     if ((d.type == 12 || d.type == 13) && ((reinterpret_cast<uintptr_t>(d.w) | d.pitch) & 15))
         return false;  // K-quant rows are staged as whole aligned 16-byte chunks
     return (reinterpret_cast<uintptr_t>(d.x) & 15) == 0;  // x is read as float4
@@ -1271,7 +1318,7 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p) {
     }
     p.grid = tiles * p.ksplit;
     p.prepared = n == 1 && p.ksplit == 1 && B <= 32 && d[0].type != 10 && d[0].type != 11;  // slabs carry no 16-column sums
-    p.slab_bytes = p.prepared ? (size_t)p.nsb * kSlabBytes : 0;
+    p.slab_bytes = p.prepared ? (size_t)p.nsb * (B <= kHlMaxBatch ? Slab<true>::kBytes : Slab<false>::kBytes) : 0;
     p.part_floats = p.ksplit > 1 ? (size_t)p.ksplit * B * rows : 0;
     return true;
 }
@@ -1290,16 +1337,16 @@ int mfma_group_plan(int n, const MfmaDesc *d, int B, int *ksplit) {
     return p.prepared ? 2 : 1;
 }
 
-template <int NT>
+template <bool HL, int NT>
 static void launch_group_nt(const MfmaGroup &g, int mask, int grid, hipStream_t s) {
     switch (mask) {
-        case 1: mfma_group<NT, 1><<<grid, kThreads, 0, s>>>(g); break;
-        case 2: mfma_group<NT, 2><<<grid, kThreads, 0, s>>>(g); break;
-        case 4: mfma_group<NT, 4><<<grid, kThreads, 0, s>>>(g); break;
-        case 8: mfma_group<NT, 8><<<grid, kThreads, 0, s>>>(g); break;
-        case 16: mfma_group<NT, 16><<<grid, kThreads, 0, s>>>(g); break;
-        case 32: mfma_group<NT, 32><<<grid, kThreads, 0, s>>>(g); break;
-        default: mfma_group<NT, 63><<<grid, kThreads, 0, s>>>(g); break;
+        case 1: mfma_group<HL, NT, 1><<<grid, kThreads, 0, s>>>(g); break;
+        case 2: mfma_group<HL, NT, 2><<<grid, kThreads, 0, s>>>(g); break;
+        case 4: mfma_group<HL, NT, 4><<<grid, kThreads, 0, s>>>(g); break;
+        case 8: mfma_group<HL, NT, 8><<<grid, kThreads, 0, s>>>(g); break;
+        case 16: mfma_group<HL, NT, 16><<<grid, kThreads, 0, s>>>(g); break;
+        case 32: mfma_group<HL, NT, 32><<<grid, kThreads, 0, s>>>(g); break;
+        default: mfma_group<HL, NT, 63><<<grid, kThreads, 0, s>>>(g); break;
     }
 }
 
@@ -1363,12 +1410,16 @@ hipError_t launch_mfma_swiglu(const MfmaDesc &gate, const MfmaDesc &up, int B, f
     q.wg0 = q.cnt0 = 0;
     q.part0 = 0;
     const int grid = q.tiles * p.ksplit;
+    const bool hl = B <= kHlMaxBatch;
+#define JH_PAIR(M) \
+    (hl ? mfma_group<true, 1, M, true><<<grid, kThreads, 0, s>>>(g) : mfma_group<false, 1, M, true><<<grid, kThreads, 0, s>>>(g))
     switch (gate.type) {
-        case 12: mfma_group<1, 1, true><<<grid, kThreads, 0, s>>>(g); break;
-        case 13: mfma_group<1, 2, true><<<grid, kThreads, 0, s>>>(g); break;
-        case 14: mfma_group<1, 4, true><<<grid, kThreads, 0, s>>>(g); break;
-        default: mfma_group<1, 8, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 12: JH_PAIR(1); break;
+        case 13: JH_PAIR(2); break;
+        case 14: JH_PAIR(4); break;
+        default: JH_PAIR(8); break;
     }
+#undef JH_PAIR
     return hipGetLastError();
 }
 
@@ -1421,8 +1472,12 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
     if (p.prepared) {
         const MfmaDesc &m = d[0];
         const int nrows = m.row_end - m.row_start;
-        x_prep<<<p.nsb, 512, 0, s>>>(m.x, B, m.cols, ws);
-#define JH_PX(F) mfma_px<F><<<p.grid, kThreads, 0, s>>>(m.w, m.pitch, m.row_start, nrows, p.nsb, ws, m.y, B)
+        const bool hl = B <= kHlMaxBatch;
+        if (hl) x_prep<true><<<p.nsb, 256, 0, s>>>(m.x, B, m.cols, ws);
+        else x_prep<false><<<p.nsb, 512, 0, s>>>(m.x, B, m.cols, ws);
+#define JH_PX(F)                                                                                                          \
+    (hl ? mfma_px<F, true><<<p.grid, kThreads, 0, s>>>(m.w, m.pitch, m.row_start, nrows, p.nsb, ws, m.y, B)              \
+        : mfma_px<F, false><<<p.grid, kThreads, 0, s>>>(m.w, m.pitch, m.row_start, nrows, p.nsb, ws, m.y, B))
         if (m.type == 12) JH_PX(FmtQ4K);
         else if (m.type == 13) JH_PX(FmtQ5K);
         else if (m.type == 14) JH_PX(FmtQ6K);
@@ -1458,8 +1513,9 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
         part += p.ksplit > 1 ? (size_t)p.ksplit * B * q.rows : 0;
         mask |= q.type == 12 ? 1 : q.type == 13 ? 2 : q.type == 14 ? 4 : q.type == 10 ? 16 : q.type == 11 ? 32 : 8;
     }
-    if (B <= 32) launch_group_nt<1>(g, mask, p.grid, s);
-    else launch_group_nt<2>(g, mask, p.grid, s);
+    if (B <= kHlMaxBatch) launch_group_nt<true, 1>(g, mask, p.grid, s);
+    else if (B <= 32) launch_group_nt<false, 1>(g, mask, p.grid, s);
+    else launch_group_nt<false, 2>(g, mask, p.grid, s);
     return hipGetLastError();
 }
 
