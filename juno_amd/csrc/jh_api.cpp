@@ -252,13 +252,17 @@ int stream_workspace(int device, hipStream_t s, size_t bytes, void **out, int **
 // can take the per-matrix kernels.
 constexpr int kMfmaNotApplicable = -1;
 
+// More than 64 columns use the workspace only to split K, and where the stream has
+// none to give (a graph capture before any eager call, no memory left) they take
+// the per-matrix kernels, which need none.
 int enqueue_mfma_group(int device, int n, const jh::MfmaDesc *d, int B, hipStream_t s) {
     const size_t wsb = jh::mfma_group_workspace_bytes(n, d, B);
     if (!wsb) return kMfmaNotApplicable;
     void *ws = nullptr;
     int *counters = nullptr;
-    int rc = stream_workspace(device, s, wsb, &ws, &counters);
-    if (rc) return rc;
+    int rc = 0, ksplit = 1;
+    if (B <= 64 || (jh::mfma_group_plan(n, d, B, &ksplit) && ksplit > 1)) rc = stream_workspace(device, s, wsb, &ws, &counters);
+    if (rc) return B <= 64 ? rc : kMfmaNotApplicable;
     hipError_t e = jh::launch_mfma_group(n, d, B, ws, counters, s);
     if (e == hipSuccess) return JH_OK;
     if (e == hipErrorNotSupported) return kMfmaNotApplicable;

@@ -94,8 +94,7 @@ struct CombineSpec {
 // check_only: hipSuccess when it applies, nothing launched
 hipError_t launch_gemv_staged_combine(const GemvArgs &a, const CombineSpec &c, hipStream_t s, bool check_only = false);
 
-// Batched decode through the LDS-staged, fp16-MFMA path (kMfmaMinBatch <= B <= 64).
-// Batched GEMVs (kMfmaMinBatch <= B <= 64) on fp16 MFMA: up to kMaxMfmaGroup matrices
+// Batched GEMVs (B >= kMfmaMinBatch) on fp16 MFMA, staged through LDS: up to kMaxMfmaGroup matrices
 // with the same cols, each with its own x [B][cols] and y [B][row_end -
 // row_start], in one launch.  mfma_group_workspace_bytes returns 0 when the
 // path does not apply (types, shapes, alignment); otherwise launch_mfma_group

@@ -1,4 +1,4 @@
-// jh_mfma.hip -- batched decode (3 <= B <= 64) on Q4_K / Q5_K / Q6_K / Q8_0 through
+// jh_mfma.hip -- batched GEMVs (B >= 3) on Q4_K / Q5_K / Q6_K / Q8_0 through
 // LDS + fp16 MFMA.
 //
 // Y[b][r] = sum_c deq(W[r][c]) * X[b][c] is a dense contraction once B >= 16:
@@ -39,6 +39,7 @@
 #include "jh_device.hpp"
 #include "jh_kernels.hpp"
 
+#include <limits.h>
 #include <mutex>
 #include <stdlib.h>
 #include <utility>
@@ -389,6 +390,24 @@ __device__ __forceinline__ void step_fence(f32x16 (&part)[NT]) {
     for (int n = 0; n < NT; n++) asm volatile("" : "+v"(part[n]));
     __builtin_amdgcn_sched_barrier(0);
 }
+// TWO (see kTwo): the folds of a super-block's quarters are summed apart, then in pairs
+template <int NT>
+__device__ __forceinline__ void next_quarter(int t, f32x16 (&part)[NT], f32x16 (&quarter)[NT], f32x16 (&half)[NT]) {
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        if (t == 3 || t == 11) {
+            quarter[n] = part[n];
+            part[n] = (f32x16){};
+        } else if (t == 7) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) half[n][i] = quarter[n][i] + part[n][i];
+            part[n] = (f32x16){};
+        } else if (t == 15) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) part[n][i] = half[n][i] + (quarter[n][i] + part[n][i]);
+        }
+    }
+}
 // tot += cs * (the super-block's folded sums)
 template <bool HL, int NT, class C>
 __device__ __forceinline__ void fold_columns(const C &c, const f32x16 (&part)[NT], float (&tot)[NT][kOut<HL>]) {
@@ -443,7 +462,7 @@ struct FmtKQ {
         const uint32_t v = sh > 0 ? w >> (sh > 0 ? sh : 0) : w << (sh < 0 ? -sh : 0);
         return __builtin_elementwise_fma(as_h2((v & 0x00F000F0u) | top), ls, off);
     }
-    template <bool HL, int NT, class C>
+    template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         // 6-bit scales and mins of the 8 sub-blocks, one per byte (q4kScaleRaw / q4kMinRaw, :1471-1482),
         // and their centres: 8 (Q5_K 16) where the min is not zero
@@ -528,11 +547,11 @@ struct FmtQ6K {
         lds_read_u<1>(p + 206, dw);
         r.dw = dw[0];
     }
-    template <bool HL, int NT, class C>
+    template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1056.f);  // 1024 + 32
         const float d = half_bits_to_float(r.dw >> 16);
-        f32x16 part[NT];
+        f32x16 part[NT], quarter[NT], half[NT];
 #pragma unroll
         for (int n = 0; n < NT; n++) part[n] = (f32x16){};
 #pragma unroll
@@ -547,6 +566,7 @@ struct FmtQ6K {
             mfma_xw<HL, NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
             fold<NT>(part, d * (float)(int8_t)byte_of(t < 4 ? r.sc.x : t < 8 ? r.sc.y : t < 12 ? r.sc.z : r.sc.w, t & 3), acc);
             if (t % (NT > 1 ? 2 : 4) == (NT > 1 ? 1 : 3)) step_fence(part);
+            if (TWO) next_quarter<NT>(t, part, quarter, half);
         }
         fold_columns<HL, NT>(c, part, tot);
     }
@@ -564,7 +584,7 @@ struct FmtQ8_0 {
         const uint8_t *p;  // 40 registers of quants and scales would spill: each block is read ahead of its MFMAs
     };
     static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int) { r.p = p; }
-    template <bool HL, int NT, class C>
+    template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1152.f);  // 1024 + 128
         f32x16 part[NT];
@@ -588,7 +608,7 @@ struct FmtQ8_0 {
                 mfma_xw<HL, NT>(c, bytes_to_h8((j ? qb.z : qb.x) ^ 0x80808080u, (j ? qb.w : qb.y) ^ 0x80808080u, off),
                                 32 * b + 16 * c.kh + 8 * j, acc);
             fold<NT>(part, half_bits_to_float(db), acc);
-            if (HL || NT > 1) step_fence(part);
+            if (HL || NT > 1 || TWO) step_fence(part);
         }
         fold_columns<HL, NT>(c, part, tot);
     }
@@ -633,7 +653,7 @@ struct FmtQ2K {
         const uint32_t v = sh > 0 ? w >> (sh > 0 ? sh : 0) : w << (sh < 0 ? -sh : 0);
         return __builtin_elementwise_fma(as_h2((v & 0x00300030u) | top), sc, off);
     }
-    template <bool HL, int NT, class C>
+    template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const float d = half_bits_to_float(r.dm), dmin = half_bits_to_float(r.dm >> 16);
         const uint32_t top = in_vgpr(0x54005400u);
@@ -708,10 +728,10 @@ struct FmtQ3K {
         for (int o = 0; o < 2; o++) r.hm[o] = lds_u32x2(p + 16 * o + 8 * kh);
         r.sd = lds_u32x4(p + 96);
     }
-    template <bool HL, int NT, class C>
+    template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1028.f);  // 1024 + 4
-        f32x16 part[NT];
+        f32x16 part[NT], quarter[NT], half[NT];
 #pragma unroll
         for (int n = 0; n < NT; n++) part[n] = (f32x16){};
         const float d = half_bits_to_float(r.sd.w);
@@ -736,6 +756,8 @@ struct FmtQ3K {
                     mfma_xw<HL, NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
                     const int s6 = (int)byte_of(j < 2 ? ua : ub, 2 * (j & 1) + rr) - 32;
                     fold<NT>(part, d * (float)s6, acc);
+                    if (TWO && t % 4 == 3) step_fence(part);
+                    if (TWO) next_quarter<NT>(t, part, quarter, half);
                 }
         }
         fold_columns<HL, NT>(c, part, tot);
@@ -770,7 +792,7 @@ constexpr int kMaxTileCounters = kCounterSlots;
 
 template <int NT, int NI>
 __device__ __forceinline__ void store_tile(const float (&tot)[NT][NI], int r, int nrows, int kh, int B, float *__restrict__ Y,
-                                           float *part, int *counters, int tile, int split, int ksplit) {
+                                           float *part, size_t plane, int *counters, int tile, int split, int ksplit) {
     const bool live = r < nrows;
     if (ksplit == 1) {
         if (!live) return;
@@ -783,7 +805,6 @@ __device__ __forceinline__ void store_tile(const float (&tot)[NT][NI], int r, in
             }
         return;
     }
-    const size_t plane = (size_t)B * nrows;
     if (live) {
         float *mine = part + split * plane;
 #pragma unroll
@@ -861,7 +882,7 @@ __device__ __forceinline__ void store_tile(const float (&tot)[NT][NI], int r, in
 
 // ------------------------------------------------------------------ batched kernel
 // One matrix of a grouped launch: the workgroups [wg0, wg0 + tiles * ksplit)
-// are its row tiles x K splits (split fastest); its partial planes start at
+// are its row tiles x column chunks (more than 64 columns) x K splits (split fastest); its partial planes start at
 // part0 floats into the group's partial buffer and its tile counters at cnt0.
 struct MfmaProblem {
     const uint8_t *w;
@@ -874,13 +895,24 @@ struct MfmaGroup {
     MfmaProblem p[kMaxMfmaGroup];
     float *part;
     int *counters;
-    int n, nsb, ksb, ksplit, B;
+    int n, nsb, ksb, ksplit, B, chunks;
     // SwiGLU pairs (mfma_group<.., true>): p[0] is gate, w2 the up matrix of the
     // same shape; a workgroup's waves 0-3 take 128 gate rows and waves 4-7 the
     // same up rows, and swiglu[b][r] = silu(gate) * up replaces both outputs
     const uint8_t *w2;
     float *swiglu;
 };
+
+// More than 64 columns (WIDE): chunks of 64 columns in one launch, in the kernel of
+// 33..64 columns: before, the VALU kernels read the weights again for every 8
+// columns (2 x 14336 x 4096 Q4_K and 4096 x 14336 Q6_K at B = 128: 5460 -> 181 us).
+// Groups with Q6_K or Q3_K take chunks of 32 and sum in more fp32 chains (the
+// quarters of a super-block's 16 folds, and even and odd super-blocks): the folds'
+// roundings are most of their error, and in one chain of each it would be larger
+// than that of the VALU kernels' many lanes (K = 4096: Q6_K 1.15e-7 against 1.02e-7
+// of the norm, Q3_K 1.13e-7 against 1.00e-7).
+template <bool WIDE, int NT>
+constexpr bool kTwo = WIDE && NT == 1;
 
 // format mask bits: Q4_K, Q5_K, Q6_K, Q8_0, Q2_K, Q3_K
 template <int MASK>
@@ -975,17 +1007,20 @@ __device__ __forceinline__ void store_pair(const float (&tot)[1][NI], int r, int
 
 // One workgroup's tile (32 rows per wave x all batch columns) over the K
 // range of its split, x converted into LDS super-block by super-block.
-template <class F, bool HL, int NT, bool PAIR>  // NT: column groups of 32 (HL: one of 16)
-__device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int split, const MfmaGroup &g, uint8_t *lds) {
+// WIDE: column chunk `chunk` of g.chunks (32 NT columns each); TWO: see kTwo.
+template <class F, bool HL, int NT, bool PAIR, bool WIDE>  // NT: column groups of 32 (HL: one of 16)
+__device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int chunk, int split, const MfmaGroup &g, uint8_t *lds) {
+    constexpr bool TWO = kTwo<WIDE, NT>;
+    const int chunks = WIDE ? g.chunks : 1, col0 = WIDE ? chunk * 32 * NT : 0;
     using I = XImage<HL, NT>;
     constexpr int NI = kOut<HL>;
     constexpr int CH = F::kChunks;          // 16-byte chunks staged per row and super-block
     constexpr int CL = (kRowsPerWave * CH + 63) / 64;  // chunks per lane
     const bool up_half = PAIR && (threadIdx.x >> 6) >= kWaves / 2;  // SwiGLU pairs: waves 4-7 take the up rows
     const uint8_t *W = up_half ? g.w2 : P.w;
-    const float *__restrict__ X = P.x;
+    const float *__restrict__ X = P.x + (size_t)col0 * (256 * g.nsb);
     const size_t pitch = P.pitch;
-    const int nrows = P.rows, row0 = P.row0, B = g.B, cols = 256 * g.nsb;
+    const int nrows = P.rows, row0 = P.row0, B = WIDE ? min(32 * NT, g.B - col0) : g.B, cols = 256 * g.nsb;
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, lr = lane & 31, kh = lane >> 5;
@@ -1038,7 +1073,11 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int sp
                 *reinterpret_cast<u32x4 *>(wslot + 16 * win_chunk<CH, RC>(lane + 64 * k)) = ch_n[k];       \
     } while (0)
 
-    float tot[NT][NI];
+    float tot[NT][NI], tot2[NI];
+    if constexpr (TWO) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) tot2[i] = 0.f;
+    }
 #pragma unroll
     for (int n = 0; n < NT; n++)
 #pragma unroll
@@ -1076,7 +1115,15 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int sp
                 JH_LOAD_W(sb + 1);
             }
             JH_MT(3 + 4 * (sb - sb0));
-            F::template compute<HL, NT>(w, Ctx<HL, NT>{lr, kh, lds + buf * I::kBytes}, tot);
+            F::template compute<HL, NT, TWO>(w, Ctx<HL, NT>{lr, kh, lds + buf * I::kBytes}, tot);
+            if constexpr (TWO) {
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    const float v = tot[0][i];
+                    tot[0][i] = tot2[i];
+                    tot2[i] = v;
+                }
+            }
             JH_MT(4 + 4 * (sb - sb0));
         }
     } else {
@@ -1098,7 +1145,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int sp
             JH_LOAD_X(min(sb + 1, sb1 - 1));
             JH_LOAD_W(min(sb + 1, sb1 - 1));
             __syncthreads();
-            F::template compute<HL, NT>(w, Ctx<HL, NT>{lr, kh, lds}, tot);
+            F::template compute<HL, NT, TWO>(w, Ctx<HL, NT>{lr, kh, lds}, tot);
         }
     }
 #undef JH_LOAD_X
@@ -1110,13 +1157,17 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int sp
                    g.swiglu, g.part, g.counters, tile, split, g.ksplit, lds);
         return;
     }
-    store_tile(tot, rbase + lr, nrows, kh, B, P.y, g.part + P.part0, g.counters + (size_t)P.cnt0 * kCounterStride, tile, split,
-               g.ksplit);
+    if constexpr (TWO) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) tot[0][i] += tot2[i];
+    }
+    store_tile(tot, rbase + lr, nrows, kh, B, P.y + (size_t)col0 * nrows, g.part + P.part0 + (size_t)col0 * nrows,
+               (size_t)g.B * nrows, g.counters + (size_t)P.cnt0 * kCounterStride, tile * chunks + chunk, split, g.ksplit);
 }
 
 // A group of matrices with the same K in one launch (1-D grid): each
 // workgroup finds its matrix and runs that matrix's format.
-template <bool HL, int NT, int MASK, bool PAIR = false>
+template <bool HL, int NT, int MASK, bool PAIR = false, bool WIDE = false>
 __global__ __launch_bounds__(kThreads) void mfma_group(MfmaGroup g) {
     __shared__ __align__(16) uint8_t lds[lds_bytes<HL, NT, MASK>()];
     const int id = blockIdx.x;
@@ -1124,14 +1175,15 @@ __global__ __launch_bounds__(kThreads) void mfma_group(MfmaGroup g) {
     for (int i = 1; i < g.n; i++)
         if (id >= g.p[i].wg0) m = i;
     const MfmaProblem &P = g.p[m];
-    const int local = id - P.wg0, tile = local / g.ksplit, split = local - tile * g.ksplit;
+    const int local = id - P.wg0, at = local / g.ksplit, split = local - at * g.ksplit;
+    const int tile = WIDE ? at / g.chunks : at, chunk = WIDE ? at - tile * g.chunks : 0;
     switch (P.type) {
-        case 12: if constexpr ((MASK & 1) != 0) gemm_body<FmtQ4K, HL, NT, PAIR>(P, tile, split, g, lds); break;
-        case 13: if constexpr ((MASK & 2) != 0) gemm_body<FmtQ5K, HL, NT, PAIR>(P, tile, split, g, lds); break;
-        case 14: if constexpr ((MASK & 4) != 0) gemm_body<FmtQ6K, HL, NT, PAIR>(P, tile, split, g, lds); break;
-        case 10: if constexpr ((MASK & 16) != 0) gemm_body<FmtQ2K, HL, NT, PAIR>(P, tile, split, g, lds); break;
-        case 11: if constexpr ((MASK & 32) != 0) gemm_body<FmtQ3K, HL, NT, PAIR>(P, tile, split, g, lds); break;
-        default: if constexpr ((MASK & 8) != 0) gemm_body<FmtQ8_0, HL, NT, PAIR>(P, tile, split, g, lds); break;
+        case 12: if constexpr ((MASK & 1) != 0) gemm_body<FmtQ4K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
+        case 13: if constexpr ((MASK & 2) != 0) gemm_body<FmtQ5K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
+        case 14: if constexpr ((MASK & 4) != 0) gemm_body<FmtQ6K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
+        case 10: if constexpr ((MASK & 16) != 0) gemm_body<FmtQ2K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
+        case 11: if constexpr ((MASK & 32) != 0) gemm_body<FmtQ3K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
+        default: if constexpr ((MASK & 8) != 0) gemm_body<FmtQ8_0, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
     }
 }
 
@@ -1233,7 +1285,7 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
         typename F::Regs w;                                                                                \
         F::load(w, wslot + lr * RC * 16 + ((myoff + (uint32_t)(SB) * F::kBytes) & 15), kh);  \
         JH_LOAD_W(SET, (SB) + 2);                                                                          \
-        F::template compute<HL, 1>(w, CtxP<HL>{lr, kh, sh_x[BUF]}, tot);                                   \
+        F::template compute<HL, 1, false>(w, CtxP<HL>{lr, kh, sh_x[BUF]}, tot);                            \
     } while (0)
 
     dma_x(sb0, 0);
@@ -1249,7 +1301,7 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
 #undef JH_STEP
 #undef JH_LOAD_W
 
-    store_tile(tot, rbase + lr, nrows, kh, B, Y, nullptr, nullptr, blockIdx.x, 0, 1);
+    store_tile(tot, rbase + lr, nrows, kh, B, Y, nullptr, 0, nullptr, blockIdx.x, 0, 1);
 }
 
 }  // namespace
@@ -1260,7 +1312,7 @@ constexpr int kHlMaxBatch = 16;
 
 static bool mfma_applies(const MfmaDesc &d, int B) {
     if ((d.type != 12 && d.type != 13 && d.type != 14 && d.type != 8 && d.type != 10 && d.type != 11) ||
-        B < kMfmaMinBatch || B > 64 || d.cols % 256 ||
+        B < kMfmaMinBatch || d.cols % 256 ||
         d.cols <= 0 || d.row_end <= d.row_start)
         return false;
     if (d.pitch > (size_t(1) << 26)) return false;  // 32 rows' offsets in 32 bits
@@ -1272,6 +1324,7 @@ static bool mfma_applies(const MfmaDesc &d, int B) {
 namespace {
 struct Plan {
     int nsb, ksb, ksplit, grid;
+    int chunks, chunk;  // B > 64: column chunks and their width, 64 or 32 columns
     bool prepared;  // one unsplit matrix, B <= 32: x_prep + mfma_px
     size_t slab_bytes, part_floats;
 };
@@ -1282,7 +1335,9 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p) {
     if (n < 1 || n > kMaxMfmaGroup) return false;
     int tiles = 0;
     size_t rows = 0;
+    bool fine = false;  // chunks of 32 columns only (see kTwo)
     for (int i = 0; i < n; i++) {
+        fine = fine || d[i].type == 14 || d[i].type == 11;
         if (!mfma_applies(d[i], B) || d[i].cols != d[0].cols) return false;
         tiles += (d[i].row_end - d[i].row_start + kRowsPerWG - 1) / kRowsPerWG;
         rows += d[i].row_end - d[i].row_start;
@@ -1295,23 +1350,38 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p) {
     // split (the partials the last workgroup sums); the smallest split wins
     // ties.  Fitted to the 8B B = 32 shapes ([gate, up]: 2 splits 44 us,
     // 3 splits 57 us, 16 splits 96 us; [o]: 8 splits ahead of 16).
-    int best = 1 << 30;
+    // More than 64 columns: also over chunks of 32 and of 64 columns, whose steps
+    // cost 5 : 8 (2.6 and 4.2 us); a split never needs more scratch than the static
+    // one holds.  (9216 x 3072 Q8_0 at B = 128, 36 row tiles: 95 us in chunks of 64, 54 us
+    // in chunks of 32; 2 x 14336 x 4096 Q4_K, 112 row tiles: 96 us in chunks of 64.)
+    long long best = LLONG_MAX;
     p.ksb = p.nsb;
     p.ksplit = 1;
-    for (int ks = 1; ks <= p.nsb; ks++) {
-        const int ksb = (p.nsb + ks - 1) / ks, kse = (p.nsb + ksb - 1) / ksb;
-        if (kse > 1 && tiles > kMaxTileCounters) break;  // a split needs a counter per tile
-        const int rounds = (tiles * kse + kMinWorkgroups - 1) / kMinWorkgroups;
-        const int cost = 4 * (rounds * (ksb + 5) + (kse > 1 ? 1 : 0)) + (kse > 1 ? kse : 0);  // quarter steps
-        if (cost < best) {
-            best = cost;
-            p.ksb = ksb;
-            p.ksplit = kse;
+    const int row_tiles = tiles;
+    for (int c = B <= 64 || fine ? 32 : 64; c >= 32; c /= 2) {
+        const int chunks = B <= 64 ? 1 : (B + c - 1) / c;
+        if ((size_t)row_tiles * chunks > (size_t(1) << 30) / p.nsb) continue;  // the grid is an int
+        const int ctiles = row_tiles * chunks;
+        for (int ks = 1; ks <= p.nsb; ks++) {
+            const int ksb = (p.nsb + ks - 1) / ks, kse = (p.nsb + ksb - 1) / ksb;
+            if (kse > 1 && ctiles > kMaxTileCounters) break;  // a split needs a counter per tile
+            if (kse > 1 && B > 64 && sizeof(float) * (size_t)kse * B * rows > kStaticScratchBytes) break;
+            const int rounds = (int)(((long long)ctiles * kse + kMinWorkgroups - 1) / kMinWorkgroups);
+            const long long cost = (4ll * ((long long)rounds * (ksb + 5) + (kse > 1 ? 1 : 0)) + (kse > 1 ? kse : 0)) * (c == 64 ? 8 : 5);
+            if (cost < best) {
+                best = cost;
+                p.ksb = ksb;
+                p.ksplit = kse;
+                p.chunks = chunks;
+                p.chunk = c;
+            }
         }
     }
+    if (best == LLONG_MAX) return false;
+    tiles = row_tiles * p.chunks;
     if (const char *f = getenv("JUNO_MFMA_KSPLIT")) {  // tuning runs: a forced split
         const int want = atoi(f);
-        if (want >= 1 && want <= p.nsb && (want == 1 || tiles <= kMaxTileCounters)) {
+        if (B <= 64 && want >= 1 && want <= p.nsb && (want == 1 || tiles <= kMaxTileCounters)) {
             p.ksb = (p.nsb + want - 1) / want;
             p.ksplit = (p.nsb + p.ksb - 1) / p.ksb;
         }
@@ -1335,6 +1405,19 @@ int mfma_group_plan(int n, const MfmaDesc *d, int B, int *ksplit) {
     if (!plan_group(n, d, B, p)) return 0;
     *ksplit = p.ksplit;
     return p.prepared ? 2 : 1;
+}
+
+template <int NT>
+static void launch_wide(const MfmaGroup &g, int mask, int grid, hipStream_t s) {
+    switch (mask) {
+        case 1: mfma_group<false, NT, 1, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 2: mfma_group<false, NT, 2, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 4: mfma_group<false, 1, 4, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 8: mfma_group<false, NT, 8, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 16: mfma_group<false, NT, 16, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 32: mfma_group<false, 1, 32, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        default: mfma_group<false, NT, NT == 1 ? 63 : 27, false, true><<<grid, kThreads, 0, s>>>(g); break;
+    }
 }
 
 template <bool HL, int NT>
@@ -1508,12 +1591,15 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
         q.wg0 = wg;
         q.cnt0 = cnt;
         q.part0 = part;
-        wg += q.tiles * p.ksplit;
-        cnt += q.tiles;
+        wg += q.tiles * p.chunks * p.ksplit;
+        cnt += q.tiles * p.chunks;
         part += p.ksplit > 1 ? (size_t)p.ksplit * B * q.rows : 0;
         mask |= q.type == 12 ? 1 : q.type == 13 ? 2 : q.type == 14 ? 4 : q.type == 10 ? 16 : q.type == 11 ? 32 : 8;
     }
-    if (B <= kHlMaxBatch) launch_group_nt<true, 1>(g, mask, p.grid, s);
+    g.chunks = p.chunks;
+    if (B > 64 && p.chunk == 64) launch_wide<2>(g, mask, p.grid, s);
+    else if (B > 64) launch_wide<1>(g, mask, p.grid, s);
+    else if (B <= kHlMaxBatch) launch_group_nt<true, 1>(g, mask, p.grid, s);
     else if (B <= 32) launch_group_nt<false, 1>(g, mask, p.grid, s);
     else launch_group_nt<false, 2>(g, mask, p.grid, s);
     return hipGetLastError();

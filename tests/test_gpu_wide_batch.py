@@ -1,0 +1,101 @@
+"""More than 64 vectors: the MFMA kernels in column chunks (64 columns, with Q6_K or
+Q3_K in the launch 32), at the edges of the chunks, ragged row tiles, K split and
+not, one matrix and groups of mixed formats.
+
+Tolerance as for the smaller batches: 2^-18 of the absolute sum of a row's terms
+(some 40 roundings of partial sums) plus 2^-18 of their root sum of squares at the
+column's largest |x| (the 22-bit split of x, 30 standard deviations).
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle as O
+from juno_amd import _lib
+from juno_amd import matvec as mv
+from test_gpu_numerics import run
+from test_oracle_q2q3 import random_blocks
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [O.Q4_K, O.Q5_K, O.Q6_K, O.Q8_0, O.Q2_K, O.Q3_K]
+
+
+def weights(qtype, rows, cols, seed):
+    if qtype in (O.Q2_K, O.Q3_K):
+        return random_blocks(qtype, rows, cols, seed)
+    return O.quantize(qtype, (np.random.default_rng(seed).standard_normal(rows * cols) * 0.02).astype(np.float32))
+
+
+def check(Y, X, deq, label):
+    ref = X.astype(np.float64) @ deq.T
+    S = np.abs(X.astype(np.float64)) @ np.abs(deq).T
+    rss = np.sqrt(deq.shape[1]) * np.abs(deq).max(1)[None, :] * np.abs(X).max(1).astype(np.float64)[:, None]
+    worst = np.max(np.abs(Y.astype(np.float64) - ref) / (2.0 ** -18 * (S + rss)))
+    print(label, "worst / bound", worst, flush=True)
+    assert worst <= 1.0
+
+
+def upload(qtype, rows, cols, raw):
+    return mv.GpuContext.shared(0).create_mat_vec().upload_quant(
+        mv.QuantizedTensor("w", qtype, rows * cols, raw.tobytes()), rows, cols)
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("rows,cols,B", [(300, 256, 65), (300, 2048, 96), (257, 1024, 97), (31, 4096, 128), (520, 512, 130)])
+def test_wide_batch(qtype, rows, cols, B):
+    raw = weights(qtype, rows, cols, B)
+    deq = O.dequantize(qtype, raw, rows, cols).astype(np.float64).reshape(rows, cols)
+    X = np.random.default_rng(B).standard_normal((B, cols)).astype(np.float32)
+    L = _lib.load()
+    with upload(qtype, rows, cols, raw) as dev:
+        Y = run(dev, X, rows)
+        check(Y, X, deq, (qtype, rows, cols, B))
+        # without allocation: the same kernels, bit for bit
+        import torch
+        dx, dy = torch.from_numpy(X).cuda(), torch.empty(B, rows, device="cuda")
+        rc = L.jh_qmatvec_batched_noalloc_dev(dev.handle, ctypes.c_void_p(dx.data_ptr()), B,
+                                              ctypes.c_void_p(dy.data_ptr()), 0, rows, None)
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        assert np.array_equal(dy.cpu().numpy().view(np.uint32), Y.view(np.uint32))
+
+
+@pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q6_K), (O.Q4_K, O.Q8_0), (O.Q5_K, O.Q2_K, O.Q4_K, O.Q8_0)])
+@pytest.mark.parametrize("captured", [False, True])
+def test_wide_group(types, captured):
+    """A group in one launch; and captured on a stream that has no workspace yet, where
+    nothing may be allocated: the call is taken all the same."""
+    import torch
+    cols, B, rows = 1024, 100, [300, 64, 257, 33][:len(types)]
+    raws = [weights(t, r, cols, 7 + i) for i, (t, r) in enumerate(zip(types, rows))]
+    X = np.random.default_rng(5).standard_normal((B, cols)).astype(np.float32)
+    devs = [upload(t, r, cols, w) for t, r, w in zip(types, rows, raws)]
+    n, P, L = len(types), ctypes.c_void_p, _lib.load()
+    dx = torch.from_numpy(X).cuda()
+    ys = [torch.zeros(B, r, device="cuda") for r in rows]
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def call():
+        rc = L.jh_qmatvec_batched_group_dev(n, (P * n)(*[d.handle for d in devs]), (P * n)(*[dx.data_ptr()] * n), B,
+                                            (P * n)(*[y.data_ptr() for y in ys]), P(st.cuda_stream))
+        assert rc == 0, _lib.last_error()
+
+    with torch.cuda.stream(st):
+        if captured:
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=st):
+                call()
+            for _ in range(3):
+                for y in ys:
+                    y.zero_()
+                g.replay()
+        else:
+            call()
+    st.synchronize()
+    for t, r, w, y in zip(types, rows, raws, ys):
+        check(y.cpu().numpy(), X, O.dequantize(t, w, r, cols).astype(np.float64).reshape(r, cols), (t, r, captured))
+    for d in devs:
+        d.close()
