@@ -168,6 +168,20 @@ int staging_for(int device, size_t bx, size_t by, Staging **out) {
     return JH_OK;
 }
 
+// Copies between pinned staging and the device.  Up to 256 KB they are kernels, in
+// the stream's own queue, where a DMA copy adds the hand-over between engines; and
+// up to 128 KB of y is stored into host memory by the GEMV itself.  Host-pointer
+// call of one vector, us, DMA copies -> now: 256 x 2048 Q4_K 21.4 -> 19.2, 5000 x
+// 1024 Q6_K 28.7 -> 21.4, 20000 x 4096 Q8_0 47.0 -> 41.0, 4096 x 14336 Q4_K 38.2 ->
+// 33.1 (34.3 with y copied by a kernel).  The rest is the wait and the launches.
+constexpr size_t kKernelCopyBytes = 256u << 10, kDirectBytes = 128u << 10;
+
+int staged_copy(const char *what, const float *src, float *dst, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+    const hipError_t e = bytes <= kKernelCopyBytes ? jh::launch_copy_floats(src, dst, (int)(bytes / 4), s)
+                                                   : hipMemcpyAsync(dst, src, bytes, kind, s);
+    return e == hipSuccess ? JH_OK : hip_fail(what, e);
+}
+
 int check_qmat(const jh_qmat *m) {
     if (!m) return fail(JH_EINVAL, "A must not be null");
     if (!m->d_raw) return fail(JH_ECLOSED, "DeviceQuantMatrix is closed");
@@ -620,9 +634,10 @@ int jh_qmatvec_batched(jh_ctx *ctx, const jh_qmat *m, const float *X, int B, flo
     Staging *s;
     if ((rc = staging_for(ctx->device, bx, by, &s))) return rc;
     memcpy(s->h_x, X, bx);
-    JH_HIP("hipMemcpyAsync(x H2D)", hipMemcpyAsync(s->d_x, s->h_x, bx, hipMemcpyHostToDevice, s->stream));
-    if ((rc = enqueue_matvec(m, s->d_x, B, s->d_y, row_start, row_end, s->stream))) return rc;
-    JH_HIP("hipMemcpyAsync(y D2H)", hipMemcpyAsync(s->h_y, s->d_y, by, hipMemcpyDeviceToHost, s->stream));
+    if ((rc = staged_copy("x H2D", s->h_x, s->d_x, bx, hipMemcpyHostToDevice, s->stream))) return rc;
+    const bool direct = by <= kDirectBytes;  // the kernel writes y into host memory itself
+    if ((rc = enqueue_matvec(m, s->d_x, B, direct ? s->h_y : s->d_y, row_start, row_end, s->stream))) return rc;
+    if (!direct && (rc = staged_copy("y D2H", s->d_y, s->h_y, by, hipMemcpyDeviceToHost, s->stream))) return rc;
     JH_HIP("hipStreamSynchronize", hipStreamSynchronize(s->stream));
     memcpy(Y, s->h_y, by);
     return ok();

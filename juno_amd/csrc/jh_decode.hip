@@ -876,6 +876,20 @@ hipError_t launch_attention(const float *q, const float *k_new, const float *v_n
     return hipGetLastError();
 }
 
+// n floats between pinned host memory and the device, either way; both 16-byte aligned
+namespace {
+__global__ __launch_bounds__(256) void copy_floats(const float *__restrict__ src, float *__restrict__ dst, int n) {
+    const int i = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (i + 4 <= n) *reinterpret_cast<float4 *>(dst + i) = *reinterpret_cast<const float4 *>(src + i);
+    else
+        for (int k = i; k < n; k++) dst[k] = src[k];
+}
+}  // namespace
+hipError_t launch_copy_floats(const float *src, float *dst, int n, hipStream_t s) {
+    copy_floats<<<(n + 1023) / 1024, 256, 0, s>>>(src, dst, n);
+    return hipGetLastError();
+}
+
 hipError_t launch_silu_mul(const float *gate, const float *up, int n, float *out, hipStream_t s) {
     silu_mul_k<<<(n + 255) / 256, 256, 0, s>>>(gate, up, n, out);
     return hipGetLastError();

@@ -166,6 +166,7 @@ void attention_chunking(int n_heads, int n_kv_heads, int head_dim, int max_seq, 
 // queue on one line's atomics.  Every launch leaves the counters it used at zero.
 constexpr int kCounterSlots = 1024;
 constexpr int kCounterStride = 32;  // ints
+hipError_t launch_copy_floats(const float *src, float *dst, int n, hipStream_t s);
 hipError_t launch_silu_mul(const float *gate, const float *up, int n, float *out, hipStream_t s);
 // y[b] += scale * B (A x[b]) for b < batch; h_ws holds batch * rank floats.
 hipError_t launch_lora(const float *a, const float *b, int rank, int in_dim, int out_dim, float scale, const float *x,
