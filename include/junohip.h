@@ -157,7 +157,7 @@ int jh_qmat_dequant_dev(const jh_qmat *m, float *d_out, void *stream);
  * on a device shares that device's array, which keeps the last call's
  * contents: calls that overlap on one device (two streams, or a graph replay
  * beside an eager call) race and must be ordered by the caller.  Results are
- * those of jh_qmatvec_batched_dev, bit for bit (calls of more than 64 vectors
+ * those of jh_qmatvec_batched_dev, bit for bit (calls of two and of more than 64 vectors
  * never need more than that array; jh_qmatvec_batched_dev captured before its
  * stream has a workspace takes kernels without scratch for them instead). */
 int jh_qmatvec_batched_noalloc_dev(const jh_qmat *m, const float *d_X, int B, float *d_Y, int row_start,

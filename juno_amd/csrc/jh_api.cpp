@@ -261,14 +261,15 @@ int stream_workspace(int device, hipStream_t s, size_t bytes, void **out, int **
     return JH_OK;
 }
 
-// The MFMA path for a group of matrices sharing K (B >= kMfmaMinBatch): kMfmaNotApplicable
+// The MFMA path for a group of matrices sharing K (B >= 2): kMfmaNotApplicable
 // (never returned through the C ABI) when it does not apply, so that the caller
 // can take the per-matrix kernels.
 constexpr int kMfmaNotApplicable = -1;
 
-// More than 64 columns use the workspace only to split K, and where the stream has
-// none to give (a graph capture before any eager call, no memory left) they take
-// the per-matrix kernels, which need none.
+// Two vectors, and more than 64 (which use the workspace only to split K), took the
+// per-matrix kernels without scratch before this path did: where the stream has no
+// workspace to give (a graph capture before any eager call, no memory left) they
+// still do.
 int enqueue_mfma_group(int device, int n, const jh::MfmaDesc *d, int B, hipStream_t s) {
     const size_t wsb = jh::mfma_group_workspace_bytes(n, d, B);
     if (!wsb) return kMfmaNotApplicable;
@@ -276,7 +277,7 @@ int enqueue_mfma_group(int device, int n, const jh::MfmaDesc *d, int B, hipStrea
     int *counters = nullptr;
     int rc = 0, ksplit = 1;
     if (B <= 64 || (jh::mfma_group_plan(n, d, B, &ksplit) && ksplit > 1)) rc = stream_workspace(device, s, wsb, &ws, &counters);
-    if (rc) return B <= 64 ? rc : kMfmaNotApplicable;
+    if (rc) return B >= jh::kMfmaMinBatch && B <= 64 ? rc : kMfmaNotApplicable;
     hipError_t e = jh::launch_mfma_group(n, d, B, ws, counters, s);
     if (e == hipSuccess) return JH_OK;
     if (e == hipErrorNotSupported) return kMfmaNotApplicable;
@@ -284,7 +285,7 @@ int enqueue_mfma_group(int device, int n, const jh::MfmaDesc *d, int B, hipStrea
 }
 
 // Enqueue y = W x for B vectors (device pointers), splitting B into the
-// kernel's supported batch widths, or using the MFMA path for B >= kMfmaMinBatch.
+// kernel's supported batch widths, or using the MFMA path where it applies.
 int enqueue_matvec(const jh_qmat *m, const float *d_x, int B, float *d_y, int row_start, int row_end,
                    hipStream_t s, bool mfma = true) {
     const int nrows = row_end - row_start;
@@ -298,7 +299,7 @@ int enqueue_matvec(const jh_qmat *m, const float *d_x, int B, float *d_y, int ro
     a.row_end = row_end;
     a.ldx = m->cols;
     a.ldy = nrows;
-    if (B >= jh::kMfmaMinBatch && mfma) {
+    if (B >= 2 && mfma) {
         const jh::MfmaDesc d{m->type, m->d_raw, m->pitch, m->cols, row_start, row_end, d_x, d_y};
         int rc = enqueue_mfma_group(m->ctx->device, 1, &d, B, s);
         if (rc != kMfmaNotApplicable) return rc;
@@ -358,7 +359,7 @@ int jh_qmatvec_batched_plan_shape(int ggml_type, int cols, int row_start, int ro
     const jh::MfmaDesc d{ggml_type, w, (size_t)(cols / qk) * bb, cols, row_start, row_end,
                          reinterpret_cast<const float *>(w), nullptr};
     *ksplit = 1;
-    *kernel = B >= jh::kMfmaMinBatch ? jh::mfma_group_plan(1, &d, B, ksplit) : 0;
+    *kernel = B >= 2 ? jh::mfma_group_plan(1, &d, B, ksplit) : 0;
     return ok();
 }
 
@@ -374,7 +375,7 @@ int jh_qmatvec_batched_plan(int n, const jh_qmat *const *mats, int B, int *kerne
                             reinterpret_cast<const float *>(mats[i]->d_raw), nullptr};
     }
     *ksplit = 1;
-    *kernel = B >= jh::kMfmaMinBatch ? jh::mfma_group_plan(n, d, B, ksplit) : 0;
+    *kernel = B >= 2 ? jh::mfma_group_plan(n, d, B, ksplit) : 0;
     return ok();
 }
 
@@ -710,7 +711,7 @@ int jh_qmatvec_batched_noalloc_dev(const jh_qmat *m, const float *d_X, int B, fl
     if (!d_X || !d_Y) return fail(JH_EINVAL, "x and y must not be null");
     if ((rc = set_device(m->ctx->device))) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (B >= jh::kMfmaMinBatch) {
+    if (B >= 2) {
         const jh::MfmaDesc d{m->type, m->d_raw, m->pitch, m->cols, row_start, row_end, d_X, d_Y};
         const size_t wsb = jh::mfma_group_workspace_bytes(1, &d, B);
         if (wsb) {
@@ -950,14 +951,17 @@ int jh_qmatvec_batched_swiglu_dev(const jh_qmat *gate, const jh_qmat *up, const 
     hipStream_t s = (hipStream_t)stream;
     const jh::MfmaDesc dg{gate->type, gate->d_raw, gate->pitch, gate->cols, 0, gate->rows, d_X, nullptr};
     const jh::MfmaDesc du{up->type, up->d_raw, up->pitch, up->cols, 0, up->rows, d_X, nullptr};
-    if (jh::mfma_swiglu_applies(dg, du, B)) {
+    if (jh::mfma_swiglu_applies(dg, du, B) && (B >= jh::kMfmaMinBatch || (d_gate && d_up))) {
         const int dev = gate->ctx->device;
         void *ws = nullptr;
         int *counters = nullptr;
-        if ((rc = stream_workspace(dev, s, jh::mfma_swiglu_workspace_bytes(dg, B), &ws, &counters))) return rc;
-        hipError_t e = jh::launch_mfma_swiglu(dg, du, B, d_out, ws, counters, s);
-        if (e == hipSuccess) return ok();
-        if (e != hipErrorNotSupported) return hip_fail("mfma swiglu launch", e);
+        rc = stream_workspace(dev, s, jh::mfma_swiglu_workspace_bytes(dg, B), &ws, &counters);
+        if (rc && B >= jh::kMfmaMinBatch) return rc;
+        if (!rc) {
+            hipError_t e = jh::launch_mfma_swiglu(dg, du, B, d_out, ws, counters, s);
+            if (e == hipSuccess) return ok();
+            if (e != hipErrorNotSupported) return hip_fail("mfma swiglu launch", e);
+        }
     }
     if (!d_gate || !d_up) return fail(JH_EINVAL, "gate and up scratch must not be null on this path (B=%d)", B);
     const jh_qmat *mats[2] = {gate, up};
@@ -987,7 +991,7 @@ int jh_qmatvec_batched_group_dev(int n, const jh_qmat *const *mats, const float 
         d[i] = jh::MfmaDesc{mats[i]->type, mats[i]->d_raw, mats[i]->pitch, mats[i]->cols, 0, mats[i]->rows, d_X[i], d_Y[i]};
     }
     hipStream_t s = (hipStream_t)stream;
-    if (B >= jh::kMfmaMinBatch) {
+    if (B >= 2) {
         rc = enqueue_mfma_group(mats[0]->ctx->device, n, d, B, s);
         if (rc != kMfmaNotApplicable) return rc ? rc : ok();
     }

@@ -94,7 +94,7 @@ struct CombineSpec {
 // check_only: hipSuccess when it applies, nothing launched
 hipError_t launch_gemv_staged_combine(const GemvArgs &a, const CombineSpec &c, hipStream_t s, bool check_only = false);
 
-// Batched GEMVs (B >= kMfmaMinBatch) on fp16 MFMA, staged through LDS: up to kMaxMfmaGroup matrices
+// Batched GEMVs (B >= kMfmaMinBatch, large ones from B = 2) on fp16 MFMA, staged through LDS: up to kMaxMfmaGroup matrices
 // with the same cols, each with its own x [B][cols] and y [B][row_end -
 // row_start], in one launch.  mfma_group_workspace_bytes returns 0 when the
 // path does not apply (types, shapes, alignment); otherwise launch_mfma_group
@@ -110,9 +110,10 @@ struct MfmaDesc {
     float *y;
 };
 constexpr int kMaxMfmaGroup = 4;
-// Smallest batch that takes the MFMA path.  The x tile is padded to 32 columns, so a launch costs about the same from
-// B = 3 to 32.  Measured 8B GEMV step: B = 2 3.24 ms (VALU kernels) vs 3.78 ms (MFMA); B = 3 5.54 vs 3.80 ms; B = 8
-// 15.4 vs 3.88 ms.
+// From this batch on every shape the path supports takes it: its fixed costs are
+// those of up to 16 columns, while the VALU kernels read the weights once per 8, 4, 2
+// or 1 columns.  8B GEMV step: B = 3 5.54 ms on the VALU kernels, 3.80 ms here; B = 8
+// 15.4 and 3.88 ms.  Two columns take it where plan_group's rule says so.
 constexpr int kMfmaMinBatch = 3;
 size_t mfma_group_workspace_bytes(int n, const MfmaDesc *d, int B);
 hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, int *counters, hipStream_t s);
@@ -126,7 +127,7 @@ int mfma_group_plan(int n, const MfmaDesc *d, int B, int *ksplit);
 // call on a device, zeroes the counters with a kernel on stream s.
 constexpr size_t kStaticScratchBytes = 8u << 20;
 hipError_t static_scratch(int device, hipStream_t s, void **workspace, int **counters);
-// out[b][r] = silu(gate_r . x_b) * (up_r . x_b) for 3 <= B <= 32: one MFMA
+// out[b][r] = silu(gate_r . x_b) * (up_r . x_b) for 2 <= B <= 32: one MFMA
 // launch whose workgroups take 128 rows of gate and the same 128 rows of up
 // (Q4_K, Q5_K, Q6_K, Q8_0; full row ranges, same shape and x).
 bool mfma_swiglu_applies(const MfmaDesc &gate, const MfmaDesc &up, int B);

@@ -1,4 +1,4 @@
-// jh_mfma.hip -- batched GEMVs (B >= 3) on Q4_K / Q5_K / Q6_K / Q8_0 through
+// jh_mfma.hip -- batched GEMVs (B >= 2) on Q4_K / Q5_K / Q6_K / Q8_0 through
 // LDS + fp16 MFMA.
 //
 // Y[b][r] = sum_c deq(W[r][c]) * X[b][c] is a dense contraction once B >= 16:
@@ -1312,7 +1312,7 @@ constexpr int kHlMaxBatch = 16;
 
 static bool mfma_applies(const MfmaDesc &d, int B) {
     if ((d.type != 12 && d.type != 13 && d.type != 14 && d.type != 8 && d.type != 10 && d.type != 11) ||
-        B < kMfmaMinBatch || d.cols % 256 ||
+        B < 2 || d.cols % 256 ||
         d.cols <= 0 || d.row_end <= d.row_start)
         return false;
     if (d.pitch > (size_t(1) << 26)) return false;  // 32 rows' offsets in 32 bits
@@ -1341,7 +1341,15 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p) {
         if (!mfma_applies(d[i], B) || d[i].cols != d[0].cols) return false;
         tiles += (d[i].row_end - d[i].row_start + kRowsPerWG - 1) / kRowsPerWG;
         rows += d[i].row_end - d[i].row_start;
+        if (B == 2 && d[i].type != 12 && d[i].type != 13 && d[i].type != 8) return false;
     }
+    // Two vectors: from 26 M weights on, in a group (a launch each otherwise) from 20 M,
+    // where the VALU kernels' arithmetic outweighs this path's fixed 9 us.  us, VALU / MFMA:
+    // 6144 x 4096 Q4_K 10.4 / 11.0, 9216 x 3072 13.8 / 11.6 and Q8_0 20.7 / 14.6, 2 x 2816 x
+    // 2048 10.2 / 9.5 (Q5_K 11.1 / 10.9, Q8_0 13.1 / 12.1), 2 x 5632 x 2048 12.7 / 9.9.
+    // Q4_K, Q5_K and Q8_0, whose error against 64 bits is smaller here (K = 4096: Q4_K
+    // 2.5e-7 / 1.8e-7, Q8_0 1.33e-7 / 1.0e-7); that of Q6_K and Q3_K is not.
+    if (B == 2 && (double)rows * d[0].cols < (n == 1 ? 26e6 : 20e6)) return false;
     p.nsb = d[0].cols / 256;
     // One workgroup fits per CU (LDS, VGPRs), so the grid runs in rounds of
     // kMinWorkgroups.  Cost of a split, in super-block steps: rounds x (super-
@@ -1390,7 +1398,8 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p) {
     p.prepared = n == 1 && p.ksplit == 1 && B <= 32 && d[0].type != 10 && d[0].type != 11;  // slabs carry no 16-column sums
     p.slab_bytes = p.prepared ? (size_t)p.nsb * (B <= kHlMaxBatch ? Slab<true>::kBytes : Slab<false>::kBytes) : 0;
     p.part_floats = p.ksplit > 1 ? (size_t)p.ksplit * B * rows : 0;
-    return true;
+    // two vectors never need more scratch than the static one holds
+    return B != 2 || p.slab_bytes + p.part_floats * sizeof(float) <= kStaticScratchBytes;
 }
 
 size_t mfma_group_workspace_bytes(int n, const MfmaDesc *d, int B) {
@@ -1444,7 +1453,7 @@ static bool mfma_pair_wanted() {
 
 bool mfma_swiglu_applies(const MfmaDesc &gate, const MfmaDesc &up, int B) {
     if (!mfma_pair_wanted()) return false;
-    if (B < kMfmaMinBatch || B > 32 || gate.type != up.type || gate.cols != up.cols || gate.pitch != up.pitch ||
+    if (B < 2 || B > 32 || gate.type != up.type || gate.cols != up.cols || gate.pitch != up.pitch ||
         gate.x != up.x || gate.row_start != 0 || up.row_start != 0 || gate.row_end != up.row_end)
         return false;
     if (gate.type != 12 && gate.type != 13 && gate.type != 14 && gate.type != 8) return false;

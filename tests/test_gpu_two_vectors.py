@@ -1,0 +1,95 @@
+"""Two vectors on either side of the size from which they take the MFMA kernels,
+single matrices, row ranges, a group and the SwiGLU pair, eager and captured on a
+stream without a workspace; and what is refused without scratch buffers.
+
+Tolerance as for the other batches: 2^-18 of the absolute sum of a row's terms plus
+2^-18 of their root sum of squares at the column's largest |x|.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle as O
+from juno_amd import _lib
+from juno_amd import matvec as mv
+from test_gpu_wide_batch import check, upload, weights
+
+pytestmark = pytest.mark.gpu
+P = ctypes.c_void_p
+
+
+
+
+@pytest.mark.parametrize("captured", [False, True])
+@pytest.mark.parametrize("qtype,rows,cols,lo", [
+    (O.Q4_K, 6347, 4096, 0), (O.Q4_K, 6348, 4096, 0), (O.Q4_K, 1950, 14336, 37), (O.Q8_0, 8465, 3072, 0),
+    (O.Q8_0, 13000, 2080, 0), (O.Q5_K, 33100, 1024, 300), (O.Q6_K, 6500, 4096, 0)])
+def test_two_vectors(qtype, rows, cols, lo, captured):
+    import torch
+    L = _lib.load()
+    raw = weights(qtype, rows, cols, 3)
+    X = np.random.default_rng(4).standard_normal((2, cols)).astype(np.float32)
+    n = rows - lo
+    with upload(qtype, rows, cols, raw) as dev:
+        dx, y, z = torch.from_numpy(X).cuda(), torch.zeros(2, n, device="cuda"), torch.zeros(2, n, device="cuda")
+        st = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            g = torch.cuda.CUDAGraph()
+            if captured:
+                g.capture_begin()
+            assert L.jh_qmatvec_batched_dev(dev.handle, P(dx.data_ptr()), 2, P(y.data_ptr()), lo, rows, P(st.cuda_stream)) == 0
+            if captured:
+                g.capture_end()
+                for _ in range(3):
+                    y.zero_()
+                    g.replay()
+            assert L.jh_qmatvec_batched_noalloc_dev(dev.handle, P(dx.data_ptr()), 2, P(z.data_ptr()), lo, rows,
+                                                    P(st.cuda_stream)) == 0, _lib.last_error()
+        st.synchronize()
+        if not captured:
+            assert torch.equal(y, z)
+    deq = O.dequantize(qtype, raw, rows, cols).reshape(rows, cols)[lo:].astype(np.float64)
+    check(y.cpu().numpy(), X, deq, (qtype, rows, cols, captured))
+
+
+@pytest.mark.parametrize("rows,cols", [(4096, 2560), (5120, 2560)])
+@pytest.mark.parametrize("captured", [False, True])
+def test_two_vector_swiglu(rows, cols, captured):
+    import torch
+    L = _lib.load()
+    raws = [weights(O.Q4_K, rows, cols, 8 + i) for i in range(2)]
+    X = np.random.default_rng(6).standard_normal((2, cols)).astype(np.float32)
+    with upload(O.Q4_K, rows, cols, raws[0]) as gate, upload(O.Q4_K, rows, cols, raws[1]) as up:
+        dx = torch.from_numpy(X).cuda()
+        out, a, b = (torch.zeros(2, rows, device="cuda") for _ in range(3))
+        st = torch.cuda.Stream()
+        torch.cuda.synchronize()
+
+        def call(pa, pb):
+            return L.jh_qmatvec_batched_swiglu_dev(gate.handle, up.handle, P(dx.data_ptr()), 2, P(out.data_ptr()), pa, pb,
+                                                   P(st.cuda_stream))
+
+        assert call(None, None) == _lib.JH_EINVAL  # two vectors need the scratch buffers, whatever the kernel
+        with torch.cuda.stream(st):
+            g = torch.cuda.CUDAGraph()
+            if captured:
+                g.capture_begin()
+            assert call(P(a.data_ptr()), P(b.data_ptr())) == 0, _lib.last_error()
+            if captured:
+                g.capture_end()
+                for _ in range(3):
+                    out.zero_()
+                    g.replay()
+        st.synchronize()
+        Y = out.cpu().numpy().astype(np.float64)
+    dg, du = (O.dequantize(O.Q4_K, r, rows, cols).reshape(rows, cols).astype(np.float64) for r in raws)
+    x64 = X.astype(np.float64)
+    u, v = x64 @ dg.T, x64 @ du.T
+    silu = u / (1.0 + np.exp(-u))
+    # the two sums' errors carried through silu (slope at most 1.1) and the product, and the product's own rounding
+    eps = [2.0 ** -18 * (np.abs(x64) @ np.abs(d).T + np.sqrt(cols) * np.abs(d).max(1)[None] * np.abs(x64).max(1)[:, None])
+           for d in (dg, du)]
+    bound = 1.1 * eps[0] * np.abs(v) + np.abs(silu) * eps[1] + 2 * eps[0] * eps[1] + 2.0 ** -20 * np.abs(silu * v)
+    assert np.max(np.abs(Y - silu * v) / bound) <= 1.0
