@@ -13,7 +13,7 @@ import pytest
 import oracle as O
 from juno_amd import _lib
 from juno_amd import matvec as mv
-from test_gpu_wide_batch import check, upload, weights
+from test_gpu_wide_batch import check, fresh_stream, upload, weights
 
 pytestmark = pytest.mark.gpu
 P = ctypes.c_void_p
@@ -33,7 +33,7 @@ def test_two_vectors(qtype, rows, cols, lo, captured):
     n = rows - lo
     with upload(qtype, rows, cols, raw) as dev:
         dx, y, z = torch.from_numpy(X).cuda(), torch.zeros(2, n, device="cuda"), torch.zeros(2, n, device="cuda")
-        st = torch.cuda.Stream()
+        st = fresh_stream() if captured else torch.cuda.current_stream()
         torch.cuda.synchronize()
         with torch.cuda.stream(st):
             g = torch.cuda.CUDAGraph()
@@ -64,7 +64,7 @@ def test_two_vector_swiglu(rows, cols, captured):
     with upload(O.Q4_K, rows, cols, raws[0]) as gate, upload(O.Q4_K, rows, cols, raws[1]) as up:
         dx = torch.from_numpy(X).cuda()
         out, a, b = (torch.zeros(2, rows, device="cuda") for _ in range(3))
-        st = torch.cuda.Stream()
+        st = fresh_stream() if captured else torch.cuda.current_stream()
         torch.cuda.synchronize()
 
         def call(pa, pb):

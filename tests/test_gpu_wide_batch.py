@@ -37,6 +37,15 @@ def check(Y, X, deq, label):
     assert worst <= 1.0
 
 
+def fresh_stream():
+    """A stream that has never been used (torch's streams come round again from a pool,
+    with the workspace of their earlier use); it stays for the process."""
+    import torch
+    s = ctypes.c_void_p()
+    assert _lib.load().hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0  # non-blocking
+    return torch.cuda.ExternalStream(s.value)
+
+
 def upload(qtype, rows, cols, raw):
     return mv.GpuContext.shared(0).create_mat_vec().upload_quant(
         mv.QuantizedTensor("w", qtype, rows * cols, raw.tobytes()), rows, cols)
@@ -75,7 +84,7 @@ def test_wide_group(types, captured):
     n, P, L = len(types), ctypes.c_void_p, _lib.load()
     dx = torch.from_numpy(X).cuda()
     ys = [torch.zeros(B, r, device="cuda") for r in rows]
-    st = torch.cuda.Stream()
+    st = fresh_stream() if captured else torch.cuda.current_stream()
     torch.cuda.synchronize()
 
     def call():
