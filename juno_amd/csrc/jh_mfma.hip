@@ -87,6 +87,10 @@ __device__ __forceinline__ void for_c(F f) {
     for_seq(f, std::make_integer_sequence<int, N>{});
 }
 
+// Maximum and minimum, NaN if an operand is (v_maximum3_f32, v_minimum3_f32).
+__device__ __forceinline__ float larger(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float smaller(float a, float b) { return __builtin_elementwise_minimum(a, b); }
+
 // Maximum over the 16 lanes of one DPP row (lanes 16 r .. 16 r + 15): xor-1 and
 // xor-2 butterflies, then the half-row and row mirrors.
 template <int CTRL>
@@ -94,10 +98,10 @@ __device__ __forceinline__ float dpp_f(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 __device__ __forceinline__ float row16_max(float v) {
-    v = fmaxf(v, dpp_f<0xB1>(v));   // quad_perm 1,0,3,2
-    v = fmaxf(v, dpp_f<0x4E>(v));   // quad_perm 2,3,0,1
-    v = fmaxf(v, dpp_f<0x141>(v));  // row_half_mirror
-    return fmaxf(v, dpp_f<0x140>(v));  // row_mirror
+    v = larger(v, dpp_f<0xB1>(v));   // quad_perm 1,0,3,2
+    v = larger(v, dpp_f<0x4E>(v));   // quad_perm 2,3,0,1
+    v = larger(v, dpp_f<0x141>(v));  // row_half_mirror
+    return larger(v, dpp_f<0x140>(v));  // row_mirror
 }
 
 // One column and super-block of x as MFMA operands: 16 consecutive lanes hold
@@ -109,17 +113,56 @@ __device__ __forceinline__ float row16_max(float v) {
 // become fp16 pairs (b0, b2), (b1, b3) by a mask alone.  The 16-value sums times
 // 2^-4 and (even q) the 32-value sums times 2^-5 stay in fp16's range for any x.
 // All sums run in fixed orders.
+//
+// EXACT (two vectors and more than 64, which the fp32 kernels took before): what the
+// limbs cannot hold.  lo is rounded to 2^-37 of the block's largest |x|, so a block is
+// left out -- zeros in place of it, and cs = -1, for which the wave adds its fp32
+// products after the walk (add_exact) -- when (unfit)
+//  * an element is not finite;
+//  * a nonzero one is below 2^-27 of the largest (it would keep fewer than 10 bits);
+//  * four neighbours are all below 2^-14 of it, and not all 0 (together they would
+//    keep fewer than the 23 bits that the limbs give the others).
+// Normal x meets the second about once in 10^7 elements, a product of two about once
+// in 10^6, and never the others.  The quick test takes zeros for small elements; the
+// right one runs where it fails.  Cost on ordinary x, us, without / with: 2 x 14336 x
+// 4096 Q4_K at B = 128 92.5 / 94.7, B = 2 24.3 / 24.6; 9216 x 3072 Q8_0 53.2 / 53.8, 14.6 / 14.75.
 constexpr int kXsShift = 5, kX16Shift = 4;
+// largest |x|, smallest nonzero one, smallest nonzero maximum of four neighbours
+__device__ __forceinline__ bool unfit(float m, float lone, float four) {
+    return !(m < INFINITY) || lone < m * 0x1p-27f || four < m * 0x1p-14f;
+}
 struct XColumn {
     half8 h[2], l[2];
     float s16, s32, cs;
 };
-__device__ __forceinline__ XColumn split_x(const float (&xv)[16]) {
+template <bool EXACT>
+__device__ __forceinline__ XColumn split_x(const float (&x_in)[16]) {
     XColumn r;
-    float m = 0.f;
+    float xv[16], quad[4];
 #pragma unroll
-    for (int j = 0; j < 16; j++) m = fmaxf(m, fabsf(xv[j]));
-    m = row16_max(m);  // the 16 lanes of the column
+    for (int j = 0; j < 16; j++) xv[j] = x_in[j];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        quad[j] = larger(larger(fabsf(xv[4 * j]), fabsf(xv[4 * j + 1])), larger(fabsf(xv[4 * j + 2]), fabsf(xv[4 * j + 3])));
+    float m = row16_max(larger(larger(quad[0], quad[1]), larger(quad[2], quad[3])));  // the 16 lanes of the column
+    bool bad = false;
+    if constexpr (EXACT) {
+        float lone = fabsf(xv[0]);
+#pragma unroll
+        for (int j = 1; j < 16; j++) lone = smaller(lone, fabsf(xv[j]));
+        const float four = smaller(smaller(quad[0], quad[1]), smaller(quad[2], quad[3]));
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(unfit(m, lone, four)) != 0, 0)) {  // of the wave's four columns
+            float lo = INFINITY, lo4 = INFINITY;
+#pragma unroll
+            for (int j = 0; j < 16; j++) lo = xv[j] != 0.f ? fminf(lo, fabsf(xv[j])) : lo;
+#pragma unroll
+            for (int j = 0; j < 4; j++) lo4 = quad[j] != 0.f ? fminf(lo4, quad[j]) : lo4;
+            bad = ((__builtin_amdgcn_ballot_w64(unfit(m, lo, lo4)) >> (threadIdx.x & 48)) & 0xFFFF) != 0;
+            m = bad ? 0.f : m;
+#pragma unroll
+            for (int j = 0; j < 16; j++) xv[j] = bad ? 0.f : xv[j];
+        }
+    }
     int k = 0;
     if (m > 0.f) {
         int e;
@@ -127,7 +170,7 @@ __device__ __forceinline__ XColumn split_x(const float (&xv)[16]) {
         k = min(13 - e, 126);  // both 2^k and 2^-k are normal
     }
     const float s = ldexpf(1.f, k);
-    r.cs = ldexpf(1.f, -k);
+    r.cs = bad ? -1.f : ldexpf(1.f, -k);
 #pragma unroll
     for (int u = 0; u < 2; u++)
 #pragma unroll
@@ -158,7 +201,7 @@ __device__ __forceinline__ XColumn split_x(const float (&xv)[16]) {
 //   x(n, off) / xlo(n, off)  unit at column offset off, column group n
 //   xs(n)                    the 8 32-value sums, limb kh (hi, lo)
 //   x16(n, limb)             the 16-value sums 8 kh .. +8
-//   cs()                     1 / scale per batch column
+//   cs()                     1 / scale per batch column (-1: the block is left to add_exact)
 // The sums' rows 16..31 are zero with HL.
 constexpr int COLH = 256 + kXPad;  // halves per LDS column of the staged x slice
 
@@ -173,9 +216,9 @@ struct XImage {
     static constexpr int kCs = 2 * (kX16 + 32 * NT * 32);      // bytes: 32 NT floats
     static constexpr int kBytes = kCs + 32 * NT * 4;
     // one lane's share of column col (lane q of its 16), with the sums that the format reads
-    template <int SUMS>
+    template <int SUMS, bool EXACT>
     static __device__ __forceinline__ void store(uint8_t *buf, const float (&xv)[16], int q, int col) {
-        const XColumn x = split_x(xv);
+        const XColumn x = split_x<EXACT>(xv);
         _Float16 *base = reinterpret_cast<_Float16 *>(buf), *hi = base + col * COLH + 16 * q;
 #pragma unroll
         for (int u = 0; u < 2; u++) {
@@ -230,8 +273,9 @@ struct Slab {
     static constexpr int kRows = kXs / 1024 + 2;  // 1 KB DMA rows
     static constexpr int kBytes = kRows * 1024;
     static __device__ __forceinline__ int slot(int v, int off) { return 16 * ((v << 5) | ((off >> 3) ^ v)); }
+    template <bool EXACT>
     static __device__ __forceinline__ void store(uint8_t *slab, const float (&xv)[16], int q, int col) {
-        const XColumn x = split_x(xv);
+        const XColumn x = split_x<EXACT>(xv);
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             *reinterpret_cast<half8 *>(slab + slot(col, 8 * (2 * q + u))) = x.h[u];
@@ -339,6 +383,10 @@ __device__ __forceinline__ u32x4 lds_u32x4(const uint8_t *p) {
     return u32x4{v[0], v[1], v[2], v[3]};
 }
 
+// 16 bytes at a 2-byte-aligned address in memory (one load on gfx950)
+typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ u32x4 load16(const uint8_t *p) { return *reinterpret_cast<const u32x4a2 *>(p); }
+
 // Window position (in chunks) of chunk j of a wave's 32 x CH chunk grid when
 // rows are RC >= CH chunks apart.
 template <int CH, int RC>
@@ -349,6 +397,7 @@ __device__ __forceinline__ int win_chunk(int j) { return RC == CH ? j : j + (RC 
 //   Regs                  the lane's weight bytes (row lr, K half kh), in VGPRs
 //   load(r, p, kh)        p = first byte of the row's stretch, in LDS
 //   compute<HL, NT>(...)  the MFMAs and the fold into the fp32 totals
+//   run(p, t, ..)         16 columns' quants and scales (p in memory), for add_exact
 // K-step t covers 16 columns; lane half kh supplies 8 of them.  Every weight
 // enters the MFMA as an exact fp16 integer (or half-integer); scales are applied
 // in fp32.  Quants of a sub-block with a nonzero min are centred (Q4_K q - 8, Q5_K
@@ -450,6 +499,20 @@ struct FmtKQ {
             r.qh[1] = *reinterpret_cast<const u32x2 *>(p + 32 + 8 * kh);
         }
     }
+    // run t: 16 columns from 16 t on as bytes q + kBias, their scale and min
+    static constexpr int kBias = 0;
+    static constexpr bool kMin = true;
+    static __device__ __forceinline__ u32x4 run(const uint8_t *p, int t, float &sc, float &mn) {
+        const int s = t >> 1, hf = t & 1;
+        const u32x4 hd = load16(p);
+        int ls, lm;
+        q4k_scale_min(hd.y, hd.z, hd.w, s, ls, lm);
+        sc = half_bits_to_float(hd.x) * (float)ls;
+        mn = half_bits_to_float(hd.x >> 16) * (float)lm;
+        u32x4 q = (load16(p + kQs + 32 * (s >> 1) + 16 * hf) >> (4 * (s & 1))) & 0x0F0F0F0Fu;
+        if (Q5) q |= ((load16(p + 16 + 16 * hf) >> s) & 0x01010101u) << 4;
+        return q;
+    }
     // the pair of one dword's bytes (odd ? (b1, b3) : (b0, b2)) of sub-block s
     template <int S, int ODD>
     static __device__ __forceinline__ half2v pair(uint32_t w, uint32_t hb, half2v ls, half2v off, uint32_t top) {
@@ -547,6 +610,16 @@ struct FmtQ6K {
         lds_read_u<1>(p + 206, dw);
         r.dw = dw[0];
     }
+    // run t: 16 columns from 16 t on as bytes q + kBias, their scale and min
+    static constexpr int kBias = 32;
+    static constexpr bool kMin = false;
+    static __device__ __forceinline__ u32x4 run(const uint8_t *p, int t, float &sc, float &mn) {
+        const int n = t >> 3, qd = (t >> 1) & 3, j = t & 1;
+        sc = half_bits_to_float(*reinterpret_cast<const uint16_t *>(p + 208)) * (float)(int8_t)p[192 + t];
+        mn = 0.f;
+        return ((load16(p + 64 * n + 32 * (qd & 1) + 16 * j) >> (qd >= 2 ? 4 : 0)) & 0x0F0F0F0Fu) |
+               (((load16(p + 128 + 32 * n + 16 * j) >> (2 * qd)) & 0x03030303u) << 4);
+    }
     template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1056.f);  // 1024 + 32
@@ -584,6 +657,14 @@ struct FmtQ8_0 {
         const uint8_t *p;  // 40 registers of quants and scales would spill: each block is read ahead of its MFMAs
     };
     static __device__ __forceinline__ void load(Regs &r, const uint8_t *p, int) { r.p = p; }
+    // run t: 16 columns from 16 t on as bytes q + kBias, their scale and min
+    static constexpr int kBias = 128;
+    static constexpr bool kMin = false;
+    static __device__ __forceinline__ u32x4 run(const uint8_t *p, int t, float &sc, float &mn) {
+        sc = half_bits_to_float(*reinterpret_cast<const uint16_t *>(p + 34 * (t >> 1)));
+        mn = 0.f;
+        return load16(p + 34 * (t >> 1) + 2 + 16 * (t & 1)) ^ 0x80808080u;
+    }
     template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1152.f);  // 1024 + 128
@@ -646,6 +727,16 @@ struct FmtQ2K {
         uint32_t dm[1];
         lds_read_u<1>(p + 80, dm);
         r.dm = dm[0];
+    }
+    // run t: 16 columns from 16 t on as bytes q + kBias, their scale and min
+    static constexpr int kBias = 0;
+    static constexpr bool kMin = true;
+    static __device__ __forceinline__ u32x4 run(const uint8_t *p, int t, float &sc, float &mn) {
+        const int k = t & 7;
+        const uint32_t dm = *reinterpret_cast<const uint32_t *>(p + 80);
+        sc = half_bits_to_float(dm) * (float)(p[t] & 15);
+        mn = half_bits_to_float(dm >> 16) * (float)(p[t] >> 4);
+        return (load16(p + 16 + 32 * (t >> 3) + 16 * (k & 1)) >> (2 * (k >> 1))) & 0x03030303u;
     }
     template <int J, int ODD>
     static __device__ __forceinline__ half2v pair(uint32_t w, half2v sc, half2v off, uint32_t top) {
@@ -728,6 +819,17 @@ struct FmtQ3K {
         for (int o = 0; o < 2; o++) r.hm[o] = lds_u32x2(p + 16 * o + 8 * kh);
         r.sd = lds_u32x4(p + 96);
     }
+    // run t: 16 columns from 16 t on as bytes q + kBias, their scale and min
+    static constexpr int kBias = 4;
+    static constexpr bool kMin = false;
+    static __device__ __forceinline__ u32x4 run(const uint8_t *p, int t, float &sc, float &mn) {
+        const int h = t >> 3, j = (t >> 1) & 3, rr = t & 1;
+        const int lo4 = (p[96 + (t & 7)] >> (4 * h)) & 15, hi2 = (p[104 + (t & 3)] >> (2 * (t >> 2))) & 3;
+        sc = half_bits_to_float(*reinterpret_cast<const uint16_t *>(p + 108)) * (float)((lo4 | (hi2 << 4)) - 32);
+        mn = 0.f;
+        return ((load16(p + 32 + 32 * h + 16 * rr) >> (2 * j)) & 0x03030303u) |
+               (((load16(p + 16 * rr) >> (4 * h + j)) & 0x01010101u) << 2);
+    }
     template <bool HL, int NT, bool TWO, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1028.f);  // 1024 + 4
@@ -763,6 +865,101 @@ struct FmtQ3K {
         fold_columns<HL, NT>(c, part, tot);
     }
 };
+
+// The columns (bits of a mask) of which a block was left out (see split_x)
+template <bool HL, int NT, class C>
+__device__ __forceinline__ uint64_t marked_columns(const C &c) {
+    const uint64_t b = __builtin_amdgcn_ballot_w64(c.cs()[threadIdx.x & (HL ? 15 : 32 * NT - 1)] < 0.f);
+    return HL ? b & 0xFFFF : NT == 1 ? b & 0xFFFFFFFFu : b;
+}
+// tot += the fp32 products of the blocks that were left out, with x itself and folded
+// like those of the fp32 kernels (scale * sum(q x) - min * sum(x)), so that infinities
+// and NaN come out as there.  x is the columns' first super-block of the walk, p the
+// lane's row there; half kh of a row's lanes takes 128 columns of a block.  Four
+// columns at a time share the weights' decode and have their loads in flight
+// together: with an outlier in every block of every vector, us, one column at a time /
+// four (two vectors: two and four runs) / the fp32 kernels, 14336 x 4096 Q4_K at B = 128
+// 2540 / 1345 / 1998, 4096 x 14336 Q6_K 4340 / 1760 / 1440, 9216 x 3072 Q8_0 at B = 2 48 /
+// 37 / 25.
+template <class F, int NT, int NI>
+__device__ __forceinline__ void add_exact(uint64_t cols, const uint8_t *p, const float *x, size_t ldx, int nsb, int kh,
+                                          float (&tot)[NT][NI]) {
+    constexpr int K = NI == 8 ? 2 : 4, kUnroll = NI == 8 ? 4 : 1;  // (HL: two vectors)
+    while (cols) {
+        int b[K];
+        uint32_t off[K];
+#pragma unroll
+        for (int c = 0; c < K; c++) {
+            b[c] = cols ? __builtin_ctzll(cols) : -1;
+            off[c] = (uint32_t)(b[c] < 0 ? b[0] : b[c]);
+            cols &= cols - 1;  // (0 stays 0)
+        }
+        float acc[K] = {};
+#pragma unroll 1
+        for (int sb = 0; sb < nsb; sb++) {
+            const float *xb[K];
+            float4 v[K];
+#pragma unroll
+            for (int c = 0; c < K; c++) {
+                xb[c] = x + off[c] * ldx + 256 * sb;
+                v[c] = load_f4(xb[c] + 4 * (threadIdx.x & 63));
+            }
+            bool bad[K], any = false;
+#pragma unroll
+            for (int c = 0; c < K; c++) {
+                const float e[4] = {fabsf(v[c].x), fabsf(v[c].y), fabsf(v[c].z), fabsf(v[c].w)};
+                const float four = larger(larger(e[0], e[1]), larger(e[2], e[3]));
+                float lone = INFINITY, m = row16_max(four);
+#pragma unroll
+                for (int i = 0; i < 4; i++) lone = e[i] != 0.f ? fminf(lone, e[i]) : lone;
+                m = larger(m, __shfl_xor(m, 16));
+                m = larger(m, __shfl_xor(m, 32));
+                bad[c] = __builtin_amdgcn_ballot_w64(unfit(m, lone, four != 0.f ? four : INFINITY)) != 0;
+                any |= bad[c];
+            }
+            if (!any) continue;
+            float s[K] = {};
+#pragma unroll kUnroll
+            for (int t = 8 * kh; t < 8 * kh + 8; t++) {
+                float sc, mn;
+                const u32x4 q = F::run(p + (size_t)sb * F::kBytes, t, sc, mn);
+                float4 u[K][4];
+#pragma unroll
+                for (int c = 0; c < K; c++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) u[c][i] = load_f4(xb[c] + 16 * t + 4 * i);
+                float dot[K] = {}, sum[K] = {};
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float w = (float)((int)byte_of(q[i], j) - F::kBias);
+#pragma unroll
+                        for (int c = 0; c < K; c++) {
+                            const float e = j == 0 ? u[c][i].x : j == 1 ? u[c][i].y : j == 2 ? u[c][i].z : u[c][i].w;
+                            dot[c] = fmaf(w, e, dot[c]);
+                            sum[c] += e;
+                        }
+                    }
+#pragma unroll
+                for (int c = 0; c < K; c++) {
+                    s[c] = fmaf(sc, dot[c], s[c]);
+                    if (F::kMin) s[c] = fmaf(-mn, sum[c], s[c]);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < K; c++) acc[c] = bad[c] ? acc[c] + s[c] : acc[c];
+        }
+#pragma unroll
+        for (int c = 0; c < K; c++) {
+            acc[c] += __shfl_xor(acc[c], 32);
+#pragma unroll
+            for (int n = 0; n < NT; n++)
+#pragma unroll
+                for (int i = 0; i < NI; i++) tot[n][i] = batch_of(n, i, kh) == b[c] ? tot[n][i] + acc[c] : tot[n][i];
+        }
+    }
+}
 
 // A wave's 32 weight rows (past the end: the last row again): a wave-uniform
 // 16-byte-aligned base and 32-bit offsets from it, which cost a lane half the
@@ -1008,7 +1205,8 @@ __device__ __forceinline__ void store_pair(const float (&tot)[1][NI], int r, int
 // One workgroup's tile (32 rows per wave x all batch columns) over the K
 // range of its split, x converted into LDS super-block by super-block.
 // WIDE: column chunk `chunk` of g.chunks (32 NT columns each); TWO: see kTwo.
-template <class F, bool HL, int NT, bool PAIR, bool WIDE>  // NT: column groups of 32 (HL: one of 16)
+// EXACT: see split_x.  NT: column groups of 32 (HL: one of 16)
+template <class F, bool HL, int NT, bool PAIR, bool WIDE, bool EXACT>
 __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int chunk, int split, const MfmaGroup &g, uint8_t *lds) {
     constexpr bool TWO = kTwo<WIDE, NT>;
     const int chunks = WIDE ? g.chunks : 1, col0 = WIDE ? chunk * 32 * NT : 0;
@@ -1073,6 +1271,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
                 *reinterpret_cast<u32x4 *>(wslot + 16 * win_chunk<CH, RC>(lane + 64 * k)) = ch_n[k];       \
     } while (0)
 
+    uint64_t marked = 0;  // columns with blocks left to add_exact
     float tot[NT][NI], tot2[NI];
     if constexpr (TWO) {
 #pragma unroll
@@ -1096,7 +1295,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
         if (sb0 < sb1) {
             if (stager) JH_LOAD_X(sb0);
             JH_LOAD_W(sb0);
-            if (stager) I::template store<F::kSums>(lds, xv_n[0], xq, xcol);
+            if (stager) I::template store<F::kSums, EXACT>(lds, xv_n[0], xq, xcol);
             if (stager && sb0 + 1 < sb1) JH_LOAD_X(sb0 + 1);
         }
         for (int sb = sb0; sb < sb1; sb++) {
@@ -1109,13 +1308,15 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
             F::load(w, wslot + lr * RC * 16 + ((myoff + (uint32_t)sb * F::kBytes) & 15), kh);
             if (sb + 1 < sb1) {
                 if (stager) {
-                    I::template store<F::kSums>(lds + (buf ^ 1) * I::kBytes, xv_n[0], xq, xcol);
+                    I::template store<F::kSums, EXACT>(lds + (buf ^ 1) * I::kBytes, xv_n[0], xq, xcol);
                     if (sb + 2 < sb1) JH_LOAD_X(sb + 2);
                 }
                 JH_LOAD_W(sb + 1);
             }
             JH_MT(3 + 4 * (sb - sb0));
-            F::template compute<HL, NT, TWO>(w, Ctx<HL, NT>{lr, kh, lds + buf * I::kBytes}, tot);
+            const Ctx<HL, NT> c{lr, kh, lds + buf * I::kBytes};
+            if constexpr (EXACT) marked |= marked_columns<HL, NT>(c);
+            F::template compute<HL, NT, TWO>(w, c, tot);
             if constexpr (TWO) {
 #pragma unroll
                 for (int i = 0; i < NI; i++) {
@@ -1134,7 +1335,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
         for (int sb = sb0; sb < sb1; sb++) {
             __syncthreads();  // the previous super-block's LDS contents are consumed
 #pragma unroll
-            for (int i = 0; i < NT; i++) I::template store<F::kSums>(lds, xv_n[i], xq, xcol + 32 * i);
+            for (int i = 0; i < NT; i++) I::template store<F::kSums, EXACT>(lds, xv_n[i], xq, xcol + 32 * i);
             JH_PARK();
             // this lane's row block inside its staged window (same wave: no barrier)
             typename F::Regs w;
@@ -1145,13 +1346,19 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
             JH_LOAD_X(min(sb + 1, sb1 - 1));
             JH_LOAD_W(min(sb + 1, sb1 - 1));
             __syncthreads();
-            F::template compute<HL, NT, TWO>(w, Ctx<HL, NT>{lr, kh, lds}, tot);
+            const Ctx<HL, NT> c{lr, kh, lds};
+            if constexpr (EXACT) marked |= marked_columns<HL, NT>(c);
+            F::template compute<HL, NT, TWO>(w, c, tot);
         }
     }
 #undef JH_LOAD_X
 #undef JH_LOAD_W
 #undef JH_PARK
 
+    if constexpr (EXACT) {
+        if (__builtin_expect(marked != 0, 0))
+            add_exact<F>(marked, W + myoff + (size_t)sb0 * F::kBytes, X + 256 * sb0, cols, sb1 - sb0, kh, tot);
+    }
     if constexpr (PAIR) {
         store_pair(tot, rbase + lr, (wave & (kWaves / 2 - 1)) * kRowsPerWave + lr, up_half, nrows, kh, B,
                    g.swiglu, g.part, g.counters, tile, split, g.ksplit, lds);
@@ -1167,7 +1374,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
 
 // A group of matrices with the same K in one launch (1-D grid): each
 // workgroup finds its matrix and runs that matrix's format.
-template <bool HL, int NT, int MASK, bool PAIR = false, bool WIDE = false>
+template <bool HL, int NT, int MASK, bool PAIR = false, bool WIDE = false, bool EXACT = WIDE>
 __global__ __launch_bounds__(kThreads) void mfma_group(MfmaGroup g) {
     __shared__ __align__(16) uint8_t lds[lds_bytes<HL, NT, MASK>()];
     const int id = blockIdx.x;
@@ -1178,17 +1385,17 @@ __global__ __launch_bounds__(kThreads) void mfma_group(MfmaGroup g) {
     const int local = id - P.wg0, at = local / g.ksplit, split = local - at * g.ksplit;
     const int tile = WIDE ? at / g.chunks : at, chunk = WIDE ? at - tile * g.chunks : 0;
     switch (P.type) {
-        case 12: if constexpr ((MASK & 1) != 0) gemm_body<FmtQ4K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
-        case 13: if constexpr ((MASK & 2) != 0) gemm_body<FmtQ5K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
-        case 14: if constexpr ((MASK & 4) != 0) gemm_body<FmtQ6K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
-        case 10: if constexpr ((MASK & 16) != 0) gemm_body<FmtQ2K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
-        case 11: if constexpr ((MASK & 32) != 0) gemm_body<FmtQ3K, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
-        default: if constexpr ((MASK & 8) != 0) gemm_body<FmtQ8_0, HL, NT, PAIR, WIDE>(P, tile, chunk, split, g, lds); break;
+        case 12: if constexpr ((MASK & 1) != 0) gemm_body<FmtQ4K, HL, NT, PAIR, WIDE, EXACT>(P, tile, chunk, split, g, lds); break;
+        case 13: if constexpr ((MASK & 2) != 0) gemm_body<FmtQ5K, HL, NT, PAIR, WIDE, EXACT>(P, tile, chunk, split, g, lds); break;
+        case 14: if constexpr ((MASK & 4) != 0) gemm_body<FmtQ6K, HL, NT, PAIR, WIDE, EXACT>(P, tile, chunk, split, g, lds); break;
+        case 10: if constexpr ((MASK & 16) != 0) gemm_body<FmtQ2K, HL, NT, PAIR, WIDE, EXACT>(P, tile, chunk, split, g, lds); break;
+        case 11: if constexpr ((MASK & 32) != 0) gemm_body<FmtQ3K, HL, NT, PAIR, WIDE, EXACT>(P, tile, chunk, split, g, lds); break;
+        default: if constexpr ((MASK & 8) != 0) gemm_body<FmtQ8_0, HL, NT, PAIR, WIDE, EXACT>(P, tile, chunk, split, g, lds); break;
     }
 }
 
 // one workgroup per super-block: 32 (HL: 16) columns x 16 lanes (columns >= B are zero)
-template <bool HL>
+template <bool HL, bool EXACT>
 __global__ __launch_bounds__(HL ? 256 : 512) void x_prep(const float *__restrict__ X, int B, int cols, uint8_t *__restrict__ slabs) {
     const int sb = blockIdx.x, q = threadIdx.x & 15, col = threadIdx.x >> 4;
     float xv[16];
@@ -1201,7 +1408,7 @@ __global__ __launch_bounds__(HL ? 256 : 512) void x_prep(const float *__restrict
         xv[4 * k + 2] = v.z;
         xv[4 * k + 3] = v.w;
     }
-    Slab<HL>::store(slabs + (size_t)sb * Slab<HL>::kBytes, xv, q, col);
+    Slab<HL>::template store<EXACT>(slabs + (size_t)sb * Slab<HL>::kBytes, xv, q, col);
 }
 
 // The B <= 32 kernel on prepared x, for matrices with enough row tiles to
@@ -1220,10 +1427,10 @@ __global__ __launch_bounds__(HL ? 256 : 512) void x_prep(const float *__restrict
 // Loads are issued unconditionally (addresses clamped to the last super-block
 // of the range) so that every wave's count of memory operations in flight is
 // the same static number at each wait.
-template <class F, bool HL>
+template <class F, bool HL, bool EXACT>
 __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pitch, int row0, int nrows,
                                                     int nsb, const uint8_t *__restrict__ slabs,
-                                                    float *__restrict__ Y, int B) {
+                                                    const float *__restrict__ X, float *__restrict__ Y, int B) {
     constexpr int CH = F::kChunks;
     constexpr int CL = (kRowsPerWave * CH + 63) / 64;
     using I = Slab<HL>;
@@ -1272,6 +1479,7 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
             SET[k] = *reinterpret_cast<const u32x4 *>(W + ((coff[k] + sbo) & ~15u));                \
     } while (0)
 
+    uint64_t marked = 0;
     float tot[1][kOut<HL>] = {};
 #define JH_STEP(SET, SB, BUF)                                                                              \
     do {                                                                                                   \
@@ -1285,7 +1493,9 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
         typename F::Regs w;                                                                                \
         F::load(w, wslot + lr * RC * 16 + ((myoff + (uint32_t)(SB) * F::kBytes) & 15), kh);  \
         JH_LOAD_W(SET, (SB) + 2);                                                                          \
-        F::template compute<HL, 1, false>(w, CtxP<HL>{lr, kh, sh_x[BUF]}, tot);                            \
+        const CtxP<HL> c{lr, kh, sh_x[BUF]};                                                               \
+        if constexpr (EXACT) marked |= marked_columns<HL, 1>(c);                                           \
+        F::template compute<HL, 1, false>(w, c, tot);                                                      \
     } while (0)
 
     dma_x(sb0, 0);
@@ -1301,6 +1511,9 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
 #undef JH_STEP
 #undef JH_LOAD_W
 
+    if constexpr (EXACT) {
+        if (__builtin_expect(marked != 0, 0)) add_exact<F>(marked, W + myoff, X, (size_t)256 * nsb, nsb, kh, tot);
+    }
     store_tile(tot, rbase + lr, nrows, kh, B, Y, nullptr, 0, nullptr, blockIdx.x, 0, 1);
 }
 
@@ -1442,6 +1655,15 @@ static void launch_group_nt(const MfmaGroup &g, int mask, int grid, hipStream_t 
     }
 }
 
+static void launch_two(const MfmaGroup &g, int mask, int grid, hipStream_t s) {
+    switch (mask) {
+        case 1: mfma_group<true, 1, 1, false, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 2: mfma_group<true, 1, 2, false, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 8: mfma_group<true, 1, 8, false, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        default: mfma_group<true, 1, 11, false, false, true><<<grid, kThreads, 0, s>>>(g); break;
+    }
+}
+
 // JUNO_MFMA_PAIR=0: the batched SwiGLU takes the grouped launch and silu_mul (A/B runs)
 static bool mfma_pair_wanted() {
     static const bool on = [] {
@@ -1502,13 +1724,14 @@ hipError_t launch_mfma_swiglu(const MfmaDesc &gate, const MfmaDesc &up, int B, f
     q.wg0 = q.cnt0 = 0;
     q.part0 = 0;
     const int grid = q.tiles * p.ksplit;
-    const bool hl = B <= kHlMaxBatch;
-#define JH_PAIR(M) \
-    (hl ? mfma_group<true, 1, M, true><<<grid, kThreads, 0, s>>>(g) : mfma_group<false, 1, M, true><<<grid, kThreads, 0, s>>>(g))
+    auto run = [&](auto *k) { k<<<grid, kThreads, 0, s>>>(g); };
+#define JH_PAIR(M)                                                                                    \
+    (B == 2 ? run(mfma_group<true, 1, M, true, false, true>)                                          \
+            : B <= kHlMaxBatch ? run(mfma_group<true, 1, M, true>) : run(mfma_group<false, 1, M, true>))
     switch (gate.type) {
         case 12: JH_PAIR(1); break;
         case 13: JH_PAIR(2); break;
-        case 14: JH_PAIR(4); break;
+        case 14: B <= kHlMaxBatch ? run(mfma_group<true, 1, 4, true>) : run(mfma_group<false, 1, 4, true>); break;  // not two
         default: JH_PAIR(8); break;
     }
 #undef JH_PAIR
@@ -1565,15 +1788,16 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
         const MfmaDesc &m = d[0];
         const int nrows = m.row_end - m.row_start;
         const bool hl = B <= kHlMaxBatch;
-        if (hl) x_prep<true><<<p.nsb, 256, 0, s>>>(m.x, B, m.cols, ws);
-        else x_prep<false><<<p.nsb, 512, 0, s>>>(m.x, B, m.cols, ws);
-#define JH_PX(F)                                                                                                          \
-    (hl ? mfma_px<F, true><<<p.grid, kThreads, 0, s>>>(m.w, m.pitch, m.row_start, nrows, p.nsb, ws, m.y, B)              \
-        : mfma_px<F, false><<<p.grid, kThreads, 0, s>>>(m.w, m.pitch, m.row_start, nrows, p.nsb, ws, m.y, B))
+        if (B == 2) x_prep<true, true><<<p.nsb, 256, 0, s>>>(m.x, B, m.cols, ws);
+        else if (hl) x_prep<true, false><<<p.nsb, 256, 0, s>>>(m.x, B, m.cols, ws);
+        else x_prep<false, false><<<p.nsb, 512, 0, s>>>(m.x, B, m.cols, ws);
+        auto px = [&](auto *k) { k<<<p.grid, kThreads, 0, s>>>(m.w, m.pitch, m.row_start, nrows, p.nsb, ws, m.x, m.y, B); };
+#define JH_PX(F) (B == 2 ? px(mfma_px<F, true, true>) : hl ? px(mfma_px<F, true, false>) : px(mfma_px<F, false, false>))
         if (m.type == 12) JH_PX(FmtQ4K);
         else if (m.type == 13) JH_PX(FmtQ5K);
-        else if (m.type == 14) JH_PX(FmtQ6K);
-        else JH_PX(FmtQ8_0);
+        else if (m.type == 8) JH_PX(FmtQ8_0);
+        else if (hl) px(mfma_px<FmtQ6K, true, false>);  // not with two vectors
+        else px(mfma_px<FmtQ6K, false, false>);
 #undef JH_PX
         return hipGetLastError();
     }
@@ -1608,6 +1832,7 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
     g.chunks = p.chunks;
     if (B > 64 && p.chunk == 64) launch_wide<2>(g, mask, p.grid, s);
     else if (B > 64) launch_wide<1>(g, mask, p.grid, s);
+    else if (B == 2) launch_two(g, mask, p.grid, s);
     else if (B <= kHlMaxBatch) launch_group_nt<true, 1>(g, mask, p.grid, s);
     else if (B <= 32) launch_group_nt<false, 1>(g, mask, p.grid, s);
     else launch_group_nt<false, 2>(g, mask, p.grid, s);
