@@ -38,7 +38,8 @@
  *     grows is replaced, never freed, so graphs captured earlier stay valid.
  *     A captured graph uses its stream's workspace: do not replay it while
  *     other work on that workspace (the same stream's calls or another replay)
- *     is running on another stream.
+ *     is running on another stream.  hipStreamPerThread has a workspace per
+ *     thread; other handles that several threads use name one stream.
  */
 #ifndef JUNOHIP_H
 #define JUNOHIP_H

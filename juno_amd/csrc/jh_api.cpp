@@ -21,6 +21,8 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <tuple>
+#include <vector>
 
 #include "jh_kernels.hpp"
 
@@ -215,13 +217,58 @@ int gemv_path();
 // A graph shares its stream's workspace: replaying it on another stream while
 // work that uses the same workspace runs is a race, like any two overlapping
 // launches on one buffer.
+//
+// hipStreamPerThread is one handle for as many streams as there are threads, so
+// its workspaces are one per thread too (WsKey::thread).  They outlive the thread
+// only as spares: the next thread that needs one takes a spare instead of
+// allocating, after a wait for the device (the ended thread's last launches may
+// still run), so that they number at most the threads alive at one time.  One that
+// a graph capture has used is no spare: the graph may be replayed.
 struct Workspace {
     uint8_t *base = nullptr;  // counters, then scratch
     size_t cap = 0;           // scratch bytes
+    bool captured = false;    // (thread workspaces only)
 };
 constexpr size_t kCounterBytes = sizeof(int) * (size_t)jh::kCounterSlots * jh::kCounterStride;
-std::mutex g_ws_mu;
-std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
+typedef std::tuple<int, hipStream_t, uint64_t> WsKey;  // device, handle, thread (0: any)
+// Never destroyed: a thread may end after this library's static destructors have run.
+struct WorkspacePool {
+    std::mutex mu;
+    std::map<WsKey, Workspace> used;
+    std::vector<std::pair<int, Workspace>> spare;  // device, workspace
+    uint64_t threads = 0;
+    void retire(int device, const Workspace &w) {
+        if (w.base && !w.captured) spare.emplace_back(device, w);
+    }
+};
+WorkspacePool &ws_pool() {
+    static WorkspacePool *p = new WorkspacePool;
+    return *p;
+}
+
+struct ThreadWorkspaces {
+    uint64_t id = 0;  // from 1 on, never given twice
+    ~ThreadWorkspaces() {
+        if (!id) return;
+        WorkspacePool &pool = ws_pool();
+        std::lock_guard<std::mutex> lk(pool.mu);
+        for (auto it = pool.used.begin(); it != pool.used.end();)
+            if (std::get<2>(it->first) == id) {
+                pool.retire(std::get<0>(it->first), it->second);
+                it = pool.used.erase(it);
+            } else {
+                ++it;
+            }
+    }
+};
+thread_local ThreadWorkspaces t_workspaces;
+
+// pool.mu held
+WsKey ws_key(WorkspacePool &pool, int device, hipStream_t s) {
+    if (s != hipStreamPerThread) return {device, s, 0};
+    if (!t_workspaces.id) t_workspaces.id = ++pool.threads;
+    return {device, s, t_workspaces.id};
+}
 
 int stream_is_capturing(hipStream_t s, bool *capturing) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -232,12 +279,16 @@ int stream_is_capturing(hipStream_t s, bool *capturing) {
 
 // Scratch of at least `bytes` and the split-K counters of stream s on `device`.
 int stream_workspace(int device, hipStream_t s, size_t bytes, void **out, int **counters = nullptr) {
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    Workspace &e = g_ws[{device, s}];
+    WorkspacePool &pool = ws_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    const WsKey key = ws_key(pool, device, s);
+    const bool of_thread = std::get<2>(key) != 0;
+    Workspace &e = pool.used[key];
+    bool capturing = false;
+    int rc;
+    if (of_thread || !e.base || e.cap < bytes)
+        if ((rc = stream_is_capturing(s, &capturing))) return rc;
     if (!e.base || e.cap < bytes) {
-        bool capturing = false;
-        int rc = stream_is_capturing(s, &capturing);
-        if (rc) return rc;
         if (capturing)
             return fail(JH_EINVAL,
                         "device workspace of %zu bytes needed during graph capture (stream has %zu): make one eager "
@@ -245,17 +296,31 @@ int stream_workspace(int device, hipStream_t s, size_t bytes, void **out, int **
                         bytes, e.cap);
         size_t want = bytes < (8u << 20) ? (8u << 20) : bytes;
         if (e.base && want < 2 * e.cap) want = 2 * e.cap;
-        void *p = nullptr;
-        if ((rc = device_alloc(&p, kCounterBytes + want))) return rc;
-        hipError_t me = hipMemsetAsync(p, 0, kCounterBytes, s);
-        if (me != hipSuccess) {
-            (void)hipFree(p);  // never handed out
-            return hip_fail("hipMemsetAsync(split-K counters)", me);
+        Workspace w;
+        if (of_thread)
+            for (auto it = pool.spare.begin(); it != pool.spare.end(); ++it)
+                if (it->first == device && it->second.cap >= bytes) {
+                    JH_HIP("hipDeviceSynchronize(workspace)", hipDeviceSynchronize());  // its last user is done, its counters are 0
+                    w = it->second;
+                    pool.spare.erase(it);
+                    break;
+                }
+        if (!w.base) {
+            void *p = nullptr;
+            if ((rc = device_alloc(&p, kCounterBytes + want))) return rc;
+            hipError_t me = hipMemsetAsync(p, 0, kCounterBytes, s);
+            if (me != hipSuccess) {
+                (void)hipFree(p);  // never handed out
+                return hip_fail("hipMemsetAsync(split-K counters)", me);
+            }
+            w.base = static_cast<uint8_t *>(p);
+            w.cap = want;
         }
         // the previous buffer (if any) is retired, not freed: see above
-        e.base = static_cast<uint8_t *>(p);
-        e.cap = want;
+        if (of_thread) pool.retire(device, e);
+        e = w;
     }
+    if (of_thread && capturing) e.captured = true;
     *out = e.base + kCounterBytes;
     if (counters) *counters = reinterpret_cast<int *>(e.base);
     return JH_OK;
@@ -381,10 +446,11 @@ int jh_qmatvec_batched_plan(int n, const jh_qmat *const *mats, int B, int *kerne
 
 int jh_stream_workspace_info(int device, void *stream, size_t *scratch_bytes, void **base) {
     if (!scratch_bytes || !base) return fail(JH_EINVAL, "scratch_bytes and base must not be null");
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    auto it = g_ws.find({device, (hipStream_t)stream});
-    *scratch_bytes = it == g_ws.end() ? 0 : it->second.cap;
-    *base = it == g_ws.end() ? nullptr : it->second.base;
+    WorkspacePool &pool = ws_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    auto it = pool.used.find(ws_key(pool, device, (hipStream_t)stream));
+    *scratch_bytes = it == pool.used.end() ? 0 : it->second.cap;
+    *base = it == pool.used.end() ? nullptr : it->second.base;
     return ok();
 }
 
