@@ -115,6 +115,7 @@ constexpr int kMaxMfmaGroup = 4;
 // or 1 columns.  8B GEMV step: B = 3 5.54 ms on the VALU kernels, 3.80 ms here; B = 8
 // 15.4 and 3.88 ms.  Two columns take it where plan_group's rule says so.
 constexpr int kMfmaMinBatch = 3;
+// More than 64 vectors are also launched with a null workspace: K is then not split.
 size_t mfma_group_workspace_bytes(int n, const MfmaDesc *d, int B);
 hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, int *counters, hipStream_t s);
 // Which kernel launch_mfma_group takes: 0 none (the path does not apply),

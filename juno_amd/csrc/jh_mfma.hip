@@ -1782,6 +1782,12 @@ hipError_t static_scratch(int device, hipStream_t s, void **workspace, int **cou
 hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, int *counters, hipStream_t s) {
     Plan p;
     if (!plan_group(n, d, B, p)) return hipErrorNotSupported;
+    if (!workspace && B <= 64) return hipErrorNotSupported;
+    if (!workspace) {  // K whole
+        p.grid /= p.ksplit;
+        p.ksplit = 1;
+        p.ksb = p.nsb;
+    }
     if (p.ksplit > 1 && !counters) return hipErrorNotSupported;
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);
     if (p.prepared) {
