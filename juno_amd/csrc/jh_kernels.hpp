@@ -113,7 +113,7 @@ constexpr int kMaxMfmaGroup = 4;
 // From this batch on every shape the path supports takes it: its fixed costs are
 // those of up to 16 columns, while the VALU kernels read the weights once per 8, 4, 2
 // or 1 columns.  8B GEMV step: B = 3 5.54 ms on the VALU kernels, 3.80 ms here; B = 8
-// 15.4 and 3.88 ms.  Two columns take it where plan_group's rule says so.
+// 15.4 and 3.88 ms.  Two columns take it where two_vectors_pay says so.
 constexpr int kMfmaMinBatch = 3;
 // More than 64 vectors are also launched with a null workspace: K is then not split.
 size_t mfma_group_workspace_bytes(int n, const MfmaDesc *d, int B);

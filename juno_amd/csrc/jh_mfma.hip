@@ -1543,8 +1543,35 @@ struct Plan {
 };
 }  // namespace
 
-// Row tiles of 256 rows; K split the same way for every matrix of the group.
-static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p) {
+// Two vectors: where this path's fixed 9 to 12 us (15 to 20 from K = 8192 on) are less
+// than the fp32 kernels take.  Those read the weights once, bound by their arithmetic,
+// in a launch per matrix (and one for silu * up); up to 2048 or 4096 rows all their
+// workgroups are resident at once, evenly over the CUs, and their time is that of a
+// row.  us, fp32 / here:
+//   one matrix, Q4_K   6144 x 4096 10.3 / 10.9, 6656 x 4096 12.7 / 11.0, 9216 x 3072 13.8 / 11.9,
+//                      4096 x 8192 12.1 / 14.2, 2048 x 14336 12.3 / 16.3, 2560 x 14336 19.0 / 16.5
+//               Q5_K   6144 x 4096 11.7 / 12.7, 6656 x 4096 13.8 / 12.5, 4096 x 8192 14.6 / 16.1,
+//                      2560 x 14336 22.4 / 18.9
+//               Q8_0   10240 x 2048 12.9 / 13.3, 11008 x 2048 14.9 / 13.4, 5632 x 4096 15.6 / 14.2,
+//                      4096 x 8192 20.0 / 17.5, 2048 x 14336 18.0 / 20.5, 2304 x 14336 31.6 / 20.7
+//   a group of two     2048 x 2048 Q4_K 7.8 / 9.7, Q8_0 9.3 / 12.1; 2048 x 3072 10.9 / 10.4, 12.1 / 12.9;
+//                      1792 x 4096 13.1 / 10.6, 19.3 / 13.1; 4096 x 2048 10.5 / 9.9, 13.5 / 12.7
+//   a SwiGLU pair      2048 x 2048 Q4_K 9.9 / 9.8, Q8_0 11.3 / 12.5; 2560 x 2048 12.0 / 10.1, 15.2 / 12.6;
+//                      5632 x 2048 14.8 / 10.6, 19.4 / 14.2
+// Only formats whose error against 64 bits is smaller here (K = 512 .. 28672: Q4_K
+// 2.4-2.9e-7 / 1.8-2.0e-7, Q5_K 2.4-2.9e-7 / 1.8-2.0e-7, Q8_0 1.20-1.41e-7 / 0.81-1.25e-7);
+// that of Q6_K and Q3_K is not, and Q2_K is not taken either.
+static bool two_vectors_pay(int n, bool pair, int type, size_t rows, int cols) {
+    const double weights = (double)rows * cols;
+    if (pair) return weights >= 10e6;
+    if (n > 1) return weights >= 14e6;
+    if (type == 8) return weights >= (rows > 2048 ? 22e6 : 36e6);
+    return weights >= (rows > 4096 ? 26e6 : 36e6);
+}
+
+// Row tiles of 256 rows; K split the same way for every matrix of the group.  pair:
+// d[0] is a SwiGLU pair's virtual matrix, gate's rows and then up's.
+static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p, bool pair = false) {
     if (n < 1 || n > kMaxMfmaGroup) return false;
     int tiles = 0;
     size_t rows = 0;
@@ -1556,13 +1583,7 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p) {
         rows += d[i].row_end - d[i].row_start;
         if (B == 2 && d[i].type != 12 && d[i].type != 13 && d[i].type != 8) return false;
     }
-    // Two vectors: from 26 M weights on, in a group (a launch each otherwise) from 20 M,
-    // where the VALU kernels' arithmetic outweighs this path's fixed 9 us.  us, VALU / MFMA:
-    // 6144 x 4096 Q4_K 10.4 / 11.0, 9216 x 3072 13.8 / 11.6 and Q8_0 20.7 / 14.6, 2 x 2816 x
-    // 2048 10.2 / 9.5 (Q5_K 11.1 / 10.9, Q8_0 13.1 / 12.1), 2 x 5632 x 2048 12.7 / 9.9.
-    // Q4_K, Q5_K and Q8_0, whose error against 64 bits is smaller here (K = 4096: Q4_K
-    // 2.5e-7 / 1.8e-7, Q8_0 1.33e-7 / 1.0e-7); that of Q6_K and Q3_K is not.
-    if (B == 2 && (double)rows * d[0].cols < (n == 1 ? 26e6 : 20e6)) return false;
+    if (B == 2 && !two_vectors_pay(n, pair, d[0].type, rows, d[0].cols)) return false;
     p.nsb = d[0].cols / 256;
     // One workgroup fits per CU (LDS, VGPRs), so the grid runs in rounds of
     // kMinWorkgroups.  Cost of a split, in super-block steps: rounds x (super-
@@ -1683,14 +1704,14 @@ bool mfma_swiglu_applies(const MfmaDesc &gate, const MfmaDesc &up, int B) {
     MfmaDesc v = gate;
     v.row_end = 2 * gate.row_end;  // the pair's virtual rows: same tiles and K split as one matrix of 2 x rows
     Plan p;
-    return plan_group(1, &v, B, p) && (p.ksplit == 1 || (gate.row_end + kRowsPerWG / 2 - 1) / (kRowsPerWG / 2) <= kMaxTileCounters);
+    return plan_group(1, &v, B, p, true) && (p.ksplit == 1 || (gate.row_end + kRowsPerWG / 2 - 1) / (kRowsPerWG / 2) <= kMaxTileCounters);
 }
 
 size_t mfma_swiglu_workspace_bytes(const MfmaDesc &gate, int B) {
     MfmaDesc v = gate;
     v.row_end = 2 * gate.row_end;
     Plan p;
-    if (!plan_group(1, &v, B, p)) return 0;
+    if (!plan_group(1, &v, B, p, true)) return 0;
     return p.ksplit > 1 ? sizeof(float) * (size_t)p.ksplit * B * v.row_end : 16;
 }
 
@@ -1700,7 +1721,7 @@ hipError_t launch_mfma_swiglu(const MfmaDesc &gate, const MfmaDesc &up, int B, f
     MfmaDesc v = gate;
     v.row_end = 2 * gate.row_end;
     Plan p;
-    plan_group(1, &v, B, p);
+    plan_group(1, &v, B, p, true);
     if (p.ksplit > 1 && !counters) return hipErrorNotSupported;
     MfmaGroup g = {};
     g.part = reinterpret_cast<float *>(workspace);

@@ -22,12 +22,17 @@ P = ctypes.c_void_p
 
 
 @pytest.mark.parametrize("captured", [False, True])
-@pytest.mark.parametrize("qtype,rows,cols,lo", [
-    (O.Q4_K, 6347, 4096, 0), (O.Q4_K, 6348, 4096, 0), (O.Q4_K, 1950, 14336, 37), (O.Q8_0, 8465, 3072, 0),
-    (O.Q8_0, 13000, 2080, 0), (O.Q5_K, 33100, 1024, 300), (O.Q6_K, 6500, 4096, 0)])
-def test_two_vectors(qtype, rows, cols, lo, captured):
+@pytest.mark.parametrize("qtype,rows,cols,lo,mfma", [
+    (O.Q4_K, 6347, 4096, 0, False), (O.Q4_K, 6348, 4096, 0, True), (O.Q4_K, 1950, 14336, 37, False),
+    (O.Q4_K, 2600, 14336, 37, True), (O.Q5_K, 4096, 8704, 0, False), (O.Q5_K, 4097, 8192, 0, True),
+    (O.Q8_0, 8465, 3072, 0, True), (O.Q8_0, 7161, 3072, 0, False), (O.Q8_0, 7162, 3072, 0, True),
+    (O.Q8_0, 13000, 2080, 0, False), (O.Q5_K, 33100, 1024, 300, True), (O.Q6_K, 6500, 4096, 0, False)])
+def test_two_vectors(qtype, rows, cols, lo, mfma, captured):
     import torch
     L = _lib.load()
+    kernel, ksplit = ctypes.c_int(), ctypes.c_int()
+    assert L.jh_qmatvec_batched_plan_shape(qtype, cols, lo, rows, 2, ctypes.byref(kernel), ctypes.byref(ksplit)) == 0
+    assert (kernel.value > 0) == mfma
     raw = weights(qtype, rows, cols, 3)
     X = np.random.default_rng(4).standard_normal((2, cols)).astype(np.float32)
     n = rows - lo
@@ -54,9 +59,9 @@ def test_two_vectors(qtype, rows, cols, lo, captured):
     check(y.cpu().numpy(), X, deq, (qtype, rows, cols, captured))
 
 
-@pytest.mark.parametrize("rows,cols", [(4096, 2560), (5120, 2560)])
+@pytest.mark.parametrize("rows,cols,fused", [(4096, 2560, True), (5120, 2560, True), (2441, 2048, False), (2442, 2048, True)])
 @pytest.mark.parametrize("captured", [False, True])
-def test_two_vector_swiglu(rows, cols, captured):
+def test_two_vector_swiglu(rows, cols, fused, captured):
     import torch
     L = _lib.load()
     raws = [weights(O.Q4_K, rows, cols, 8 + i) for i in range(2)]
@@ -84,6 +89,8 @@ def test_two_vector_swiglu(rows, cols, captured):
                     g.replay()
         st.synchronize()
         Y = out.cpu().numpy().astype(np.float64)
+        if not captured:  # the pair kernel leaves the scratch buffers alone
+            assert bool((a == 0).all() and (b == 0).all()) == fused
     dg, du = (O.dequantize(O.Q4_K, r, rows, cols).reshape(rows, cols).astype(np.float64) for r in raws)
     x64 = X.astype(np.float64)
     u, v = x64 @ dg.T, x64 @ du.T
@@ -93,3 +100,27 @@ def test_two_vector_swiglu(rows, cols, captured):
            for d in (dg, du)]
     bound = 1.1 * eps[0] * np.abs(v) + np.abs(silu) * eps[1] + 2 * eps[0] * eps[1] + 2.0 ** -20 * np.abs(silu * v)
     assert np.max(np.abs(Y - silu * v) / bound) <= 1.0
+
+
+@pytest.mark.parametrize("rows,mfma", [((3400, 17, 0), False), ((3400, 19, 0), True), ((1024, 1024, 1371), True)])
+def test_two_vector_group(rows, mfma):
+    """A group on either side of its limit (14 M weights), all members at the bar of one."""
+    import torch
+    L, cols = _lib.load(), 4096
+    rows = [r for r in rows if r]
+    raws = [weights(t, r, cols, 50 + i) for i, (t, r) in enumerate(zip((O.Q4_K, O.Q8_0, O.Q5_K), rows))]
+    devs = [upload(t, r, cols, w) for t, r, w in zip((O.Q4_K, O.Q8_0, O.Q5_K), rows, raws)]
+    n = len(devs)
+    hs = (P * n)(*[d.handle for d in devs])
+    kernel, ksplit = ctypes.c_int(), ctypes.c_int()
+    assert L.jh_qmatvec_batched_plan(n, hs, 2, ctypes.byref(kernel), ctypes.byref(ksplit)) == 0
+    assert (kernel.value > 0) == mfma
+    X = np.random.default_rng(51).standard_normal((2, cols)).astype(np.float32)
+    dx, ys = torch.from_numpy(X).cuda(), [torch.zeros(2, r, device="cuda") for r in rows]
+    torch.cuda.synchronize()
+    assert L.jh_qmatvec_batched_group_dev(n, hs, (P * n)(*[dx.data_ptr()] * n), 2, (P * n)(*[y.data_ptr() for y in ys]), None) == 0
+    torch.cuda.synchronize()
+    for t, r, w, y in zip((O.Q4_K, O.Q8_0, O.Q5_K), rows, raws, ys):
+        check(y.cpu().numpy(), X, O.dequantize(t, w, r, cols).reshape(r, cols).astype(np.float64), (t, r, mfma))
+    for d in devs:
+        d.close()
