@@ -181,10 +181,10 @@ __device__ __forceinline__ XColumn split_x(const float (&x_in)[16]) {
             r.h[u][i] = h;
             r.l[u][i] = (_Float16)fmaf(x, s, -(float)h);
         }
-    float g[4];
+    float g[4];  // of x s: sums of x itself pass the largest float from 2^123 on
 #pragma unroll
-    for (int i = 0; i < 4; i++) g[i] = (xv[4 * i] + xv[4 * i + 1]) + (xv[4 * i + 2] + xv[4 * i + 3]);
-    const float sub = ((g[0] + g[1]) + (g[2] + g[3])) * s;
+    for (int i = 0; i < 4; i++) g[i] = fmaf(xv[4 * i], s, xv[4 * i + 1] * s) + fmaf(xv[4 * i + 2], s, xv[4 * i + 3] * s);
+    const float sub = (g[0] + g[1]) + (g[2] + g[3]);
     r.s16 = ldexpf(sub, -kX16Shift);
     r.s32 = ldexpf(sub + dpp_f<0xB1>(sub), -kXsShift);  // this lane's and its neighbour's
     return r;
