@@ -181,7 +181,7 @@ __device__ __forceinline__ XColumn split_x(const float (&x_in)[16]) {
             r.h[u][i] = h;
             r.l[u][i] = (_Float16)fmaf(x, s, -(float)h);
         }
-    float g[4];  // of x s: sums of x itself pass the largest float from 2^123 on
+    float g[4];  // of x s: sums of x itself pass the largest float from 2^124 on
 #pragma unroll
     for (int i = 0; i < 4; i++) g[i] = fmaf(xv[4 * i], s, xv[4 * i + 1] * s) + fmaf(xv[4 * i + 2], s, xv[4 * i + 3] * s);
     const float sub = (g[0] + g[1]) + (g[2] + g[3]);

@@ -52,17 +52,17 @@ def test_limb_layouts(qtype, B, kind):
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("B", [3, 17, 33, 65])
 def test_sums_of_x_past_the_largest_float(qtype, B):
-    """x of one sign near 2^123: 32 of them together are past the largest float, the
+    """x of one sign from 2^124 on: 16 of them together are past the largest float, the
     results are not.  The bound is the other test's."""
-    rows, cols = 70, 512
+    rows, cols = 70, 256
     rng = np.random.default_rng(B * 100 + qtype)
     raw = random_blocks(qtype, rows, cols, B) if qtype in (O.Q2_K, O.Q3_K) else O.quantize(
         qtype, (rng.standard_normal(rows * cols) * 0.002 + 0.001).astype(np.float32))
     deq = O.dequantize(qtype, raw, rows, cols).astype(np.float64).reshape(rows, cols)
-    keep = np.abs(deq).sum(1) <= 12.0  # rows whose terms together stay below the largest float
+    keep = np.abs(deq).sum(1) <= 7.0  # rows whose terms together stay below the largest float
     assert keep.any() and (qtype in (O.Q2_K, O.Q3_K) or keep.all())
     deq[~keep] = 0.0
-    X = (np.ldexp(1.0 + rng.random((B, cols)), 123)).astype(np.float32)
+    X = (np.ldexp(1.0 + rng.random((B, cols)), 124)).astype(np.float32)
     be = mv.GpuContext.shared(0).create_mat_vec()
     with be.upload_quant(mv.QuantizedTensor("w", qtype, rows * cols, raw.tobytes()), rows, cols) as dev:
         Y = run(dev, X, rows).astype(np.float64)
