@@ -872,20 +872,34 @@ __device__ __forceinline__ uint64_t marked_columns(const C &c) {
     const uint64_t b = __builtin_amdgcn_ballot_w64(c.cs()[threadIdx.x & (HL ? 15 : 32 * NT - 1)] < 0.f);
     return HL ? b & 0xFFFF : NT == 1 ? b & 0xFFFFFFFFu : b;
 }
+
+// What a walk has met of them: the columns, and the super-blocks modulo 64.  Mostly that
+// is a block or two (activations that are products, silu * up, have one in 10^6
+// elements), so add_exact looks at the x of those super-blocks only, and one column at a
+// time has the loads of four runs in flight.  8B feed-forward at B = 128, us: all
+// super-blocks of the walk, four columns at a time 197-206; now 182, as without such
+// blocks.  With one outlier, 14336 x 4096 Q4_K 75.9 -> 61.6, 4096 x 14336 Q6_K 100 -> 83.
+struct Marks {
+    uint64_t cols = 0, blocks = 0;
+    __device__ __forceinline__ void add(uint64_t c, int sb) {
+        cols |= c;
+        blocks |= c ? 1ull << (sb & 63) : 0;
+    }
+};
+
 // tot += the fp32 products of the blocks that were left out, with x itself and folded
 // like those of the fp32 kernels (scale * sum(q x) - min * sum(x)), so that infinities
-// and NaN come out as there.  x is the columns' first super-block of the walk, p the
-// lane's row there; half kh of a row's lanes takes 128 columns of a block.  Four
-// columns at a time share the weights' decode and have their loads in flight
+// and NaN come out as there.  x and p are the columns' and the lane's row's super-block
+// 0; half kh of a row's lanes takes 128 columns of a block.  From three columns on four
+// at a time share the weights' decode and have their loads in flight
 // together: with an outlier in every block of every vector, us, one column at a time /
 // four (two vectors: two and four runs) / the fp32 kernels, 14336 x 4096 Q4_K at B = 128
 // 2540 / 1345 / 1998, 4096 x 14336 Q6_K 4340 / 1760 / 1440, 9216 x 3072 Q8_0 at B = 2 48 /
 // 37 / 25.
-template <class F, int NT, int NI>
-__device__ __forceinline__ void add_exact(uint64_t cols, const uint8_t *p, const float *x, size_t ldx, int nsb, int kh,
-                                          float (&tot)[NT][NI]) {
-    constexpr int K = NI == 8 ? 2 : 4, kUnroll = NI == 8 ? 4 : 1;  // (HL: two vectors)
-    while (cols) {
+template <class F, int K, int kUnroll, int NT, int NI>
+__device__ __forceinline__ void add_columns(const Marks &marks, const uint8_t *p, const float *x, size_t ldx, int sb0, int sb1,
+                                            int kh, float (&tot)[NT][NI]) {
+    for (uint64_t cols = marks.cols; cols;) {
         int b[K];
         uint32_t off[K];
 #pragma unroll
@@ -896,7 +910,8 @@ __device__ __forceinline__ void add_exact(uint64_t cols, const uint8_t *p, const
         }
         float acc[K] = {};
 #pragma unroll 1
-        for (int sb = 0; sb < nsb; sb++) {
+        for (int sb = sb0; sb < sb1; sb++) {
+            if (!(marks.blocks >> (sb & 63) & 1)) continue;
             const float *xb[K];
             float4 v[K];
 #pragma unroll
@@ -959,6 +974,14 @@ __device__ __forceinline__ void add_exact(uint64_t cols, const uint8_t *p, const
                 for (int i = 0; i < NI; i++) tot[n][i] = batch_of(n, i, kh) == b[c] ? tot[n][i] + acc[c] : tot[n][i];
         }
     }
+}
+
+template <class F, int NT, int NI>
+__device__ __forceinline__ void add_exact(const Marks &marks, const uint8_t *p, const float *x, size_t ldx, int sb0, int sb1,
+                                          int kh, float (&tot)[NT][NI]) {
+    if constexpr (NI == 8) add_columns<F, 2, 4>(marks, p, x, ldx, sb0, sb1, kh, tot);  // (HL: two vectors)
+    else if (__builtin_popcountll(marks.cols) <= 2) add_columns<F, 1, 4>(marks, p, x, ldx, sb0, sb1, kh, tot);
+    else add_columns<F, 4, 1>(marks, p, x, ldx, sb0, sb1, kh, tot);
 }
 
 // A wave's 32 weight rows (past the end: the last row again): a wave-uniform
@@ -1271,7 +1294,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
                 *reinterpret_cast<u32x4 *>(wslot + 16 * win_chunk<CH, RC>(lane + 64 * k)) = ch_n[k];       \
     } while (0)
 
-    uint64_t marked = 0;  // columns with blocks left to add_exact
+    Marks marked;  // blocks left to add_exact
     float tot[NT][NI], tot2[NI];
     if constexpr (TWO) {
 #pragma unroll
@@ -1315,7 +1338,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
             }
             JH_MT(3 + 4 * (sb - sb0));
             const Ctx<HL, NT> c{lr, kh, lds + buf * I::kBytes};
-            if constexpr (EXACT) marked |= marked_columns<HL, NT>(c);
+            if constexpr (EXACT) marked.add(marked_columns<HL, NT>(c), sb);
             F::template compute<HL, NT, TWO>(w, c, tot);
             if constexpr (TWO) {
 #pragma unroll
@@ -1347,7 +1370,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
             JH_LOAD_W(min(sb + 1, sb1 - 1));
             __syncthreads();
             const Ctx<HL, NT> c{lr, kh, lds};
-            if constexpr (EXACT) marked |= marked_columns<HL, NT>(c);
+            if constexpr (EXACT) marked.add(marked_columns<HL, NT>(c), sb);
             F::template compute<HL, NT, TWO>(w, c, tot);
         }
     }
@@ -1356,8 +1379,8 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
 #undef JH_PARK
 
     if constexpr (EXACT) {
-        if (__builtin_expect(marked != 0, 0))
-            add_exact<F>(marked, W + myoff + (size_t)sb0 * F::kBytes, X + 256 * sb0, cols, sb1 - sb0, kh, tot);
+        if (__builtin_expect(marked.cols != 0, 0))
+            add_exact<F>(marked, W + myoff, X, cols, sb0, sb1, kh, tot);
     }
     if constexpr (PAIR) {
         store_pair(tot, rbase + lr, (wave & (kWaves / 2 - 1)) * kRowsPerWave + lr, up_half, nrows, kh, B,
@@ -1479,7 +1502,7 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
             SET[k] = *reinterpret_cast<const u32x4 *>(W + ((coff[k] + sbo) & ~15u));                \
     } while (0)
 
-    uint64_t marked = 0;
+    Marks marked;
     float tot[1][kOut<HL>] = {};
 #define JH_STEP(SET, SB, BUF)                                                                              \
     do {                                                                                                   \
@@ -1494,7 +1517,7 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
         F::load(w, wslot + lr * RC * 16 + ((myoff + (uint32_t)(SB) * F::kBytes) & 15), kh);  \
         JH_LOAD_W(SET, (SB) + 2);                                                                          \
         const CtxP<HL> c{lr, kh, sh_x[BUF]};                                                               \
-        if constexpr (EXACT) marked |= marked_columns<HL, 1>(c);                                           \
+        if constexpr (EXACT) marked.add(marked_columns<HL, 1>(c), SB);                                     \
         F::template compute<HL, 1, false>(w, c, tot);                                                      \
     } while (0)
 
@@ -1512,7 +1535,7 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
 #undef JH_LOAD_W
 
     if constexpr (EXACT) {
-        if (__builtin_expect(marked != 0, 0)) add_exact<F>(marked, W + myoff, X, (size_t)256 * nsb, nsb, kh, tot);
+        if (__builtin_expect(marked.cols != 0, 0)) add_exact<F>(marked, W + myoff, X, (size_t)256 * nsb, 0, nsb, kh, tot);
     }
     store_tile(tot, rbase + lr, nrows, kh, B, Y, nullptr, 0, nullptr, blockIdx.x, 0, 1);
 }
