@@ -270,6 +270,26 @@ WsKey ws_key(WorkspacePool &pool, int device, hipStream_t s) {
     return {device, s, t_workspaces.id};
 }
 
+// While it lives, this thread may allocate and free although another stream of the
+// process is being captured: in the default (global) mode that would be refused and
+// would end the capture.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    RelaxedCapture(const RelaxedCapture &) = delete;
+};
+
+// A wait for the device under RelaxedCapture: hipDeviceSynchronize ends another
+// stream's capture in every mode; hipFree waits as it does, and ends none.
+int wait_for_device() {
+    void *p = nullptr;
+    int rc = device_alloc(&p, 256);
+    if (rc) return rc;
+    JH_HIP("hipFree(wait)", hipFree(p));
+    return JH_OK;
+}
+
 int stream_is_capturing(hipStream_t s, bool *capturing) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     JH_HIP("hipStreamIsCapturing", hipStreamIsCapturing(s, &st));
@@ -294,13 +314,14 @@ int stream_workspace(int device, hipStream_t s, size_t bytes, void **out, int **
                         "device workspace of %zu bytes needed during graph capture (stream has %zu): make one eager "
                         "call of the same size on this stream before capturing",
                         bytes, e.cap);
+        const RelaxedCapture relaxed;
         size_t want = bytes < (8u << 20) ? (8u << 20) : bytes;
         if (e.base && want < 2 * e.cap) want = 2 * e.cap;
         Workspace w;
         if (of_thread)
             for (auto it = pool.spare.begin(); it != pool.spare.end(); ++it)
                 if (it->first == device && it->second.cap >= bytes) {
-                    JH_HIP("hipDeviceSynchronize(workspace)", hipDeviceSynchronize());  // its last user is done, its counters are 0
+                    if ((rc = wait_for_device())) return rc;  // its last user is done, its counters are 0
                     w = it->second;
                     pool.spare.erase(it);
                     break;
