@@ -87,8 +87,8 @@ template <int T> __device__ __forceinline__ void dequant_unit(const uint8_t *W, 
     else reinterpret_cast<quadf *>(out)[t] = deq_quad<T>(W, t);
 }
 
-template <int T> __global__ void dequant_k(const uint8_t *__restrict__ W, int64_t units, float *__restrict__ out) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+template <int T> __global__ void dequant_k(const uint8_t *__restrict__ W, int64_t block0, int64_t units, float *__restrict__ out) {
+    const int64_t t = (block0 + blockIdx.x) * blockDim.x + threadIdx.x;
     if (t < units) dequant_unit<T>(W, t, out);
 }
 
@@ -103,6 +103,20 @@ __global__ void dequant_row_k(const uint8_t *__restrict__ W, const int *__restri
     if (t >= units) return;
     const int tok = min(max(d_tokens[blockIdx.y], 0), rows - 1);
     dequant_unit<T>(W + (size_t)tok * pitch, t, out + (int64_t)blockIdx.y * row_elems);
+}
+
+// launch(first block, blocks) over `blocks` of 256 threads, 2^31 threads at a time: one
+// launch of 2^32 threads or more (from 2^34 elements on, at four a lane) leaves part of
+// the array unwritten, without an error
+template <class F>
+hipError_t in_launches(int64_t blocks, F launch) {
+    constexpr int64_t kMax = int64_t(1) << 23;
+    for (int64_t b = 0; b < blocks; b += kMax) {
+        launch(b, (unsigned)(blocks - b < kMax ? blocks - b : kMax));
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace
@@ -124,17 +138,17 @@ hipError_t launch_dequant(int type, const uint8_t *w, int rows, int cols, float 
     const int64_t units = dequant_units(type, (int64_t)rows * cols);
     if (units < 0) return hipErrorInvalidValue;
     if (units == 0) return hipSuccess;
-    dim3 block(256), grid((unsigned)((units + 255) / 256));
-    switch (type) {
-    case 12: dequant_k<12><<<grid, block, 0, s>>>(w, units, out); break;
-    case 13: dequant_k<13><<<grid, block, 0, s>>>(w, units, out); break;
-    case 14: dequant_k<14><<<grid, block, 0, s>>>(w, units, out); break;
-    case 8: dequant_k<8><<<grid, block, 0, s>>>(w, units, out); break;
-    case 10: dequant_k<10><<<grid, block, 0, s>>>(w, units, out); break;
-    case 11: dequant_k<11><<<grid, block, 0, s>>>(w, units, out); break;
-    case 0: dequant_k<0><<<grid, block, 0, s>>>(w, units, out); break;
-    }
-    return hipGetLastError();
+    return in_launches((units + 255) / 256, [&](int64_t b0, unsigned grid) {
+        switch (type) {
+        case 12: dequant_k<12><<<grid, 256, 0, s>>>(w, b0, units, out); break;
+        case 13: dequant_k<13><<<grid, 256, 0, s>>>(w, b0, units, out); break;
+        case 14: dequant_k<14><<<grid, 256, 0, s>>>(w, b0, units, out); break;
+        case 8: dequant_k<8><<<grid, 256, 0, s>>>(w, b0, units, out); break;
+        case 10: dequant_k<10><<<grid, 256, 0, s>>>(w, b0, units, out); break;
+        case 11: dequant_k<11><<<grid, 256, 0, s>>>(w, b0, units, out); break;
+        case 0: dequant_k<0><<<grid, 256, 0, s>>>(w, b0, units, out); break;
+        }
+    });
 }
 
 hipError_t launch_dequant_row(int type, const uint8_t *w, int rows, int cols, size_t pitch, const int *d_tokens,
@@ -238,8 +252,9 @@ __device__ __forceinline__ uint32_t pack4(int a, int b, int c, int d) {
 }
 
 // quantizeQ8_0 (LoraMerge.java:265-277): 8 lanes per block
-__global__ __launch_bounds__(256) void quant_q8_0(const float *__restrict__ src, int64_t quads, uint8_t *__restrict__ dst) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void quant_q8_0(const float *__restrict__ src, int64_t block0, int64_t quads,
+                                                  uint8_t *__restrict__ dst) {
+    const int64_t t = (block0 + blockIdx.x) * blockDim.x + threadIdx.x;
     if (t >= quads) return;  // whole groups of 8 lanes
     const quadf v = reinterpret_cast<const quadf *>(src)[t];
     uint8_t *o = dst + (t >> 3) * 34;
@@ -265,10 +280,11 @@ __global__ __launch_bounds__(256) void quant_q8_0(const float *__restrict__ src,
 // (d = maxRange / 1953, 5th bits in qh); the quants use the fp32 d / dmin.
 // Sub-block s is lanes 8 s .. 8 s + 7.
 template <bool Q5>
-__global__ __launch_bounds__(256) void quant_kq(const float *__restrict__ src, int64_t nblk, uint8_t *__restrict__ dst) {
+__global__ __launch_bounds__(256) void quant_kq(const float *__restrict__ src, int64_t block0, int64_t nblk,
+                                                  uint8_t *__restrict__ dst) {
     constexpr int kBytes = Q5 ? 176 : 144, kQs = Q5 ? 48 : 16;
     constexpr float kQmax = Q5 ? 31.f : 15.f, kRange = Q5 ? 1953.f : 945.f;
-    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t t = (block0 + blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (t >= nblk) return;  // whole waves
     const int lane = threadIdx.x & 63, s = lane >> 3, i0 = 4 * (lane & 7);
     const quadf v = reinterpret_cast<const quadf *>(src + t * 256)[lane];
@@ -322,8 +338,9 @@ __global__ __launch_bounds__(256) void quant_kq(const float *__restrict__ src, i
 
 // quantizeQ6_K (LoraMerge.java:437-469): sub-block s is lanes 4 s .. 4 s + 3; a
 // lane's elements are quarter (lane >> 3) & 3 of half lane >> 5.
-__global__ __launch_bounds__(256) void quant_q6k(const float *__restrict__ src, int64_t nblk, uint8_t *__restrict__ dst) {
-    const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+__global__ __launch_bounds__(256) void quant_q6k(const float *__restrict__ src, int64_t block0, int64_t nblk,
+                                                   uint8_t *__restrict__ dst) {
+    const int64_t t = (block0 + blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (t >= nblk) return;  // whole waves
     const int lane = threadIdx.x & 63, half = lane >> 5, quarter = (lane >> 3) & 3, i0 = 4 * (lane & 7);
     const quadf v = reinterpret_cast<const quadf *>(src + t * 256)[lane];
@@ -365,14 +382,14 @@ hipError_t launch_quantize(int type, const float *src, int64_t n, uint8_t *dst, 
     if (nblk == 0) return hipSuccess;
     // a wave per 256 elements
     const int64_t waves = type == 8 ? (nblk + 7) / 8 : nblk;
-    dim3 block(256), grid((unsigned)((waves + 3) / 4));
-    switch (type) {
-    case 8: quant_q8_0<<<grid, block, 0, s>>>(src, nblk * 8, dst); break;
-    case 12: quant_kq<false><<<grid, block, 0, s>>>(src, nblk, dst); break;
-    case 13: quant_kq<true><<<grid, block, 0, s>>>(src, nblk, dst); break;
-    case 14: quant_q6k<<<grid, block, 0, s>>>(src, nblk, dst); break;
-    }
-    return hipGetLastError();
+    return in_launches((waves + 3) / 4, [&](int64_t b0, unsigned grid) {
+        switch (type) {
+        case 8: quant_q8_0<<<grid, 256, 0, s>>>(src, b0, nblk * 8, dst); break;
+        case 12: quant_kq<false><<<grid, 256, 0, s>>>(src, b0, nblk, dst); break;
+        case 13: quant_kq<true><<<grid, 256, 0, s>>>(src, b0, nblk, dst); break;
+        case 14: quant_q6k<<<grid, 256, 0, s>>>(src, b0, nblk, dst); break;
+        }
+    });
 }
 
 }  // namespace jh
