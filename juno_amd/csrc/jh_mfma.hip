@@ -1580,20 +1580,20 @@ struct Plan {
 //   a group of two     2048 x 2048 Q4_K 7.8 / 9.7, Q8_0 9.3 / 12.1; 2048 x 3072 10.9 / 10.4, 12.1 / 12.9;
 //                      1792 x 4096 13.1 / 10.6, 19.3 / 13.1; 4096 x 2048 10.5 / 9.9, 13.5 / 12.7
 //   a SwiGLU pair      2048 x 2048 Q4_K 9.9 / 9.8, Q8_0 11.3 / 12.5; 2560 x 2048 12.0 / 10.1, 15.2 / 12.6;
-//                      5632 x 2048 14.8 / 10.6, 19.4 / 14.2
+//                      5632 x 2048 14.8 / 10.6, 19.4 / 14.2; it has the limit of the group, whose bits it gives
 // Only formats whose error against 64 bits is smaller here (K = 512 .. 28672: Q4_K
 // 2.4-2.9e-7 / 1.8-2.0e-7, Q5_K 2.4-2.9e-7 / 1.8-2.0e-7, Q8_0 1.20-1.41e-7 / 0.81-1.25e-7);
 // that of Q6_K and Q3_K is not, and Q2_K is not taken either.
 static bool two_vectors_pay(int n, bool pair, int type, size_t rows, int cols) {
     const double weights = (double)rows * cols;
-    if (pair) return weights >= 10e6;
-    if (n > 1) return weights >= 14e6;
+    if (pair || n > 1) return weights >= 14e6;
     if (type == 8) return weights >= (rows > 2048 ? 22e6 : 36e6);
     return weights >= (rows > 4096 ? 26e6 : 36e6);
 }
 
 // Row tiles of 256 rows; K split the same way for every matrix of the group.  pair:
-// d[0] is a SwiGLU pair's virtual matrix, gate's rows and then up's.
+// d[0] is a SwiGLU pair's virtual matrix, gate's rows and then up's: K is split as for
+// the group of the two.
 static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p, bool pair = false) {
     if (n < 1 || n > kMaxMfmaGroup) return false;
     int tiles = 0;
@@ -1602,7 +1602,8 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p, bool pair = fal
     for (int i = 0; i < n; i++) {
         fine = fine || d[i].type == 14 || d[i].type == 11;
         if (!mfma_applies(d[i], B) || d[i].cols != d[0].cols) return false;
-        tiles += (d[i].row_end - d[i].row_start + kRowsPerWG - 1) / kRowsPerWG;
+        const int each = (d[i].row_end - d[i].row_start) / (pair ? 2 : 1);
+        tiles += (pair ? 2 : 1) * ((each + kRowsPerWG - 1) / kRowsPerWG);
         rows += d[i].row_end - d[i].row_start;
         if (B == 2 && d[i].type != 12 && d[i].type != 13 && d[i].type != 8) return false;
     }
@@ -1725,7 +1726,7 @@ bool mfma_swiglu_applies(const MfmaDesc &gate, const MfmaDesc &up, int B) {
     if (gate.type != 12 && gate.type != 13 && gate.type != 14 && gate.type != 8) return false;
     if (((reinterpret_cast<uintptr_t>(up.w) | up.pitch) & 15) && (up.type == 12 || up.type == 13)) return false;
     MfmaDesc v = gate;
-    v.row_end = 2 * gate.row_end;  // the pair's virtual rows: same tiles and K split as one matrix of 2 x rows
+    v.row_end = 2 * gate.row_end;  // the pair's virtual rows
     Plan p;
     return plan_group(1, &v, B, p, true) && (p.ksplit == 1 || (gate.row_end + kRowsPerWG / 2 - 1) / (kRowsPerWG / 2) <= kMaxTileCounters);
 }

@@ -59,7 +59,7 @@ def test_two_vectors(qtype, rows, cols, lo, mfma, captured):
     check(y.cpu().numpy(), X, deq, (qtype, rows, cols, captured))
 
 
-@pytest.mark.parametrize("rows,cols,fused", [(4096, 2560, True), (5120, 2560, True), (2441, 2048, False), (2442, 2048, True)])
+@pytest.mark.parametrize("rows,cols,fused", [(4096, 2560, True), (5120, 2560, True), (3417, 2048, False), (3418, 2048, True)])
 @pytest.mark.parametrize("captured", [False, True])
 def test_two_vector_swiglu(rows, cols, fused, captured):
     import torch
@@ -124,3 +124,26 @@ def test_two_vector_group(rows, mfma):
         check(y.cpu().numpy(), X, O.dequantize(t, w, r, cols).reshape(r, cols).astype(np.float64), (t, r, mfma))
     for d in devs:
         d.close()
+
+
+@pytest.mark.parametrize("B", [2, 3, 17])
+@pytest.mark.parametrize("rows,cols", [(2600, 2048), (10753, 2048), (3073, 5120)])
+def test_swiglu_pair_has_the_groups_bits(rows, cols, B):
+    """The pair kernel against the grouped call and silu * up, also where the pair's
+    rows together fill another number of row tiles than each matrix's do, and below the
+    pair's limit."""
+    import torch
+    L = _lib.load()
+    raws = [weights(O.Q4_K, rows, cols, 80 + i) for i in range(2)]
+    x = torch.from_numpy(np.random.default_rng(81).standard_normal((B, cols)).astype(np.float32)).cuda()
+    out, a, b, want = (torch.zeros(B, rows, device="cuda") for _ in range(4))
+    torch.cuda.synchronize()
+    with upload(O.Q4_K, rows, cols, raws[0]) as gate, upload(O.Q4_K, rows, cols, raws[1]) as up:
+        assert L.jh_qmatvec_batched_swiglu_dev(gate.handle, up.handle, P(x.data_ptr()), B, P(out.data_ptr()), P(a.data_ptr()),
+                                               P(b.data_ptr()), None) == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        assert L.jh_qmatvec_batched_group_dev(2, (P * 2)(gate.handle, up.handle), (P * 2)(x.data_ptr(), x.data_ptr()), B,
+                                              (P * 2)(a.data_ptr(), b.data_ptr()), None) == 0, _lib.last_error()
+        assert L.jh_silu_mul_dev(P(a.data_ptr()), P(b.data_ptr()), B * rows, P(want.data_ptr()), None) == 0
+        torch.cuda.synchronize()
+    assert torch.equal(out, want)
