@@ -160,7 +160,8 @@ int jh_qmat_dequant_dev(const jh_qmat *m, float *d_out, void *stream);
  * beside an eager call) race and must be ordered by the caller.  Results are
  * those of jh_qmatvec_batched_dev, bit for bit (calls of two and of more than 64 vectors
  * never need more than that array; jh_qmatvec_batched_dev captured before its
- * stream has a workspace takes kernels without scratch for them instead). */
+ * stream has a workspace takes kernels without scratch for them instead, with other
+ * roundings). */
 int jh_qmatvec_batched_noalloc_dev(const jh_qmat *m, const float *d_X, int B, float *d_Y, int row_start,
                                    int row_end, void *stream);
 
@@ -236,7 +237,8 @@ int jh_rmsnorm_qmatvec_group_dev(int n, const jh_qmat *const *mats, const float 
                                  void *stream);
 
 /* Batched form: out[b][r] = silu(gate_r . X_b) * (up_r . X_b) for B rows of X.
- * For 3 <= B <= 32 (Q4_K, Q5_K, Q6_K, Q8_0) one MFMA launch whose workgroups
+ * For 3 <= B <= 32 (Q4_K, Q5_K, Q6_K, Q8_0), and for pairs of 14 M weights or more at
+ * B = 2 (not Q6_K), one MFMA launch whose workgroups
  * take 128 rows of gate and the same rows of up and store the product; B = 1
  * is jh_qmatvec_swiglu_dev; otherwise jh_qmatvec_batched_group_dev into the
  * caller's d_gate / d_up scratch ([B][rows] each, used only on that path) and
@@ -247,8 +249,9 @@ int jh_qmatvec_batched_swiglu_dev(const jh_qmat *gate, const jh_qmat *up, const 
 /* Batched form of jh_qmatvec_group_dev: Y_i[B][rows_i] = X_i[B][cols] W_i^T
  * for n <= 4 matrices, full row ranges, one launch when B >= 3 and the
  * matrices share cols (the MFMA path; formats may differ, e.g. the Q4_K q / k
- * and Q6_K v of a Q4_K_M layer), else one call per matrix.  Same results as
- * n calls of jh_qmatvec_batched_dev.  The reference's forwardBatch runs the
+ * and Q6_K v of a Q4_K_M layer), or at B = 2 from 14 M weights of Q4_K, Q5_K and
+ * Q8_0 on; else one call per matrix.  Equal, to the GEMV tolerance, to
+ * n calls of jh_qmatvec_batched_dev (whose kernel or split of K may be another).  The reference's forwardBatch runs the
  * requests one by one (InferencePipeline.java:62-69); this is the grouped
  * projection step of its batched replacement. */
 int jh_qmatvec_batched_group_dev(int n, const jh_qmat *const *mats, const float *const *d_X, int B,
@@ -266,6 +269,12 @@ int jh_qmatvec_batched_plan(int n, const jh_qmat *const *mats, int B, int *kerne
  * checks of the kernels' address arithmetic. */
 int jh_qmatvec_batched_plan_shape(int ggml_type, int cols, int row_start, int row_end, int B, int *kernel,
                                   int *ksplit);
+/* More of that launch: out[0..n) = kernel, K split, super-blocks (256 columns of W) per
+ * split, vectors per column chunk and column chunks, the byte offsets in the staged
+ * x of its lo limbs, 32- and 16-value sums and scales, its size, a row's weight window
+ * as loaded and as spaced in 16-byte chunks, and the LDS bytes; 0s where the MFMA
+ * path does not apply, and past these 13. */
+int jh_qmatvec_batched_layout_shape(int ggml_type, int cols, int row_start, int row_end, int B, int *out, int n);
 
 /* Diagnostics of the per-stream library workspace (see Conventions): the
  * scratch bytes the stream `stream` on `device` currently has (0 before its

@@ -43,6 +43,7 @@ SIGNATURES = {
     "jh_sync_faults": (_I, [_I, _P]),
     "jh_debug_timeline": (_I, [_I, _I, _P, ctypes.c_size_t]),
     "jh_qmatvec_batched_plan_shape": (_I, [_I, _I, _I, _I, _I, _P, _P]),
+    "jh_qmatvec_batched_layout_shape": (_I, [_I, _I, _I, _I, _I, _P, _I]),
     "jh_qmatvec_batched_group_dev": (_I, [_I, _P, _P, _I, _P, _P]),
     "jh_qmatvec_swiglu_dev": (_I, [_P, _P, _P, _P, _P]),
     "jh_rmsnorm_qmatvec_swiglu_dev": (_I, [_P, _P, _P, _P, _P, ctypes.c_float, _P, _P, _P, _P]),

@@ -434,19 +434,38 @@ extern "C" {
 
 const char *jh_last_error(void) { return g_last_error.c_str(); }
 
-int jh_qmatvec_batched_plan_shape(int ggml_type, int cols, int row_start, int row_end, int B, int *kernel,
-                                  int *ksplit) {
-    if (!kernel || !ksplit) return fail(JH_EINVAL, "kernel and ksplit must not be null");
+static int shape_desc(int ggml_type, int cols, int row_start, int row_end, jh::MfmaDesc *d) {
     int qk, bb;
     if (!type_geometry(ggml_type, &qk, &bb)) return fail(JH_EUNSUPPORTED, "no block geometry for GGML type %d", ggml_type);
     if (cols <= 0 || cols % qk || row_start < 0 || row_end < row_start)
         return fail(JH_EINVAL, "invalid shape: cols=%d rows [%d, %d)", cols, row_start, row_end);
     // the planner reads formats, sizes and alignment only: a 256-byte-aligned stand-in address will do
     const uint8_t *w = reinterpret_cast<const uint8_t *>(uintptr_t(1) << 20);
-    const jh::MfmaDesc d{ggml_type, w, (size_t)(cols / qk) * bb, cols, row_start, row_end,
-                         reinterpret_cast<const float *>(w), nullptr};
+    *d = jh::MfmaDesc{ggml_type, w, (size_t)(cols / qk) * bb, cols, row_start, row_end, reinterpret_cast<const float *>(w), nullptr};
+    return JH_OK;
+}
+
+int jh_qmatvec_batched_plan_shape(int ggml_type, int cols, int row_start, int row_end, int B, int *kernel,
+                                  int *ksplit) {
+    if (!kernel || !ksplit) return fail(JH_EINVAL, "kernel and ksplit must not be null");
+    jh::MfmaDesc d;
+    int rc = shape_desc(ggml_type, cols, row_start, row_end, &d);
+    if (rc) return rc;
     *ksplit = 1;
     *kernel = B >= 2 ? jh::mfma_group_plan(1, &d, B, ksplit) : 0;
+    return ok();
+}
+
+int jh_qmatvec_batched_layout_shape(int ggml_type, int cols, int row_start, int row_end, int B, int *out, int n) {
+    if (!out || n < 0) return fail(JH_EINVAL, "out must not be null, n must be >= 0");
+    jh::MfmaDesc d;
+    int rc = shape_desc(ggml_type, cols, row_start, row_end, &d);
+    if (rc) return rc;
+    jh::MfmaLayout l = {};
+    if (B >= 2) jh::mfma_layout(d, B, l);
+    const int v[] = {l.kernel,    l.ksplit,    l.ksb,      l.columns, l.column_chunks, l.image_lo, l.image_xs,
+                     l.image_x16, l.image_cs,  l.image,    l.chunks16, l.row_chunks16, l.lds};
+    for (int i = 0; i < n; i++) out[i] = i < (int)(sizeof(v) / sizeof(v[0])) ? v[i] : 0;
     return ok();
 }
 

@@ -121,6 +121,15 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
 // Which kernel launch_mfma_group takes: 0 none (the path does not apply),
 // 1 mfma_group (K split *ksplit ways), 2 x_prep + mfma_px (one unsplit matrix).
 int mfma_group_plan(int n, const MfmaDesc *d, int B, int *ksplit);
+// The launch of one matrix as the CPU checks of its addresses need it: the plan, the x
+// image (or prepared slab: kernel 2) as byte offsets of its lo limbs, 32- and 16-value
+// sums and column scales, and the weight windows in 16-byte chunks per row.
+struct MfmaLayout {
+    int kernel, ksplit, ksb, columns, column_chunks;
+    int image_lo, image_xs, image_x16, image_cs, image;
+    int chunks16, row_chunks16, lds;
+};
+bool mfma_layout(const MfmaDesc &d, int B, MfmaLayout &l);
 // The file-scope device scratch of the MFMA path for callers that cannot
 // allocate (jh_qmatvec_batched_noalloc_dev): kStaticScratchBytes of workspace
 // plus the split-K counters, one copy per device.  static_scratch returns this

@@ -1674,16 +1674,80 @@ int mfma_group_plan(int n, const MfmaDesc *d, int B, int *ksplit) {
     return p.prepared ? 2 : 1;
 }
 
-template <int NT>
-static void launch_wide(const MfmaGroup &g, int mask, int grid, hipStream_t s) {
+namespace {
+template <bool HL, int NT>
+void image_layout(MfmaLayout &l) {
+    using I = XImage<HL, NT>;
+    l.image_lo = 2 * I::kLo;
+    l.image_xs = 2 * I::kXs;
+    l.image_x16 = 2 * I::kX16;
+    l.image_cs = I::kCs;
+    l.image = I::kBytes;
+}
+template <bool HL>
+void slab_layout(MfmaLayout &l) {
+    l.image_lo = HL ? 0 : Slab<HL>::kLo;
+    l.image_xs = Slab<HL>::kXs;
+    l.image_x16 = 0;
+    l.image_cs = Slab<HL>::kCs;
+    l.image = Slab<HL>::kBytes;
+}
+template <class F, int MASK>
+void format_layout(MfmaLayout &l, bool hl, int nt) {
+    l.chunks16 = F::kChunks;
+    l.row_chunks16 = nt == 1 ? F::kRowChunks : F::kChunks;
+    l.lds = l.kernel == 2 ? 2 * l.image + kWaves * kRowsPerWave * F::kRowChunks * 16 + kWinPad
+            : nt == 2     ? lds_bytes<false, 2, MASK>()
+            : hl          ? lds_bytes<true, 1, MASK>()
+                          : lds_bytes<false, 1, MASK>();
+}
+}  // namespace
+
+bool mfma_layout(const MfmaDesc &d, int B, MfmaLayout &l) {
+    Plan p;
+    l = {};
+    if (!plan_group(1, &d, B, p)) return false;
+    const bool hl = B <= kHlMaxBatch;
+    const int nt = B > 64 ? p.chunk / 32 : B > 32 ? 2 : 1;
+    l.kernel = p.prepared ? 2 : 1;
+    l.ksplit = p.ksplit;
+    l.ksb = p.ksb;
+    l.columns = B > 64 ? p.chunk : hl ? 16 : 32 * nt;
+    l.column_chunks = p.chunks;
+    if (p.prepared) hl ? slab_layout<true>(l) : slab_layout<false>(l);
+    else if (nt == 2) image_layout<false, 2>(l);
+    else hl ? image_layout<true, 1>(l) : image_layout<false, 1>(l);
+    switch (d.type) {
+        case 12: format_layout<FmtQ4K, 1>(l, hl, nt); break;
+        case 13: format_layout<FmtQ5K, 2>(l, hl, nt); break;
+        case 14: format_layout<FmtQ6K, 4>(l, hl, nt); break;
+        case 10: format_layout<FmtQ2K, 16>(l, hl, nt); break;
+        case 11: format_layout<FmtQ3K, 32>(l, hl, nt); break;
+        default: format_layout<FmtQ8_0, 8>(l, hl, nt); break;
+    }
+    return true;
+}
+
+// chunks of 64 columns: no Q6_K or Q3_K (plan_group)
+static void launch_wide64(const MfmaGroup &g, int mask, int grid, hipStream_t s) {
     switch (mask) {
-        case 1: mfma_group<false, NT, 1, false, true><<<grid, kThreads, 0, s>>>(g); break;
-        case 2: mfma_group<false, NT, 2, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 1: mfma_group<false, 2, 1, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 2: mfma_group<false, 2, 2, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 8: mfma_group<false, 2, 8, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 16: mfma_group<false, 2, 16, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        default: mfma_group<false, 2, 27, false, true><<<grid, kThreads, 0, s>>>(g); break;
+    }
+}
+
+static void launch_wide32(const MfmaGroup &g, int mask, int grid, hipStream_t s) {
+    switch (mask) {
+        case 1: mfma_group<false, 1, 1, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 2: mfma_group<false, 1, 2, false, true><<<grid, kThreads, 0, s>>>(g); break;
         case 4: mfma_group<false, 1, 4, false, true><<<grid, kThreads, 0, s>>>(g); break;
-        case 8: mfma_group<false, NT, 8, false, true><<<grid, kThreads, 0, s>>>(g); break;
-        case 16: mfma_group<false, NT, 16, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 8: mfma_group<false, 1, 8, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        case 16: mfma_group<false, 1, 16, false, true><<<grid, kThreads, 0, s>>>(g); break;
         case 32: mfma_group<false, 1, 32, false, true><<<grid, kThreads, 0, s>>>(g); break;
-        default: mfma_group<false, NT, NT == 1 ? 63 : 27, false, true><<<grid, kThreads, 0, s>>>(g); break;
+        default: mfma_group<false, 1, 63, false, true><<<grid, kThreads, 0, s>>>(g); break;
     }
 }
 
@@ -1881,8 +1945,8 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
         mask |= q.type == 12 ? 1 : q.type == 13 ? 2 : q.type == 14 ? 4 : q.type == 10 ? 16 : q.type == 11 ? 32 : 8;
     }
     g.chunks = p.chunks;
-    if (B > 64 && p.chunk == 64) launch_wide<2>(g, mask, p.grid, s);
-    else if (B > 64) launch_wide<1>(g, mask, p.grid, s);
+    if (B > 64 && p.chunk == 64) launch_wide64(g, mask, p.grid, s);
+    else if (B > 64) launch_wide32(g, mask, p.grid, s);
     else if (B == 2) launch_two(g, mask, p.grid, s);
     else if (B <= kHlMaxBatch) launch_group_nt<true, 1>(g, mask, p.grid, s);
     else if (B <= 32) launch_group_nt<false, 1>(g, mask, p.grid, s);

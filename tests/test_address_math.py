@@ -57,85 +57,165 @@ def within(lo, hi, size, what):
     assert lo >= 0 and hi <= size, f"{what}: bytes [{lo}, {hi}) outside [0, {size})"
 
 
-# ------------------------------------------------------------------ batched MFMA kernel (jh_mfma.hip)
-# Format constants: kBytes / kChunks / kRowChunks (jh_mfma.hip:293-295, 391-395, 451-453, 499-501, 561-563)
-MF = {Q4_K: (144, 9, 9), Q5_K: (176, 11, 11), Q6_K: (210, 14, 15), Q8_0: (272, 19, 20), Q2_K: (84, 6, 7),
-      Q3_K: (110, 8, 9)}
-ROWS_PER_WAVE, WAVES, ROWS_PER_WG, MIN_WG, COUNTER_SLOTS = 32, 8, 256, 256, 1024  # jh_mfma.hip:52-56, jh_kernels.hpp:149
-XPAD = 8
-COLH = 256 + XPAD
-SLAB_BYTES, SLAB_ROWS = 34 * 1024, 34
+# ------------------------------------------------------------------ batched MFMA kernels (jh_mfma.hip)
+# kBytes, kChunks, kRowChunks and the sums of x it reads (kSums) of each format
+MF = {Q4_K: (144, 9, 9, 32), Q5_K: (176, 11, 11, 32), Q6_K: (210, 14, 15, 0), Q8_0: (272, 18, 19, 0), Q2_K: (84, 6, 7, 16),
+      Q3_K: (110, 8, 9, 0)}
+ROWS_PER_WAVE, WAVES, ROWS_PER_WG, MIN_WG, COUNTER_SLOTS = 32, 8, 256, 256, 1024
+STATIC_SCRATCH = 8 << 20
+COLH = 256 + 8  # halves per column of the staged x, kXPad among them
 WIN_PAD = 16
+HL_MAX = 16     # kHlMaxBatch
 
 
-def plan(tiles_list, nsb, B, types):
-    """plan_group (jh_mfma.hip:1206-1241): the K split by its cost model."""
-    tiles = sum(tiles_list)
-    best, ksb, ksplit = 1 << 30, nsb, 1
-    for ks in range(1, nsb + 1):
-        kb = (nsb + ks - 1) // ks
-        kse = (nsb + kb - 1) // kb
-        if kse > 1 and tiles > COUNTER_SLOTS:
-            break
-        rounds = (tiles * kse + MIN_WG - 1) // MIN_WG
-        cost = 4 * (rounds * (kb + 5) + (1 if kse > 1 else 0)) + (kse if kse > 1 else 0)
-        if cost < best:
-            best, ksb, ksplit = cost, kb, kse
-    prepared = len(tiles_list) == 1 and ksplit == 1 and B <= 32 and types[0] not in (Q2_K, Q3_K)
-    return ksb, ksplit, prepared
+def two_vectors_pay(t, rows, cols):
+    if t not in (Q4_K, Q5_K, Q8_0):
+        return False
+    if t == Q8_0:
+        return rows * cols >= (22e6 if rows > 2048 else 36e6)
+    return rows * cols >= (26e6 if rows > 4096 else 36e6)
 
 
-def lds_w_offset(nt):  # jh_mfma.hip:748
-    return (2 * 32 * nt * COLH + 32 * nt * 16 + 32 * nt * 32) * 2 + 32 * nt * 8
+def plan(t, rows, cols, B):
+    """plan_group for one matrix: None, or (ksb, ksplit, columns per chunk, chunks, prepared)."""
+    nsb = cols // 256
+    if B == 2 and not two_vectors_pay(t, rows, cols):
+        return None
+    tiles = -(-rows // ROWS_PER_WG)
+    best = None
+    for c in (64, 32) if B > 64 and t not in (Q6_K, Q3_K) else (32,):
+        chunks = 1 if B <= 64 else -(-B // c)
+        for ks in range(1, nsb + 1):
+            ksb = -(-nsb // ks)
+            kse = -(-nsb // ksb)
+            if kse > 1 and (tiles * chunks > COUNTER_SLOTS or (B > 64 and 4 * kse * B * rows > STATIC_SCRATCH)):
+                break
+            rounds = -(-tiles * chunks * kse // MIN_WG)
+            cost = (4 * (rounds * (ksb + 5) + (kse > 1)) + (kse if kse > 1 else 0)) * (8 if c == 64 else 5)
+            if best is None or cost < best[0]:
+                best = (cost, ksb, kse, c, chunks)
+    _, ksb, kse, c, chunks = best
+    prepared = kse == 1 and B <= 32 and t not in (Q2_K, Q3_K)
+    return ksb, kse, c, chunks, prepared
 
 
-def lds_bytes(nt, types):  # jh_mfma.hip:750-753
-    return (2 if nt == 1 else 1) * lds_w_offset(nt) + WAVES * ROWS_PER_WAVE * max(MF[t][2] for t in types) * 16 + WIN_PAD
+class Image:
+    """The x of one super-block in LDS (XImage, or Slab where x is prepared): where a
+    lane's values go and where operands are read, in bytes."""
+
+    def __init__(self, hl, nt, prepared):
+        self.hl, self.nt, self.prepared = hl, nt, prepared
+        self.cols = 16 if hl else 32 * nt  # columns staged
+        if prepared:
+            self.lo = 0 if hl else 16384
+            self.xs, self.x16 = (16384 if hl else 32768), 0
+            self.cs = self.xs + 1024
+            self.size = (self.xs // 1024 + 2) * 1024
+        else:
+            self.lo = 2 * (16 if hl else 32 * nt) * COLH
+            self.xs = 2 * (1 if hl else 2) * 32 * nt * COLH
+            self.x16 = self.xs + 2 * 32 * nt * 16
+            self.cs = self.x16 + 2 * 32 * nt * 32
+            self.size = self.cs + 32 * nt * 4
+
+    def unit(self, v, off, lo):
+        """Byte of the 8 values from `off` on of A row v (!hl: of its lo plane)."""
+        if self.prepared:
+            return (self.lo if lo else 0) + 16 * ((v << 5) | ((off >> 3) ^ v))
+        return (self.lo if lo else 0) + 2 * (v * COLH + off)
+
+    def writes(self):
+        """name -> (start, length) of everything one super-block's staging writes."""
+        col = np.arange(self.cols)[:, None, None]
+        q, u = np.arange(16)[None, :, None], np.arange(2)[None, None, :]
+        off = 16 * q + 8 * u
+        out = {"hi": (self.unit(col, off, False), 16)}
+        # with both limbs in one operand the lo limbs are A rows 16 .. 31
+        out["lo"] = (self.unit(16 + col, off, False) if self.hl and self.prepared else self.unit(col, off, True), 16)
+        rows = 32 * self.nt
+        out["sums32"] = (self.xs + 2 * np.arange(rows * 16), 2)
+        if not self.prepared:
+            out["sums16"] = (self.x16 + 2 * np.arange(rows * 32), 2)
+        out["scales"] = (self.cs + 4 * col.reshape(-1), 4)
+        return out
+
+    def reads(self):
+        row, kh = np.arange(32 * self.nt)[:, None], np.arange(2)[None, :]
+        off = 16 * np.arange(16)[:, None, None] + 8 * kh
+        out = {"x": (self.unit(row, off, False), 16)}
+        if not self.hl:
+            out["xlo"] = (self.unit(row, off, True), 16)
+        out["sums32"] = (self.xs + 2 * (row * 16 + 8 * kh), 16)
+        if not self.prepared:
+            out["sums16"] = (self.x16 + 2 * (row[..., None] * 32 + 8 * kh[..., None] + 16 * np.arange(2)), 16)
+        n, i = np.arange(self.nt)[:, None, None], np.arange(2 if self.hl else 4)[None, :, None]
+        out["scales"] = (self.cs + 4 * (n * 32 + 8 * i + 4 * kh[None]), 16)
+        return out
 
 
-def win_chunk(j, ch, rc):  # jh_mfma.hip:278-279
+def bytes_of(a):
+    start, n = a
+    return np.unique((np.asarray(start).reshape(-1, 1) + np.arange(n)).reshape(-1))
+
+
+@pytest.mark.parametrize("hl,nt,prepared", [(True, 1, False), (False, 1, False), (False, 2, False), (True, 1, True),
+                                            (False, 1, True)])
+def test_x_image(hl, nt, prepared):
+    """What the staging writes does not overlap and stays in the image, and what the
+    operand reads touch has been written."""
+    im = Image(hl, nt, prepared)
+    parts = {k: bytes_of(v) for k, v in im.writes().items()}
+    everything = np.concatenate(list(parts.values()))
+    assert len(np.unique(everything)) == len(everything)
+    within(everything, everything + 1, im.size, "x image write")
+    for name, r in im.reads().items():
+        assert np.all(np.asarray(r[0]) % min(r[1], 16) == 0), name
+        assert np.isin(bytes_of(r), everything).all(), name
+
+
+def win_chunk(j, ch, rc):
     return j + (rc - ch) * (j // ch)
 
 
-def check_mfma_weights(t, rows_alloc, p, row0, nrows, tiles, sb_ranges, nt, lds_total, prepared):
-    """Weight chunk loads (JH_LOAD_W, jh_mfma.hip:874-879 / 1136-1140) and the
-    window writes and field reads (:939-945, 964-969)."""
-    kbytes, ch, rc_fmt = MF[t]
-    rc = rc_fmt if (nt == 1) else ch  # RC: padded window rows at NT = 1 (jh_mfma.hip:867)
-    if prepared:
-        rc = rc_fmt                      # mfma_px always uses the padded rows (:1106)
+def check_mfma_weights(t, rows_alloc, p, row0, nrows, tiles, sb_ranges, nt, image_bytes, lds_total, prepared):
+    """RowSpan's 32-bit offsets, the weight chunk loads (JH_LOAD_W), the windows'
+    writes (JH_PARK) and field reads, and the fields that run() reads in memory."""
+    kbytes, ch, rc_fmt, _ = MF[t]
+    rc = rc_fmt if nt == 1 else ch
     cl = (ROWS_PER_WAVE * ch + 63) // 64
-    lane = np.arange(64)
-    k = np.arange(cl)
+    lane, k = np.arange(64), np.arange(cl)
     j = np.minimum(lane[:, None] + 64 * k[None, :], ROWS_PER_WAVE * ch - 1)           # (64, CL)
-    tile = np.arange(tiles)[:, None, None, None]
-    wave = np.arange(WAVES)[None, :, None, None]
-    rbase = tile * ROWS_PER_WG + wave * ROWS_PER_WAVE
-    row = row0 + np.minimum(rbase + j[None, None] // ch, nrows - 1)                   # row_off (:858)
-    coff = row * p + 16 * (j[None, None] % ch)
+    rbase = (np.arange(tiles)[:, None] * ROWS_PER_WG + np.arange(WAVES)[None] * ROWS_PER_WAVE)[..., None, None]
+
+    def row(rho):
+        return np.minimum(rbase + rho, nrows - 1)
+
+    first = (row0 + row(0)) * p
+    base = first & ~15
+
+    def offset(rho):
+        o = (first & 15) + (row(rho) - row(0)) * p
+        assert o.max() + max(b for _, b in sb_ranges) * kbytes + 16 * ch < 1 << 32
+        return o
+
+    coff, myoff = offset(j[None, None] // ch) + 16 * (j[None, None] % ch), offset((lane & 31)[None, None, :, None])
     alloc = rows_alloc * p + TAIL
+    windows = 0 if prepared else (2 if nt == 1 else 1) * image_bytes  # mfma_px: an array of their own
+    size = WAVES * ROWS_PER_WAVE * rc * 16 + WIN_PAD if prepared else lds_total
+    wave0 = windows + np.arange(WAVES)[None, :, None, None] * (ROWS_PER_WAVE * rc * 16)
     for sb0, sb1 in sb_ranges:
         for sb in {sb0, sb1 - 1}:
-            a = (coff + sb * kbytes) & ~15
+            a = base + ((coff + sb * kbytes) & ~15)
             within(a, a + 16, alloc, f"mfma weights type {t} sb {sb}")
-            # the lane's own block inside its window: myoff + sb*kBytes, misalignment 0..15,
-            # fields read up to kBytes plus one dword of realignment (lds_read_u, :255-263)
-            myoff = (row0 + np.minimum(rbase[:, :, 0, 0][..., None] + (lane & 31)[None, None, :], nrows - 1)) * p
-            mis = (myoff + sb * kbytes) & 15
-            lr = lane & 31
-            start = lds_w_offset(nt) * (1 if (nt == 2 or prepared) else 2) \
-                + wave[:, :, 0, 0][..., None] * (ROWS_PER_WAVE * rc * 16) + lr[None, None, :] * rc * 16 + mis
-            if prepared:  # mfma_px: the windows are an array of their own (sh_w, jh_mfma.hip:1106)
-                start = start - lds_w_offset(nt)
-                within(start, start + kbytes + 4, WAVES * ROWS_PER_WAVE * rc * 16 + WIN_PAD, f"px window type {t}")
-            else:
-                within(start, start + kbytes + 4, lds_total, f"mfma window read type {t}")
-    wpos = win_chunk(j, ch, rc)
-    if not prepared:
-        base = lds_w_offset(nt) * (2 if nt == 1 else 1)
-        w = base + WAVES * 0 + (np.arange(WAVES)[:, None, None] * ROWS_PER_WAVE * rc * 16) + 16 * wpos[None]
-        live = (lane[:, None] + 64 * k[None, :]) < ROWS_PER_WAVE * ch
-        within(w[:, live], w[:, live] + 16, lds_total, f"mfma window write type {t}")
+            # a row's block inside its window, read up to a dword past it (lds_read_u)
+            at = wave0 + (lane & 31)[None, None, :, None] * rc * 16 + ((myoff + sb * kbytes) & 15)
+            within(at, at + kbytes + 4, size, f"mfma window read type {t}")
+            assert ((myoff + sb * kbytes) & 15).max() + kbytes <= 16 * ch  # the block was loaded whole
+            a = base + myoff + sb * kbytes  # run(): the fields of a block, all inside it
+            within(a, a + kbytes, alloc, f"mfma fp32 products type {t} sb {sb}")
+    live = (lane[:, None] + 64 * k[None, :]) < ROWS_PER_WAVE * ch
+    w = wave0 + 16 * win_chunk(j, ch, rc)[None, None]
+    within(w[..., live], w[..., live] + 16, size, f"mfma window write type {t}")
 
 
 @pytest.mark.parametrize("t,rows,cols", [s for s in SHAPES if s[2] % 256 == 0])
@@ -143,35 +223,56 @@ def test_mfma_addresses(t, rows, cols):
     L = _lib.load()
     p = pitch(t, cols)
     nsb = cols // 256
-    for B in (3, 8, 16, 20, 31, 32, 33, 48, 64):
-        nt = 1 if B <= 32 else 2
+    for B in (2, 3, 8, 16, 17, 20, 31, 32, 33, 48, 64, 65, 97, 128, 130):
         for r0, r1 in ranges(rows):
             nrows = r1 - r0
-            tiles = (nrows + ROWS_PER_WG - 1) // ROWS_PER_WG
-            ksb, ksplit, prepared = plan([tiles], nsb, B, [t])
-            # the library plans the same launch (jh_qmatvec_batched_plan: kernel 2 = prepared x, 1 = grouped)
-            kern, ks = ctypes.c_int(), ctypes.c_int()
+            tiles = -(-nrows // ROWS_PER_WG)
+            pl = plan(t, nrows, cols, B)
+            # the library plans the same launch with the same layout
+            kern, ks, lay = ctypes.c_int(), ctypes.c_int(), (ctypes.c_int * 13)()
             assert L.jh_qmatvec_batched_plan_shape(t, cols, r0, r1, B, ctypes.byref(kern), ctypes.byref(ks)) == 0
+            assert L.jh_qmatvec_batched_layout_shape(t, cols, r0, r1, B, lay, 13) == 0
+            if pl is None:
+                assert kern.value == 0 and not any(lay)
+                continue
+            ksb, ksplit, chunk, chunks, prepared = pl
+            hl = B <= HL_MAX
+            nt = chunk // 32 if B > 64 else 2 if B > 32 else 1
+            im = Image(hl, nt, prepared)
+            kbytes, ch, rc_fmt, _ = MF[t]
+            rc = rc_fmt if nt == 1 else ch
+            windows = WAVES * ROWS_PER_WAVE * (rc_fmt if prepared or nt == 1 else max(rc_fmt, ch)) * 16 + WIN_PAD
+            lds = (2 if nt == 1 else 1) * im.size + windows
             assert (kern.value, ks.value) == (2 if prepared else 1, ksplit), (t, rows, cols, B, r0, r1)
+            assert list(lay) == [kern.value, ksplit, ksb, chunk if B > 64 else im.cols, chunks, im.lo, im.xs, im.x16, im.cs,
+                                 im.size, ch, rc, lds], (t, rows, cols, B, r0, r1)
+            assert lds <= 160 * 1024
             sb_ranges = [(sp * ksb, min(nsb, sp * ksb + ksb)) for sp in range(ksplit)]
-            sb_ranges = [r for r in sb_ranges if r[0] < r[1]]
-            lds_total = lds_bytes(nt, [t])
-            assert lds_total <= 160 * 1024
-            check_mfma_weights(t, rows, p, r0, nrows, tiles, sb_ranges, nt, lds_total, prepared)
-            # x: X + min(b, B-1)*cols + SB*256 + 16*xq + 4k (JH_LOAD_X, :880-890): in [0, B*cols)
-            bmax = min(32 * nt - 1, B - 1)
-            within(0, (bmax * cols + (nsb - 1) * 256 + 16 * 15 + 16) * 4, B * cols * 4, "x")
-            # y and the split-K partials (store_tile, :626-700): b < B, r < nrows, splits < ksplit
-            within(0, ((B - 1) * nrows + nrows) * 4, B * nrows * 4, "y")
-            if ksplit > 1:
-                plane = B * nrows
-                within(0, ((ksplit - 1) * plane + (B - 1) * nrows + nrows) * 4, ksplit * B * nrows * 4, "partials")
-                assert tiles <= COUNTER_SLOTS  # a counter per tile (:1228)
-            if prepared:  # x_prep slabs and the DMA rows (:1040-1054, :1119-1128)
-                r = np.minimum(np.arange(WAVES)[:, None] + WAVES * np.arange((SLAB_ROWS + WAVES - 1) // WAVES), SLAB_ROWS - 1)
-                src = (nsb - 1) * SLAB_BYTES + 16 * 63 + 1024 * r
-                within(src, src + 16, nsb * SLAB_BYTES, "prepared x slab DMA source")
-                within(1024 * r, 1024 * r + 16 * 64, SLAB_BYTES, "prepared x slab DMA target")
+            assert all(a < b for a, b in sb_ranges)
+            check_mfma_weights(t, rows, p, r0, nrows, tiles, sb_ranges, nt, im.size, lds, prepared)
+            plane, covered = B * nrows, 0
+            for c in range(chunks):
+                col0 = c * chunk if B > 64 else 0
+                bc = min(32 * nt, B - col0) if B > 64 else B  # this chunk's columns
+                covered += bc
+                assert 1 <= bc <= im.cols
+                # x (JH_LOAD_X; add_exact reads the same columns): column min(b, bc - 1) of the chunk
+                last = col0 * cols + (min(im.cols - 1, bc - 1)) * cols + (nsb - 1) * 256 + 16 * 15 + 16
+                within(col0 * cols * 4, last * 4, B * cols * 4, "x")
+                # y and the split-K partials: b < bc, r < nrows, splits < ksplit
+                last = col0 * nrows + (bc - 1) * nrows + nrows
+                within(col0 * nrows * 4, last * 4, B * nrows * 4, "y")
+                within(0, ((ksplit - 1) * plane + last) * 4, ksplit * plane * 4, "partials")
+                if ksplit > 1:
+                    within(c, (tiles - 1) * chunks + c + 1, COUNTER_SLOTS, "tile counters")
+            assert covered == B
+            if prepared:  # x_prep's slabs and the DMA rows
+                rows_kb = im.size // 1024
+                r = np.minimum(np.arange(WAVES)[:, None] + WAVES * np.arange(-(-rows_kb // WAVES)), rows_kb - 1)
+                src = (nsb - 1) * im.size + 16 * 63 + 1024 * r
+                within(src, src + 16, nsb * im.size, "prepared x slab DMA source")
+                within(1024 * r, 1024 * r + 16 * 64, im.size, "prepared x slab DMA target")
+                assert set(r.reshape(-1)) == set(range(rows_kb))
 
 
 # ------------------------------------------------------------------ staged B = 1 kernel (jh_gemv_staged.hip)

@@ -108,3 +108,41 @@ def test_wide_group(types, captured):
         check(y.cpu().numpy(), X, O.dequantize(t, w, r, cols).astype(np.float64).reshape(r, cols), (t, r, captured))
     for d in devs:
         d.close()
+
+
+def layout(qtype, rows, cols, B):
+    out = (ctypes.c_int * 13)()
+    assert _lib.load().jh_qmatvec_batched_layout_shape(qtype, cols, 0, rows, B, out, 13) == 0
+    return dict(zip(("kernel", "ksplit", "ksb", "columns", "chunks"), out))
+
+
+@pytest.mark.parametrize("qtype", [O.Q4_K, O.Q5_K, O.Q8_0, O.Q2_K])
+@pytest.mark.parametrize("rows,cols,B", [(20300, 512, 100), (20300, 512, 127), (20300, 1024, 128), (20300, 1024, 130)])
+def test_chunks_of_64(qtype, rows, cols, B):
+    """Where the planner takes chunks of 64 columns: full ones, and last ones of 36, 63
+    and 2."""
+    assert layout(qtype, rows, cols, B)["columns"] == 64
+    raw = weights(qtype, rows, cols, B)
+    X = np.random.default_rng(B).standard_normal((B, cols)).astype(np.float32)
+    with upload(qtype, rows, cols, raw) as dev:
+        Y = run(dev, X, rows)
+    check(Y, X, O.dequantize(qtype, raw, rows, cols).astype(np.float64).reshape(rows, cols), (qtype, rows, cols, B))
+
+
+def test_group_in_chunks_of_64():
+    import torch
+    types, rows, cols, B = (O.Q4_K, O.Q8_0, O.Q5_K, O.Q2_K), (10200, 5100, 257, 4700), 512, 100
+    assert layout(O.Q4_K, 256 * sum(-(-r // 256) for r in rows), cols, B)["columns"] == 64  # the group's row tiles
+    raws = [weights(t, r, cols, 17 + i) for i, (t, r) in enumerate(zip(types, rows))]
+    X = np.random.default_rng(18).standard_normal((B, cols)).astype(np.float32)
+    devs = [upload(t, r, cols, w) for t, r, w in zip(types, rows, raws)]
+    n, P = len(types), ctypes.c_void_p
+    dx, ys = torch.from_numpy(X).cuda(), [torch.zeros(B, r, device="cuda") for r in rows]
+    torch.cuda.synchronize()
+    assert _lib.load().jh_qmatvec_batched_group_dev(n, (P * n)(*[d.handle for d in devs]), (P * n)(*[dx.data_ptr()] * n), B,
+                                                    (P * n)(*[y.data_ptr() for y in ys]), None) == 0
+    torch.cuda.synchronize()
+    for t, r, w, y in zip(types, rows, raws, ys):
+        check(y.cpu().numpy(), X, O.dequantize(t, w, r, cols).astype(np.float64).reshape(r, cols), (t, r))
+    for d in devs:
+        d.close()
