@@ -21,11 +21,13 @@
 //    Each workgroup converts the fp32 x slice of a super-block straight into
 //    its LDS image while it stages the weights (no separate prep launch).
 //    Up to 16 columns (HL) the two limbs share one MFMA, rows 0..15 and 16..31
-//    of its A operand.  What bounds the walk is the reading of x from LDS: every
-//    wave needs all of it for its own 32 rows, 33 KB per super-block and wave at
-//    143 B/ns per CU (1.85 us for 8 waves, against 1.2 us of MFMA); HL halves that
-//    and the MFMAs (us, 16 columns, before -> after: 2 x 14336 x 4096 Q4_K 36 -> 29,
-//    4096 x 14336 Q6_K 30 -> 27, 4096^2 Q4_K 13.5 -> 11.6, 9216 x 3072 Q8_0 18.1 -> 16.0).
+//    of its A operand, which takes out half the MFMAs and half the reads of x from
+//    LDS (us, 16 columns, before -> after: 2 x 14336 x 4096 Q4_K 36 -> 29, 4096 x 14336
+//    Q6_K 30 -> 27, 4096^2 Q4_K 13.5 -> 11.6, 9216 x 3072 Q8_0 18.1 -> 16.0).
+//  * What bounds it: no unit alone.  2 x 14336 x 4096 Q4_K at B = 32 (36.7 us) keeps the
+//    VALUs busy 46 % of the cycles, LDS 26 %, the matrix cores 22 %, and its waves wait
+//    for 27 % of theirs: one workgroup per CU goes through load, conversion, decode,
+//    MFMAs and barrier in step.
 //  * Work split: a workgroup is kWaves waves x 32 rows, all B columns, and a
 //    range of super-blocks.  Per super-block it stages the x slice in LDS
 //    (shared by all its rows) and each wave stages its rows' packed blocks in
@@ -439,7 +441,9 @@ __device__ __forceinline__ void step_fence(f32x16 (&part)[NT]) {
     for (int n = 0; n < NT; n++) asm volatile("" : "+v"(part[n]));
     __builtin_amdgcn_sched_barrier(0);
 }
-// TWO (see kTwo): the folds of a super-block's quarters are summed apart, then in pairs
+// How the super-blocks' sums are added up (see kChains): up to 64 columns; chunks of 32; of 64
+enum Sums { kPlain, kChained, kWide64 };
+// kChained: the folds of a super-block's quarters are summed apart, then in pairs
 template <int NT>
 __device__ __forceinline__ void next_quarter(int t, f32x16 (&part)[NT], f32x16 (&quarter)[NT], f32x16 (&half)[NT]) {
 #pragma unroll
@@ -525,7 +529,7 @@ struct FmtKQ {
         const uint32_t v = sh > 0 ? w >> (sh > 0 ? sh : 0) : w << (sh < 0 ? -sh : 0);
         return __builtin_elementwise_fma(as_h2((v & 0x00F000F0u) | top), ls, off);
     }
-    template <bool HL, int NT, bool TWO, class C>
+    template <bool HL, int NT, Sums SUMS, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         // 6-bit scales and mins of the 8 sub-blocks, one per byte (q4kScaleRaw / q4kMinRaw, :1471-1482),
         // and their centres: 8 (Q5_K 16) where the min is not zero
@@ -620,7 +624,7 @@ struct FmtQ6K {
         return ((load16(p + 64 * n + 32 * (qd & 1) + 16 * j) >> (qd >= 2 ? 4 : 0)) & 0x0F0F0F0Fu) |
                (((load16(p + 128 + 32 * n + 16 * j) >> (2 * qd)) & 0x03030303u) << 4);
     }
-    template <bool HL, int NT, bool TWO, class C>
+    template <bool HL, int NT, Sums SUMS, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1056.f);  // 1024 + 32
         const float d = half_bits_to_float(r.dw >> 16);
@@ -639,7 +643,7 @@ struct FmtQ6K {
             mfma_xw<HL, NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
             fold<NT>(part, d * (float)(int8_t)byte_of(t < 4 ? r.sc.x : t < 8 ? r.sc.y : t < 12 ? r.sc.z : r.sc.w, t & 3), acc);
             if (t % (NT > 1 ? 2 : 4) == (NT > 1 ? 1 : 3)) step_fence(part);
-            if (TWO) next_quarter<NT>(t, part, quarter, half);
+            if (SUMS == kChained) next_quarter<NT>(t, part, quarter, half);
         }
         fold_columns<HL, NT>(c, part, tot);
     }
@@ -665,7 +669,7 @@ struct FmtQ8_0 {
         mn = 0.f;
         return load16(p + 34 * (t >> 1) + 2 + 16 * (t & 1)) ^ 0x80808080u;
     }
-    template <bool HL, int NT, bool TWO, class C>
+    template <bool HL, int NT, Sums SUMS, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1152.f);  // 1024 + 128
         f32x16 part[NT];
@@ -689,7 +693,7 @@ struct FmtQ8_0 {
                 mfma_xw<HL, NT>(c, bytes_to_h8((j ? qb.z : qb.x) ^ 0x80808080u, (j ? qb.w : qb.y) ^ 0x80808080u, off),
                                 32 * b + 16 * c.kh + 8 * j, acc);
             fold<NT>(part, half_bits_to_float(db), acc);
-            if (HL || NT > 1 || TWO) step_fence(part);
+            if (HL || NT > 1 || SUMS == kChained) step_fence(part);
         }
         fold_columns<HL, NT>(c, part, tot);
     }
@@ -704,15 +708,15 @@ struct FmtQ8_0 {
 // the centre's share and the min term are MFMAs per super-block against the
 // 16-column sums of x.  The sums are folded with d every 8 K-steps: every 16 is
 // 6 % faster at B = 48 but its error against 64 bits (K = 1024: 1.77e-7) is larger
-// than the VALU kernel's 1.61e-7; every 8 gives 1.52e-7, every 4 1.40e-7 (and
-// folding each K-step with d*(sc&15) is 7 % slower).
+// than the VALU kernel's 1.61e-7; every 8 gives 1.52e-7, every 4 1.40e-7, which
+// chunks of 32 columns take; chunks of 64, with one chain of super-blocks, fold every 2
+// (folding each K-step with d*(sc&15) is 7 % slower).
 // Blocks are 4-byte aligned (84 = 4 * 21).
 struct FmtQ2K {
     static constexpr int kSums = 16;
     static constexpr int kBytes = 84;
     static constexpr int kChunks = (kBytes + 12 + 15) / 16;  // a 4-byte-aligned block spans <= 6 chunks
     static constexpr int kRowChunks = kChunks + 1;           // 28-dword window rows (2-way bank conflicts)
-    static constexpr int kFold = 8;  // K-steps per fold: see above
     struct Regs {
         u32x2 q[2][2];  // [h][k&1]: qs bytes 32h + 16(k&1) + 8kh .. +8
         u32x4 sc;       // the 16 scale bytes
@@ -744,8 +748,9 @@ struct FmtQ2K {
         const uint32_t v = sh > 0 ? w >> (sh > 0 ? sh : 0) : w << (sh < 0 ? -sh : 0);
         return __builtin_elementwise_fma(as_h2((v & 0x00300030u) | top), sc, off);
     }
-    template <bool HL, int NT, bool TWO, class C>
+    template <bool HL, int NT, Sums SUMS, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
+        constexpr int kFold = SUMS == kPlain ? 8 : SUMS == kChained ? 4 : 2;  // K-steps per fold: see above
         const float d = half_bits_to_float(r.dm), dmin = half_bits_to_float(r.dm >> 16);
         const uint32_t top = in_vgpr(0x54005400u);
         const half2v k = dup(1024.f);
@@ -830,7 +835,7 @@ struct FmtQ3K {
         return ((load16(p + 32 + 32 * h + 16 * rr) >> (2 * j)) & 0x03030303u) |
                (((load16(p + 16 * rr) >> (4 * h + j)) & 0x01010101u) << 2);
     }
-    template <bool HL, int NT, bool TWO, class C>
+    template <bool HL, int NT, Sums SUMS, class C>
     static __device__ __forceinline__ void compute(const Regs &r, const C &c, float (&tot)[NT][kOut<HL>]) {
         const half2v off = dup(1028.f);  // 1024 + 4
         f32x16 part[NT], quarter[NT], half[NT];
@@ -858,8 +863,8 @@ struct FmtQ3K {
                     mfma_xw<HL, NT>(c, bytes_to_h8(u0, u1, off), 16 * t + 8 * c.kh, acc);
                     const int s6 = (int)byte_of(j < 2 ? ua : ub, 2 * (j & 1) + rr) - 32;
                     fold<NT>(part, d * (float)s6, acc);
-                    if (TWO && t % 4 == 3) step_fence(part);
-                    if (TWO) next_quarter<NT>(t, part, quarter, half);
+                    if (SUMS == kChained && t % 4 == 3) step_fence(part);
+                    if (SUMS == kChained) next_quarter<NT>(t, part, quarter, half);
                 }
         }
         fold_columns<HL, NT>(c, part, tot);
@@ -1010,7 +1015,7 @@ struct RowSpan {
 // launch costs ~5 us.
 constexpr int kMaxTileCounters = kCounterSlots;
 
-template <int NT, int NI>
+template <bool WIDE = false, int NT, int NI>
 __device__ __forceinline__ void store_tile(const float (&tot)[NT][NI], int r, int nrows, int kh, int B, float *__restrict__ Y,
                                            float *part, size_t plane, int *counters, int tile, int split, int ksplit) {
     const bool live = r < nrows;
@@ -1082,13 +1087,25 @@ __device__ __forceinline__ void store_tile(const float (&tot)[NT][NI], int r, in
                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
         }
+        if constexpr (WIDE) {  // pairs first: see kChains
 #pragma unroll
-        for (int kk = 0; kk < KB; kk++)
-            if (k0 + kk < ks)
+            for (int n = 0; n < NT; n++)
 #pragma unroll
-                for (int n = 0; n < NT; n++)
+                for (int i = 0; i < NI; i++) {
 #pragma unroll
-                    for (int i = 0; i < NI; i++) acc[n][i] += v[kk][n][i];
+                    for (int kk = 1; kk < KB; kk++) v[kk][n][i] = k0 + kk < ks ? v[kk][n][i] : 0.f;
+                    const float s = v[0][n][i] + v[1][n][i];
+                    acc[n][i] += KB == 4 ? s + (v[KB - 2][n][i] + v[KB - 1][n][i]) : s;
+                }
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < KB; kk++)
+                if (k0 + kk < ks)
+#pragma unroll
+                    for (int n = 0; n < NT; n++)
+#pragma unroll
+                        for (int i = 0; i < NI; i++) acc[n][i] += v[kk][n][i];
+        }
     }
 #pragma unroll
     for (int n = 0; n < NT; n++)
@@ -1125,14 +1142,20 @@ struct MfmaGroup {
 
 // More than 64 columns (WIDE): chunks of 64 columns in one launch, in the kernel of
 // 33..64 columns: before, the VALU kernels read the weights again for every 8
-// columns (2 x 14336 x 4096 Q4_K and 4096 x 14336 Q6_K at B = 128: 5460 -> 181 us).
-// Groups with Q6_K or Q3_K take chunks of 32 and sum in more fp32 chains (the
-// quarters of a super-block's 16 folds, and even and odd super-blocks): the folds'
-// roundings are most of their error, and in one chain of each it would be larger
-// than that of the VALU kernels' many lanes (K = 4096: Q6_K 1.15e-7 against 1.02e-7
-// of the norm, Q3_K 1.13e-7 against 1.00e-7).
+// columns (8B feed-forward at B = 128, whole block: 5456 -> 181 us).
+// The VALU kernels sum a row in many lanes; one chain of fp32 sums per output over all
+// of K is less exact than that.  So chunks of 32, whose accumulators leave the registers
+// for it, sum in kChains chains over the super-blocks in turn and Q6_K and Q3_K, whose 16
+// folds per super-block are most of their error, in quarters of a super-block as well.
+// Groups with one of these two take chunks of 32 only, and those with Q8_0 where a
+// workgroup walks more than kLongWalk super-blocks; and the splits' partials are added in
+// pairs.  Error against 64 bits at B = 128, one or two chains / now / VALU kernels, 1e-7 of
+// the norm: 20480 rows, K = 8192 Q8_0 1.39 / 1.13 / 1.28, Q3_K 1.14 / 1.05 / 1.12, Q6_K 1.14 /
+// 1.05 / 1.14; 2048 x 3840 Q3_K 1.014 / 0.959 / 1.000.  us: 4096 x 14336 Q6_K 80.5 / 83, Q3_K
+// 70.6 / 72, 16384 x 8192 Q8_0 141 / 150, 20000 x 14336 429 / 487, Q2_K 303 / 378.
 template <bool WIDE, int NT>
-constexpr bool kTwo = WIDE && NT == 1;
+constexpr Sums kSumsOf = !WIDE ? kPlain : NT == 1 ? kChained : kWide64;
+constexpr int kChains = 4, kLongWalk = 16;
 
 // format mask bits: Q4_K, Q5_K, Q6_K, Q8_0, Q2_K, Q3_K
 template <int MASK>
@@ -1227,11 +1250,11 @@ __device__ __forceinline__ void store_pair(const float (&tot)[1][NI], int r, int
 
 // One workgroup's tile (32 rows per wave x all batch columns) over the K
 // range of its split, x converted into LDS super-block by super-block.
-// WIDE: column chunk `chunk` of g.chunks (32 NT columns each); TWO: see kTwo.
+// WIDE: column chunk `chunk` of g.chunks (32 NT columns each).
 // EXACT: see split_x.  NT: column groups of 32 (HL: one of 16)
 template <class F, bool HL, int NT, bool PAIR, bool WIDE, bool EXACT>
 __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int chunk, int split, const MfmaGroup &g, uint8_t *lds) {
-    constexpr bool TWO = kTwo<WIDE, NT>;
+    constexpr Sums SUMS = kSumsOf<WIDE, NT>;
     const int chunks = WIDE ? g.chunks : 1, col0 = WIDE ? chunk * 32 * NT : 0;
     using I = XImage<HL, NT>;
     constexpr int NI = kOut<HL>;
@@ -1295,10 +1318,12 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
     } while (0)
 
     Marks marked;  // blocks left to add_exact
-    float tot[NT][NI], tot2[NI];
-    if constexpr (TWO) {
+    float tot[NT][NI], more[kChains - 1][NI];  // (kChained: the other chains)
+    if constexpr (SUMS == kChained) {
 #pragma unroll
-        for (int i = 0; i < NI; i++) tot2[i] = 0.f;
+        for (int k = 0; k < kChains - 1; k++)
+#pragma unroll
+            for (int i = 0; i < NI; i++) more[k][i] = 0.f;
     }
 #pragma unroll
     for (int n = 0; n < NT; n++)
@@ -1339,13 +1364,15 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
             JH_MT(3 + 4 * (sb - sb0));
             const Ctx<HL, NT> c{lr, kh, lds + buf * I::kBytes};
             if constexpr (EXACT) marked.add(marked_columns<HL, NT>(c), sb);
-            F::template compute<HL, NT, TWO>(w, c, tot);
-            if constexpr (TWO) {
+            F::template compute<HL, NT, SUMS>(w, c, tot);
+            if constexpr (SUMS == kChained) {
 #pragma unroll
                 for (int i = 0; i < NI; i++) {
                     const float v = tot[0][i];
-                    tot[0][i] = tot2[i];
-                    tot2[i] = v;
+                    tot[0][i] = more[0][i];
+#pragma unroll
+                    for (int k = 0; k + 1 < kChains - 1; k++) more[k][i] = more[k + 1][i];
+                    more[kChains - 2][i] = v;
                 }
             }
             JH_MT(4 + 4 * (sb - sb0));
@@ -1371,7 +1398,7 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
             __syncthreads();
             const Ctx<HL, NT> c{lr, kh, lds};
             if constexpr (EXACT) marked.add(marked_columns<HL, NT>(c), sb);
-            F::template compute<HL, NT, TWO>(w, c, tot);
+            F::template compute<HL, NT, SUMS>(w, c, tot);
         }
     }
 #undef JH_LOAD_X
@@ -1387,11 +1414,11 @@ __device__ __forceinline__ void gemm_body(const MfmaProblem &P, int tile, int ch
                    g.swiglu, g.part, g.counters, tile, split, g.ksplit, lds);
         return;
     }
-    if constexpr (TWO) {
+    if constexpr (SUMS == kChained) {
 #pragma unroll
-        for (int i = 0; i < NI; i++) tot[0][i] += tot2[i];
+        for (int i = 0; i < NI; i++) tot[0][i] = (tot[0][i] + more[0][i]) + (more[1][i] + more[2][i]);
     }
-    store_tile(tot, rbase + lr, nrows, kh, B, P.y + (size_t)col0 * nrows, g.part + P.part0 + (size_t)col0 * nrows,
+    store_tile<WIDE>(tot, rbase + lr, nrows, kh, B, P.y + (size_t)col0 * nrows, g.part + P.part0 + (size_t)col0 * nrows,
                (size_t)g.B * nrows, g.counters + (size_t)P.cnt0 * kCounterStride, tile * chunks + chunk, split, g.ksplit);
 }
 
@@ -1518,7 +1545,7 @@ __global__ __launch_bounds__(kThreads) void mfma_px(const uint8_t *W, size_t pit
         JH_LOAD_W(SET, (SB) + 2);                                                                          \
         const CtxP<HL> c{lr, kh, sh_x[BUF]};                                                               \
         if constexpr (EXACT) marked.add(marked_columns<HL, 1>(c), SB);                                     \
-        F::template compute<HL, 1, false>(w, c, tot);                                                      \
+        F::template compute<HL, 1, kPlain>(w, c, tot);                                                      \
     } while (0)
 
     dma_x(sb0, 0);
@@ -1598,9 +1625,10 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p, bool pair = fal
     if (n < 1 || n > kMaxMfmaGroup) return false;
     int tiles = 0;
     size_t rows = 0;
-    bool fine = false;  // chunks of 32 columns only (see kTwo)
+    bool fine = false, fine_long = false;  // chunks of 32 columns only, always or for long walks (see kChains)
     for (int i = 0; i < n; i++) {
         fine = fine || d[i].type == 14 || d[i].type == 11;
+        fine_long = fine_long || d[i].type == 8;
         if (!mfma_applies(d[i], B) || d[i].cols != d[0].cols) return false;
         const int each = (d[i].row_end - d[i].row_start) / (pair ? 2 : 1);
         tiles += (pair ? 2 : 1) * ((each + kRowsPerWG - 1) / kRowsPerWG);
@@ -1630,6 +1658,7 @@ static bool plan_group(int n, const MfmaDesc *d, int B, Plan &p, bool pair = fal
         const int ctiles = row_tiles * chunks;
         for (int ks = 1; ks <= p.nsb; ks++) {
             const int ksb = (p.nsb + ks - 1) / ks, kse = (p.nsb + ksb - 1) / ksb;
+            if (c == 64 && fine_long && ksb > kLongWalk) continue;
             if (kse > 1 && ctiles > kMaxTileCounters) break;  // a split needs a counter per tile
             if (kse > 1 && B > 64 && sizeof(float) * (size_t)kse * B * rows > kStaticScratchBytes) break;
             const int rounds = (int)(((long long)ctiles * kse + kMinWorkgroups - 1) / kMinWorkgroups);
@@ -1893,9 +1922,13 @@ hipError_t launch_mfma_group(int n, const MfmaDesc *d, int B, void *workspace, i
     if (!plan_group(n, d, B, p)) return hipErrorNotSupported;
     if (!workspace && B <= 64) return hipErrorNotSupported;
     if (!workspace) {  // K whole
-        p.grid /= p.ksplit;
+        const int tiles = p.grid / (p.ksplit * p.chunks);
         p.ksplit = 1;
         p.ksb = p.nsb;
+        for (int i = 0; i < n; i++)
+            if (d[i].type == 8 && p.nsb > kLongWalk) p.chunk = 32;
+        p.chunks = (B + p.chunk - 1) / p.chunk;
+        p.grid = tiles * p.chunks;
     }
     if (p.ksplit > 1 && !counters) return hipErrorNotSupported;
     uint8_t *ws = reinterpret_cast<uint8_t *>(workspace);

@@ -90,6 +90,8 @@ def plan(t, rows, cols, B):
             kse = -(-nsb // ksb)
             if kse > 1 and (tiles * chunks > COUNTER_SLOTS or (B > 64 and 4 * kse * B * rows > STATIC_SCRATCH)):
                 break
+            if c == 64 and t == Q8_0 and ksb > 16:  # kLongWalk
+                continue
             rounds = -(-tiles * chunks * kse // MIN_WG)
             cost = (4 * (rounds * (ksb + 5) + (kse > 1)) + (kse if kse > 1 else 0)) * (8 if c == 64 else 5)
             if best is None or cost < best[0]:

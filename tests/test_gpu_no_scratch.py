@@ -22,19 +22,19 @@ def ksplit(dev, B):
     return ks.value
 
 
-@pytest.mark.parametrize("qtype", [O.Q6_K, O.Q3_K])
-@pytest.mark.parametrize("B", [65, 100])
-def test_captured_first(qtype, B):
+@pytest.mark.parametrize("qtype,rows,of,cols,B", [
+    (O.Q6_K, 300, 12000, 4096, 65), (O.Q6_K, 300, 12000, 4096, 100), (O.Q3_K, 300, 12000, 4096, 65),
+    (O.Q3_K, 300, 12000, 4096, 100), (O.Q8_0, 10240, 12800, 8192, 100)])  # Q8_0: split, in chunks of 64; whole, of 32
+def test_captured_first(qtype, rows, of, cols, B):
     import torch
     L = _lib.load()
-    rows, copies, cols = 300, 40, 4096
-    raw = weights(qtype, rows, cols, 40)
+    raw = weights(qtype, 100, cols, 40).reshape(100, -1)
     x = torch.from_numpy(np.random.default_rng(41).standard_normal((B, cols)).astype(np.float32)).cuda()
-    y, tall = torch.zeros(B, rows, device="cuda"), torch.zeros(B, rows * copies, device="cuda")
-    with upload(qtype, rows, cols, raw) as dev, upload(
-            qtype, rows * copies, cols, np.tile(raw.reshape(rows, -1), (copies, 1)).reshape(-1)) as many:
+    y, tall = torch.zeros(B, rows, device="cuda"), torch.zeros(B, of, device="cuda")
+    tile = np.tile(raw, (-(-of // 100), 1))
+    with upload(qtype, rows, cols, tile[:rows].reshape(-1)) as dev, upload(qtype, of, cols, tile[:of].reshape(-1)) as many:
         assert ksplit(dev, B) > 1 and ksplit(many, B) == 1
-        assert L.jh_qmatvec_batched_dev(many.handle, P(x.data_ptr()), B, P(tall.data_ptr()), 0, rows * copies, None) == 0
+        assert L.jh_qmatvec_batched_dev(many.handle, P(x.data_ptr()), B, P(tall.data_ptr()), 0, of, None) == 0
         torch.cuda.synchronize()
         st = fresh_stream()
         g = torch.cuda.CUDAGraph()

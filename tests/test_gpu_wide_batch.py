@@ -146,3 +146,41 @@ def test_group_in_chunks_of_64():
         check(y.cpu().numpy(), X, O.dequantize(t, w, r, cols).astype(np.float64).reshape(r, cols), (t, r))
     for d in devs:
         d.close()
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("cols", [1024, 4096])
+def test_no_less_exact_than_the_fp32_kernels(qtype, cols):
+    """The error of 96 vectors against 64 bits, in the norm, is no larger than that of
+    the kernels that took such batches before (two vectors at a time: on a small matrix
+    they still do)."""
+    rows, B = 520, 96
+    raw = weights(qtype, rows, cols, 90)
+    X = np.random.default_rng(91).standard_normal((B, cols)).astype(np.float32)
+    assert layout(qtype, rows, cols, B)["kernel"] == 1 and layout(qtype, rows, cols, 2)["kernel"] == 0
+    with upload(qtype, rows, cols, raw) as dev:
+        Y = run(dev, X, rows).astype(np.float64)
+        Z = np.concatenate([run(dev, X[b:b + 2], rows) for b in range(0, B, 2)]).astype(np.float64)
+    ref = X.astype(np.float64) @ O.dequantize(qtype, raw, rows, cols).astype(np.float64).reshape(rows, cols).T
+    ours, fp32 = (np.linalg.norm(v - ref) / np.linalg.norm(ref) for v in (Y, Z))
+    print(qtype, cols, "error", ours, "fp32 kernels", fp32, flush=True)
+    assert ours <= fp32
+
+
+@pytest.mark.parametrize("qtype,rows,cols", [(O.Q8_0, 12800, 8192), (O.Q2_K, 10240, 4096)])
+def test_no_less_exact_where_k_is_not_split(qtype, rows, cols):
+    """The same for long walks of one workgroup, on the first rows (row ranges of 640,
+    which two vectors take on the fp32 kernels)."""
+    B = 100
+    assert layout(qtype, rows, cols, B)["ksplit"] == 1
+    raw = weights(qtype, 640, cols, 92)
+    X = np.random.default_rng(93).standard_normal((B, cols)).astype(np.float32)
+    with upload(qtype, rows, cols, np.tile(raw.reshape(640, -1), (rows // 640, 1)).reshape(-1)) as dev:
+        Y = run(dev, X, rows)[:, :640].astype(np.float64)
+    assert layout(qtype, 640, cols, 2)["kernel"] == 0
+    with upload(qtype, 640, cols, raw) as dev:
+        Z = np.concatenate([run(dev, X[b:b + 2], 640) for b in range(0, B, 2)]).astype(np.float64)
+    ref = X.astype(np.float64) @ O.dequantize(qtype, raw, 640, cols).astype(np.float64).reshape(640, cols).T
+    ours, fp32 = (np.linalg.norm(v - ref) / np.linalg.norm(ref) for v in (Y, Z))
+    print(qtype, rows, cols, "error", ours, "fp32 kernels", fp32, flush=True)
+    assert ours <= fp32
