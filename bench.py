@@ -90,7 +90,7 @@ def make_step(torch, L, mats, B, stream, grouped=True):
     [down]; then the lm_head.  Each stage has its own input vector, as in a
     real step (attention-norm output, attention output, FFN-norm output,
     SwiGLU product).  B > 1 groups the same way through the batched group
-    entry point (one MFMA launch per group at B >= 16)."""
+    entry point (one MFMA launch per group at B >= 3)."""
     g = torch.Generator(device="cuda")
     g.manual_seed(1)
     x_attn = torch.randn(B, HIDDEN, generator=g, device="cuda")
@@ -459,8 +459,8 @@ def profile_mode(torch, L, be):
 
 def profile_mfma_mode(torch, L, be):
     """Launches for MFMA counter runs (rocprofv3 --pmc): 8 layers' grouped
-    Q4_K [gate, up] GEMVs at B = 32 (mfma_group<1, 1>) and at B = 64
-    (mfma_group<2, 1>), eagerly, 4 times each, then the calibration copy."""
+    Q4_K [gate, up] GEMVs at B = 32 (mfma_group<false, 1, 1, ..>) and at B = 64
+    (mfma_group<false, 2, 1, ..>), eagerly, 4 times each, then the calibration copy."""
     g = torch.Generator(device="cuda")
     g.manual_seed(0)
     mats = []
