@@ -122,10 +122,14 @@ struct Staging {
     size_t cap_hx = 0, cap_hy = 0;
 };
 
+void free_stream_workspace(int device, hipStream_t s);
+
 struct ThreadStaging {
     Staging per_dev[64];
     ~ThreadStaging() {
-        for (auto &s : per_dev) {
+        for (int dev = 0; dev < 64; dev++) {
+            Staging &s = per_dev[dev];
+            if (s.stream) free_stream_workspace(dev, s.stream);
             if (s.d_x) (void)hipFree(s.d_x);
             if (s.d_y) (void)hipFree(s.d_y);
             if (s.h_x) (void)hipHostFree(s.h_x);
@@ -244,6 +248,17 @@ struct WorkspacePool {
 WorkspacePool &ws_pool() {
     static WorkspacePool *p = new WorkspacePool;
     return *p;
+}
+
+// The workspace of a stream of the library's own (a thread's staging stream), which
+// ends: its calls are synchronous and never captured.
+void free_stream_workspace(int device, hipStream_t s) {
+    WorkspacePool &pool = ws_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    auto it = pool.used.find(WsKey{device, s, 0});
+    if (it == pool.used.end()) return;
+    if (it->second.base) (void)hipFree(it->second.base);
+    pool.used.erase(it);
 }
 
 struct ThreadWorkspaces {

@@ -12,6 +12,7 @@ import pytest
 
 import oracle as O
 from juno_amd import _lib
+from juno_amd import matvec as mv
 from test_gpu_wide_batch import upload, weights
 
 pytestmark = pytest.mark.gpu
@@ -123,3 +124,41 @@ def test_a_captured_workspace_is_not_handed_on():
         torch.cuda.synchronize()
         assert base and base not in others
         assert L.hipGraphDestroy(g) == 0
+
+
+@pytest.mark.parametrize("B", [2, 16])
+def test_host_calls_give_their_workspace_back(B):
+    """Host-pointer calls run on a stream per thread; its workspace (8 MB and more) ends
+    with the thread."""
+    import torch
+    rows, cols, n = 6656, 4096, 8
+    raw = weights(O.Q4_K, rows, cols, 33)
+    X = np.random.default_rng(34).standard_normal((B, cols)).astype(np.float32)
+    meet = threading.Barrier(n)
+    be = mv.GpuContext.shared(0).create_mat_vec()
+    with upload(O.Q4_K, rows, cols, raw) as dev:
+
+        def work():
+            y = np.asarray(be.sgemv_batched(dev, X, 0, rows)).copy()
+            meet.wait(30)  # all alive at once
+            return y
+
+        want = in_threads([work] * n)
+        torch.cuda.synchronize()
+        free0 = torch.cuda.mem_get_info()[0]
+        got = in_threads([work] * n)
+        torch.cuda.synchronize()
+        assert all(np.array_equal(a.view(np.uint32), want[0].view(np.uint32)) for a in want + got)
+        held = []
+
+        def hold():
+            be.sgemv_batched(dev, X, 0, rows)
+            meet.wait(30)
+            if not held:
+                held.append(torch.cuda.mem_get_info()[0])
+            meet.wait(30)
+
+        in_threads([hold] * n)
+        torch.cuda.synchronize()
+        assert free0 - held[0] >= n << 22  # theirs while they live
+        assert free0 - torch.cuda.mem_get_info()[0] < 8 << 20
