@@ -2,7 +2,7 @@
 load and store and every LDS window access of the batched MFMA kernel
 (jh_mfma.hip gemm_body / mfma_px), the staged B = 1 kernel
 (jh_gemv_staged.hip) and the one-shot kernels (jh_gemv.hip), for every
-BASELINE shape, batch and row range, must stay inside the buffer it targets.
+benchmark shape, batch and row range, must stay inside the buffer it targets.
 
 Each model below restates one kernel's index formulas with its file:line, per
 lane, wave, workgroup and step (numpy over all of them at once, at the extreme
@@ -35,7 +35,7 @@ def pitch(t, cols):
     return cols // qk * bb
 
 
-# TinyLlama (config 1 and 2), Llama-3-8B (3 and 4), Phi-3-mini (5)
+# the matrices of TinyLlama, Llama-3-8B and Phi-3-mini, and some odd ones
 SHAPES = sorted({
     (Q4_K, 5632, 2048), (Q4_K, 2048, 2048), (Q4_K, 256, 2048), (Q6_K, 256, 2048), (Q6_K, 2048, 5632),
     (Q6_K, 32000, 2048),
